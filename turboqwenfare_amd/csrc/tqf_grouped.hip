@@ -10,8 +10,8 @@
 // prefill chunk.
 //
 // Kernels (stream-ordered, no host round trip):
-//   plan     one workgroup: counting sort of the T*8 (token, k) pairs by
-//            expert (stable in pair order), the tile list of 32-pair tiles;
+//   plan     counting sort of the T*8 (token, k) pairs by expert (stable in
+//            pair order), the tile list of 32-pair tiles;
 //   gate_up  grid (F / 128 column blocks, tiles): gate and up on bf16 MFMA,
 //            SwiGLU, h stored as bf16 hi + lo;
 //   down     grid (H / 256 column blocks, tiles): down on bf16 MFMA;
@@ -83,143 +83,123 @@ __device__ __forceinline__ int d_row(int v, int half) { return 8 * (v / 4) + 4 *
 }  // namespace
 
 // ---- plan: counting sort of the (token, k) pairs by expert ------------------
-// Positions are stable in pair order (p = 8 t + k).  The pairs go in batches
-// of kPlanRounds x 1024: in each round a wavefront ranks equal experts with
-// ballots and the first lane of each peer group writes the group's size to
-// the count slot (round, wavefront) of its expert; one thread per expert
-// then turns its slots into exclusive prefixes (slot order is pair order),
-// so a pair's position is base[e] + the positions of e in earlier batches +
-// its slot's prefix + its rank, with three workgroup barriers per batch.
-// base[e] is the exclusive scan of the expert counts: with one batch these
-// are the slot totals; with more, a first pass counts every pair (one count
-// per peer group).  Tile i of expert e covers positions off[e] + 32 i ..
-// + rows; a tile entry is {first position, e | rows << 16}.
-constexpr int kPlanRounds = 4;
-constexpr uint32_t kPlanBatch = kPlanRounds * kPlanThreads;
-constexpr int kPlanSlots = kPlanRounds * kPlanWaves;
+// Positions are stable in pair order (p = 8 t + k).  Workgroup b places the
+// 1024 pairs p = 1024 b .. and needs nothing from the others: it counts all
+// ids itself (LDS atomics, pairs before and after its own batch apart), its
+// wavefronts rank equal experts of the batch with ballots, and the first lane
+// of each peer group writes the group's size to the count slot of its
+// wavefront, which one thread per expert turns into exclusive prefixes.  A
+// pair's position is base[e] (the exclusive scan of all counts) + the pairs
+// of e before the batch + its slot's prefix + its rank.  Workgroup 0 writes
+// the tile list: tile i of expert e covers positions off[e] + 32 i .. + rows;
+// an entry is {first position, e | rows << 16}.
+// Bound by its serial steps, not by bytes.  One workgroup that walked the
+// batches took 8.4-10.8 us at 4096 pairs and 74-88 us at 32768; this takes
+// 5.0-6.1 and 8.9-11.0 us.
 __global__ __launch_bounds__(kPlanThreads) void gg_plan_kernel(
     const uint16_t *__restrict__ ids, uint32_t pairs, uint32_t E, int32_t *__restrict__ pos_of_pair,
     int32_t *__restrict__ pair_of_pos, uint2 *__restrict__ tiles, int32_t *__restrict__ n_tiles,
     int32_t *__restrict__ status) {
-    __shared__ uint16_t cnt[kPlanSlots][256];  // per slot: count of expert e, then its prefix
-    __shared__ int32_t hist[256], base[256], tbase[256], done[256], total[256];
+    __shared__ uint16_t cnt[kPlanWaves][256];  // this batch, per wavefront: count of expert e, then its prefix
+    __shared__ int32_t before[256], after[256], total[256], base[256], tbase[256];
     __shared__ int32_t s_bad;
     const int tid = threadIdx.x, wave = tid / kWave, lane = tid % kWave;
     const uint64_t below = (1ull << lane) - 1;
-    const bool one = pairs <= kPlanBatch;
+    const uint32_t b0 = blockIdx.x * kPlanThreads;
     if (tid < 256) {
-        hist[tid] = 0;
-        done[tid] = 0;
+        before[tid] = 0;
+        after[tid] = 0;
     }
+    for (int i = tid; i < kPlanWaves * 256 / 8; i += kPlanThreads)
+        reinterpret_cast<uint4 *>(&cnt[0][0])[i] = make_uint4(0, 0, 0, 0);
     if (tid == 0) s_bad = 0;
     __syncthreads();
-    if (!one) {
-        for (uint32_t r = 0; r < pairs; r += kPlanThreads) {
-            const uint32_t p = r + tid;
-            uint32_t key = 256u;  // no expert
-            if (p < pairs) {
-                const uint32_t e = ids[p];
-                if (e < E) key = e;
-                else s_bad = 1;
+    const uint32_t p = b0 + tid;
+    uint32_t key = 256u;  // no expert
+    if (p < pairs) {
+        const uint32_t e = ids[p];
+        if (e < E) key = e;
+        else s_bad = 1;
+    }
+    if (gridDim.x > 1) {  // the other batches' ids, eight loads in flight per thread
+        for (uint32_t r = tid; r < pairs; r += 8 * kPlanThreads) {
+            uint32_t e[8];
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                const uint32_t q = r + (uint32_t)i * kPlanThreads;
+                e[i] = q < pairs ? ids[q] : 0xFFFFu;
             }
-            const uint64_t peers = match_peers(key);
-            if (key < 256u && (peers & below) == 0) atomicAdd(&hist[key], (int)__popcll(peers));
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                const uint32_t q = r + (uint32_t)i * kPlanThreads;
+                if (q >= pairs) continue;
+                if (e[i] >= E) s_bad = 1;
+                else if (q - b0 >= (uint32_t)kPlanThreads) atomicAdd(q < b0 ? &before[e[i]] : &after[e[i]], 1);
+            }
         }
     }
-    bool planned = false;
-    for (uint32_t b0 = 0; b0 < pairs; b0 += kPlanBatch) {
-        uint32_t key[kPlanRounds];
-        int rank[kPlanRounds];
+    const uint64_t peers = match_peers(key);
+    const int rank = __popcll(peers & below);
+    if (key < 256u && rank == 0) cnt[wave][key] = (uint16_t)__popcll(peers);
+    __syncthreads();
+    if (s_bad) {
+        if (blockIdx.x == 0 && tid == 0) {
+            *n_tiles = 0;
+            if (status) *status = TQF_HIP_ERR_INVALID;
+        }
+        return;
+    }
+    if (tid < 256) {
+        int s = 0;
 #pragma unroll
-        for (int i = 0; i < kPlanRounds; ++i) {
-            const uint32_t p = b0 + (uint32_t)i * kPlanThreads + tid;
-            key[i] = 256u;
-            if (p < pairs) {
-                const uint32_t e = ids[p];
-                if (e < E) key[i] = e;
-                else s_bad = 1;
+        for (int v = 0; v < kPlanWaves; ++v) {
+            const int c = cnt[v][tid];
+            cnt[v][tid] = (uint16_t)s;
+            s += c;
+        }
+        total[tid] = before[tid] + s + after[tid];
+    }
+    __syncthreads();
+    if (wave == 0) {  // exclusive scans of pair and tile counts, 4 experts per lane
+        int c[4], tc[4], s = 0, ts = 0;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            c[j] = total[4 * lane + j];
+            tc[j] = (c[j] + kTileM - 1) / kTileM;
+            s += c[j];
+            ts += tc[j];
+        }
+        int is = s, its = ts;
+#pragma unroll
+        for (int d = 1; d < kWave; d *= 2) {
+            const int x = __shfl_up(is, d), y = __shfl_up(its, d);
+            if (lane >= d) {
+                is += x;
+                its += y;
             }
         }
-        for (int i = tid; i < kPlanSlots * 256 / 8; i += kPlanThreads)
-            reinterpret_cast<uint4 *>(&cnt[0][0])[i] = make_uint4(0, 0, 0, 0);
-        __syncthreads();
-        if (s_bad) {
-            if (tid == 0) {
-                *n_tiles = 0;
-                if (status) *status = TQF_HIP_ERR_INVALID;
-            }
-            return;
-        }
+        int o = is - s, to = its - ts;
 #pragma unroll
-        for (int i = 0; i < kPlanRounds; ++i) {
-            const uint64_t peers = match_peers(key[i]);
-            rank[i] = __popcll(peers & below);
-            if (key[i] < 256u && rank[i] == 0) cnt[i * kPlanWaves + wave][key[i]] = (uint16_t)__popcll(peers);
+        for (int j = 0; j < 4; ++j) {
+            base[4 * lane + j] = o;
+            tbase[4 * lane + j] = to;
+            o += c[j];
+            to += tc[j];
         }
-        __syncthreads();
-        if (tid < (int)E) {
-            int s = 0;
-            for (int v = 0; v < kPlanSlots; ++v) {
-                const int c = cnt[v][tid];
-                cnt[v][tid] = (uint16_t)s;
-                s += c;
-            }
-            total[tid] = s;
-            if (one) hist[tid] = s;
+        if (blockIdx.x == 0 && lane == kWave - 1) *n_tiles = its;
+    }
+    __syncthreads();
+    if (key < 256u) {
+        const int pos = base[key] + before[key] + cnt[wave][key] + rank;
+        pos_of_pair[p] = pos;
+        pair_of_pos[pos] = (int32_t)p;
+    }
+    if (blockIdx.x == 0 && tid < (int)E) {
+        const int c = total[tid];
+        for (int i = 0; i * kTileM < c; ++i) {
+            const int rows = c - i * kTileM < kTileM ? c - i * kTileM : kTileM;
+            tiles[tbase[tid] + i] = make_uint2((uint32_t)(base[tid] + i * kTileM), (uint32_t)tid | ((uint32_t)rows << 16));
         }
-        __syncthreads();
-        if (!planned) {
-            planned = true;
-            if (wave == 0) {  // exclusive scans of pair and tile counts, 4 experts per lane
-                int c[4], tc[4], s = 0, ts = 0;
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    const uint32_t e = 4 * lane + j;
-                    c[j] = e < E ? hist[e] : 0;
-                    tc[j] = (c[j] + kTileM - 1) / kTileM;
-                    s += c[j];
-                    ts += tc[j];
-                }
-                int is = s, its = ts;
-#pragma unroll
-                for (int d = 1; d < kWave; d *= 2) {
-                    const int a = __shfl_up(is, d), b = __shfl_up(its, d);
-                    if (lane >= d) {
-                        is += a;
-                        its += b;
-                    }
-                }
-                int o = is - s, to = its - ts;
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    const uint32_t e = 4 * lane + j;
-                    base[e] = o;
-                    tbase[e] = to;
-                    o += c[j];
-                    to += tc[j];
-                }
-                if (lane == kWave - 1) *n_tiles = its;
-            }
-            __syncthreads();
-            for (uint32_t e = tid; e < E; e += kPlanThreads) {
-                const int c = hist[e];
-                for (int i = 0; i * kTileM < c; ++i) {
-                    const int rows = c - i * kTileM < kTileM ? c - i * kTileM : kTileM;
-                    tiles[tbase[e] + i] = make_uint2((uint32_t)(base[e] + i * kTileM), e | ((uint32_t)rows << 16));
-                }
-            }
-        }
-#pragma unroll
-        for (int i = 0; i < kPlanRounds; ++i) {
-            if (key[i] < 256u) {
-                const uint32_t p = b0 + (uint32_t)i * kPlanThreads + tid;
-                const int pos = base[key[i]] + done[key[i]] + cnt[i * kPlanWaves + wave][key[i]] + rank[i];
-                pos_of_pair[p] = pos;
-                pair_of_pos[pos] = (int32_t)p;
-            }
-        }
-        __syncthreads();
-        if (tid < (int)E) done[tid] += total[tid];
     }
 }
 
@@ -592,7 +572,7 @@ GroupedBuffers grouped_buffers(void *scratch, uint32_t T, uint32_t E, uint32_t H
 
 hipError_t launch_grouped_plan(hipStream_t s, const uint16_t *ids, uint32_t T, uint32_t E,
                                const GroupedBuffers &g, int32_t *status) {
-    hipLaunchKernelGGL(gg_plan_kernel, dim3(1), dim3(kPlanThreads), 0, s, ids, T * kTopK, E,
+    hipLaunchKernelGGL(gg_plan_kernel, dim3((T * kTopK + kPlanThreads - 1) / kPlanThreads), dim3(kPlanThreads), 0, s, ids, T * kTopK, E,
                        g.pos_of_pair, g.pair_of_pos, g.tiles, g.n_tiles, status);
     return hipGetLastError();
 }
