@@ -199,3 +199,25 @@ def test_grouped_bad_id_in_any_plan_batch(backend, small, t, where):
     assert np.array_equal(backend.read(dy, np.float32, (t, 256)), backend.grouped_gemm(small.layer, x, ids, w))
     for b in (dx, dids, dw, dy, dst):
         backend.free(b)
+
+
+def _routes_with_counts(t, counts, seed):
+    """ids [t, 8] in which expert e has counts[e] pairs (the first experts; the
+    others share what is left evenly), in a seeded order."""
+    left = 8 * t - sum(counts)
+    rest = len(counts) + np.arange(left) % (E - len(counts))
+    flat = np.concatenate([np.repeat(np.arange(len(counts)), counts), rest])
+    rng = np.random.default_rng(seed)
+    w = rng.uniform(0.05, 0.2, (t, 8)).astype(np.float32)
+    return rng.permutation(flat).reshape(t, 8).astype(np.uint16), w
+
+
+# Tiles hold up to 32 rows below 1024 tokens (experts average under 32 pairs), up
+# to 64 from there on, in 16-row subtiles: counts on both sides of each edge.
+# 150 and 1023 / 1024 tokens also straddle the plan's 1024-pair workgroups.
+@pytest.mark.parametrize("t", [150, 1023, 1024])
+def test_grouped_tile_edges(backend, small, t):
+    counts = [1, 15, 16, 17, 31, 32, 33, 47, 48, 49, 63, 64, 65, 97, 129]
+    ids, w = _routes_with_counts(t, counts, t)
+    x = synth.bf16_round(synth.normal((t, small.H), seed=t))
+    assert rel_err(backend.grouped_gemm(small.layer, x, ids, w), small.want(x, ids, w)) < FFN_TOL

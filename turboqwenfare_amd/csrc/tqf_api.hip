@@ -2014,13 +2014,13 @@ int32_t enqueue_grouped(tqf_hip_ctx *ctx, const LayerDev &L, const uint16_t *x, 
     const double pairs = (double)t * kTopK;
     {
         Prof p(ctx);
-        hipError_t e = launch_grouped_plan(ctx->stream, ids, t, L.n_experts, g, status);
+        hipError_t e = launch_grouped_plan(ctx->stream, ids, x, t, L.n_experts, L.hidden, g, status);
         if (e != hipSuccess) return hip_fail(ctx, "grouped plan kernel launch", e);
-        p.end(TQF_HIP_KERNEL_GROUPED_AUX, pairs * 2, 0, nullptr);
+        p.end(TQF_HIP_KERNEL_GROUPED_AUX, pairs * 2 + t * L.hidden * 2.0, 0, nullptr);
     }
     {
         Prof p(ctx);
-        hipError_t e = launch_grouped_gate_up(ctx->stream, L, x, g);
+        hipError_t e = launch_grouped_gate_up(ctx->stream, L, g);
         if (e != hipSuccess) return hip_fail(ctx, "grouped gate/up kernel launch", e);
         p.end(TQF_HIP_KERNEL_GROUPED_GATE_UP, 0, 0, nullptr);
     }

@@ -11,31 +11,30 @@
 //
 // Kernels (stream-ordered, no host round trip):
 //   plan     counting sort of the T*8 (token, k) pairs by expert (stable in
-//            pair order), the tile list of 32-pair tiles;
-//   gate_up  grid (F / 128 column blocks, tiles): gate and up on bf16 MFMA,
-//            SwiGLU, h stored as bf16 hi + lo;
-//   down     grid (H / 256 column blocks, tiles): down on bf16 MFMA;
+//            pair order), the tile list; x put in MFMA operand order;
+//   gate_up  grid (F / 64 column blocks, tiles): gate and up on bf16 MFMA,
+//            SwiGLU, h stored as bf16 hi + lo in operand order;
+//   down     grid (H / 128 column blocks, tiles): down on bf16 MFMA;
 //   combine  y[t] = sum_k w[t,k] * out[pos(t,k)] in route order.
 // (Dealing a tile's column blocks to one XCD, so that they share its
-// activation rows in one L2, measured no faster: the GEMM kernels are bound
-// by per-workgroup latency, not by fetch bandwidth.)
+// activation rows in one L2, measured no faster.)
 //
 // Exactness of the weights.  A Q4_0 block is (q - 8) * d with a per-row,
 // per-32-column f16 scale d.  Rounding (q - 8) * d to bf16 would cost 8 bits,
-// so the MFMA B operand is the exact bf16 value 128 + q (bit pattern 0x43,q:
-// one v_perm_b32 per two elements), the bias is removed by starting each
-// block's accumulation from sum_k x_k * (-136) (MFMAs against a constant
-// operand, shared by every column tile of the wavefront), and the block's
+// so the MFMA B operand is the exact bf16 value 16 + q, the bias is removed by
+// starting each block's accumulation from sum_k x_k * (-24), and the block's
 // fp32 result is scaled by d and accumulated in fp32.  Every product is exact
-// (bf16 x bf16 fits fp32); rounding happens only in the fp32 sums.
+// (bf16 x bf16 fits fp32); rounding happens only in the fp32 sums.  (128 + q
+// needs one shift less per operand, but starts the sums from -136 times the
+// activations: 3.3e-6 of y against 64 bits, 2.5e-6 with 16 + q.)
 // Activations: x is bf16 on entry (exact); h is split into bf16 hi + lo
-// (16 significant bits), so down runs two MFMAs per 16 k.
+// (16 significant bits), so down runs two MFMAs per block.
 //
-// v_mfma_f32_32x32x16_bf16 lane layout (l = lane, h = l / 32): A holds row
-// l % 32, k = 8h .. 8h + 7; B holds column l % 32, the same k; D holds column
-// l % 32, rows 8 (v / 4) + 4h + v % 4 for v = 0..15.  For a Q4 block the two
-// MFMAs take k 0..15 (low nibbles of qs bytes 8h..8h+7) and k 16..31 (high
-// nibbles of the same bytes).
+// v_mfma_f32_16x16x32_bf16 lane layout (l = lane, g = l / 16): A holds row l %
+// 16, k = 8g .. 8g + 7; B holds column l % 16, the same k; D holds column l %
+// 16, rows 4g + v for v = 0..3.  Both operands take the block's elements in the
+// order of the nibbles: k = 8g + i is element 4g + i for i < 4 (low nibbles of
+// qs dword g), 16 + 4g + i - 4 for i >= 4 (its high nibbles).
 #include <hip/hip_runtime.h>
 
 #include "tqf_device.h"
@@ -46,41 +45,61 @@ namespace tqf {
 namespace {
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
-constexpr int kTileM = 32;          // pairs per tile (MFMA rows)
 constexpr int kPlanThreads = 1024;
 constexpr int kPlanWaves = kPlanThreads / kWave;
-constexpr uint32_t kNeg136 = 0xC308C308u;  // bf16 pair (-136, -136)
 
-__device__ __forceinline__ bf16x8 load_bf16x8(const uint16_t *p) {
-    const u32x4 v = *(const __attribute__((address_space(1))) u32x4 *)(p);
+__device__ __forceinline__ f32x4 mfma(bf16x8 a, bf16x8 b, f32x4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
+}
+
+// Four qs bytes of a block -> the B operand 16 + q of their eight elements:
+// the low nibbles (elements 4g .. 4g + 3 for dword g), then the high nibbles
+// (elements 16 + 4g ..).  16 + q is bf16 0x4180 | q << 3.
+// `bit7` is 0x80808080 from a register (a shift and one v_and_or_b32 for four
+// nibbles: two literals do not fit one instruction).
+__device__ __forceinline__ bf16x8 biased_operand(uint32_t c, uint32_t bit7) {
+    constexpr uint32_t kHi = 0x41414141u, kSel01 = 0x04010400u, kSel23 = 0x04030402u;
+    const uint32_t l = ((c << 3) & 0x78787878u) | bit7, h = ((c >> 1) & 0x78787878u) | bit7;
+    const u32x4 v = {__builtin_amdgcn_perm(kHi, l, kSel01), __builtin_amdgcn_perm(kHi, l, kSel23),
+                     __builtin_amdgcn_perm(kHi, h, kSel01), __builtin_amdgcn_perm(kHi, h, kSel23)};
     return __builtin_bit_cast(bf16x8, v);
 }
 
-__device__ __forceinline__ f32x16 mfma(bf16x8 a, bf16x8 b, f32x16 c) {
-    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
-}
-
-// This lane's 8 qs bytes of one block (c0 = bytes 0..3, c1 = bytes 4..7 of
-// its half) -> B operands 128 + q for k 0..15 (lo) and k 16..31 (hi).
-__device__ __forceinline__ void biased_operands(uint32_t c0, uint32_t c1, bf16x8 &lo, bf16x8 &hi) {
-    constexpr uint32_t kExp = 0x43434343u, kSel01 = 0x04010400u, kSel23 = 0x04030402u;
-    const uint32_t l0 = c0 & 0x0F0F0F0Fu, l1 = c1 & 0x0F0F0F0Fu;
-    const uint32_t h0 = (c0 >> 4) & 0x0F0F0F0Fu, h1 = (c1 >> 4) & 0x0F0F0F0Fu;
-    const u32x4 a = {__builtin_amdgcn_perm(kExp, l0, kSel01), __builtin_amdgcn_perm(kExp, l0, kSel23),
-                     __builtin_amdgcn_perm(kExp, l1, kSel01), __builtin_amdgcn_perm(kExp, l1, kSel23)};
-    const u32x4 b = {__builtin_amdgcn_perm(kExp, h0, kSel01), __builtin_amdgcn_perm(kExp, h0, kSel23),
-                     __builtin_amdgcn_perm(kExp, h1, kSel01), __builtin_amdgcn_perm(kExp, h1, kSel23)};
-    lo = __builtin_bit_cast(bf16x8, a);
-    hi = __builtin_bit_cast(bf16x8, b);
-}
-
-// Row of D[v] for this lane.
-__device__ __forceinline__ int d_row(int v, int half) { return 8 * (v / 4) + 4 * half + (v % 4); }
-
 }  // namespace
+
+// Activations in the order of the MFMA operands.  The MFMA of a Q4 block reads
+// the block's 32 activations as four 16-byte pieces, piece g (for lane group
+// g) holding elements 4g .. 4g + 3 and 16 + 4g .. 16 + 4g + 3, which is the
+// order the nibbles of dword g come in.  A permuted row is [block][set][4
+// pieces]: one set for x, two (bf16 hi, lo) for h.  Beside it -24 times each
+// block's sum, [block][row], for the bias correction.  x is permuted by extra
+// workgroups of the plan launch, which end before the plan's own; h is written
+// this way by gate/up.
+constexpr float kBias = -24.0f;
+__device__ __forceinline__ float bf16_lo(uint32_t w) { return __uint_as_float(w << 16); }
+__device__ __forceinline__ float bf16_hi(uint32_t w) { return __uint_as_float(w & 0xFFFF0000u); }
+__device__ __forceinline__ uint32_t bf16_bits(float v) { return __builtin_bit_cast(uint16_t, (__bf16)v); }
+// Piece i of x [T x 32 blocks]: i = 4 (blocks t + block) + piece.
+__device__ __forceinline__ void permute_piece(const uint16_t *x, uint32_t i, uint32_t blocks, uint32_t T, uint4 *xp,
+                                              float *x_sums) {
+    const uint16_t *src = x + (size_t)(i >> 2) * 32 + (i & 3) * 4;  // x is 2-byte aligned only
+    uint32_t v[4];
+#pragma unroll
+    for (int d = 0; d < 4; ++d) {
+        const uint16_t *p = src + (d >> 1) * 16 + (d & 1) * 2;
+        v[d] = (uint32_t)p[0] | ((uint32_t)p[1] << 16);
+    }
+    xp[i] = make_uint4(v[0], v[1], v[2], v[3]);
+    float s = ((bf16_lo(v[0]) + bf16_hi(v[0])) + (bf16_lo(v[1]) + bf16_hi(v[1]))) +
+              ((bf16_lo(v[2]) + bf16_hi(v[2])) + (bf16_lo(v[3]) + bf16_hi(v[3])));
+    s += dpp_f<kDppXor1>(s);  // the block's four pieces are adjacent lanes
+    s += dpp_f<kDppXor2>(s);
+    const uint32_t q = i >> 2, t = q / blocks;
+    if ((i & 3) == 0) x_sums[(size_t)(q - t * blocks) * T + t] = kBias * s;
+}
 
 // ---- plan: counting sort of the (token, k) pairs by expert ------------------
 // Positions are stable in pair order (p = 8 t + k).  Workgroup b places the
@@ -91,15 +110,29 @@ __device__ __forceinline__ int d_row(int v, int half) { return 8 * (v / 4) + 4 *
 // wavefront, which one thread per expert turns into exclusive prefixes.  A
 // pair's position is base[e] (the exclusive scan of all counts) + the pairs
 // of e before the batch + its slot's prefix + its rank.  Workgroup 0 writes
-// the tile list: tile i of expert e covers positions off[e] + 32 i .. + rows;
-// an entry is {first position, e | rows << 16}.
+// the tile list.  An expert's c pairs make ceil(c / tile_m) tiles of equal size,
+// rounded up to 16 rows (the MFMA's); an entry is {first position, e | rows
+// << 16}.  The tiles of experts with more than 16 pairs come first: they take
+// longest.
 // Bound by its serial steps, not by bytes.  One workgroup that walked the
 // batches took 8.4-10.8 us at 4096 pairs and 74-88 us at 32768; this takes
 // 5.0-6.1 and 8.9-11.0 us.
+__device__ __forceinline__ int tile_rows(int c, int tile_m) {
+    const int n = (c + tile_m - 1) / tile_m;
+    return n ? ((c + n - 1) / n + 15) / 16 * 16 : 16;
+}
 __global__ __launch_bounds__(kPlanThreads) void gg_plan_kernel(
-    const uint16_t *__restrict__ ids, uint32_t pairs, uint32_t E, int32_t *__restrict__ pos_of_pair,
+    const uint16_t *__restrict__ ids, uint32_t pairs, uint32_t E, int tile_m, int32_t *__restrict__ pos_of_pair,
     int32_t *__restrict__ pair_of_pos, uint2 *__restrict__ tiles, int32_t *__restrict__ n_tiles,
-    int32_t *__restrict__ status) {
+    int32_t *__restrict__ status, const uint16_t *__restrict__ x, uint32_t x_blocks, uint4 *__restrict__ xp,
+    float *__restrict__ x_sums) {
+    const uint32_t plan_blocks = (pairs + kPlanThreads - 1) / kPlanThreads;
+    if (blockIdx.x >= plan_blocks) {
+        const uint32_t i = (blockIdx.x - plan_blocks) * kPlanThreads + threadIdx.x;
+        const uint32_t T = pairs / kTopK;
+        if (i < 4 * x_blocks * T) permute_piece(x, i, x_blocks, T, xp, x_sums);
+        return;
+    }
     __shared__ uint16_t cnt[kPlanWaves][256];  // this batch, per wavefront: count of expert e, then its prefix
     __shared__ int32_t before[256], after[256], total[256], base[256], tbase[256];
     __shared__ int32_t s_bad;
@@ -121,7 +154,7 @@ __global__ __launch_bounds__(kPlanThreads) void gg_plan_kernel(
         if (e < E) key = e;
         else s_bad = 1;
     }
-    if (gridDim.x > 1) {  // the other batches' ids, eight loads in flight per thread
+    if (plan_blocks > 1) {  // the other batches' ids, eight loads in flight per thread
         for (uint32_t r = tid; r < pairs; r += 8 * kPlanThreads) {
             uint32_t e[8];
 #pragma unroll
@@ -161,11 +194,12 @@ __global__ __launch_bounds__(kPlanThreads) void gg_plan_kernel(
     }
     __syncthreads();
     if (wave == 0) {  // exclusive scans of pair and tile counts, 4 experts per lane
-        int c[4], tc[4], s = 0, ts = 0;
+        int c[4], tc[4], s = 0, ts = 0;  // tile counts: over 16 pairs in the low half, others in the high half
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
             c[j] = total[4 * lane + j];
-            tc[j] = (c[j] + kTileM - 1) / kTileM;
+            tc[j] = (c[j] + tile_m - 1) / tile_m;
+            if (c[j] <= 16) tc[j] <<= 16;
             s += c[j];
             ts += tc[j];
         }
@@ -178,15 +212,16 @@ __global__ __launch_bounds__(kPlanThreads) void gg_plan_kernel(
                 its += y;
             }
         }
+        const int all = __shfl(its, kWave - 1), large = all & 0xFFFF;
         int o = is - s, to = its - ts;
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
             base[4 * lane + j] = o;
-            tbase[4 * lane + j] = to;
+            tbase[4 * lane + j] = tc[j] >> 16 ? large + (to >> 16) : to & 0xFFFF;
             o += c[j];
             to += tc[j];
         }
-        if (blockIdx.x == 0 && lane == kWave - 1) *n_tiles = its;
+        if (blockIdx.x == 0 && lane == 0) *n_tiles = large + (all >> 16);
     }
     __syncthreads();
     if (key < 256u) {
@@ -195,318 +230,342 @@ __global__ __launch_bounds__(kPlanThreads) void gg_plan_kernel(
         pair_of_pos[pos] = (int32_t)p;
     }
     if (blockIdx.x == 0 && tid < (int)E) {
-        const int c = total[tid];
-        for (int i = 0; i * kTileM < c; ++i) {
-            const int rows = c - i * kTileM < kTileM ? c - i * kTileM : kTileM;
-            tiles[tbase[tid] + i] = make_uint2((uint32_t)(base[tid] + i * kTileM), (uint32_t)tid | ((uint32_t)rows << 16));
+        const int c = total[tid], step = tile_rows(c, tile_m);
+        for (int i = 0; i * step < c; ++i) {
+            const int rows = c - i * step < step ? c - i * step : step;
+            tiles[tbase[tid] + i] = make_uint2((uint32_t)(base[tid] + i * step), (uint32_t)tid | ((uint32_t)rows << 16));
         }
     }
 }
 
 // ---- the tiled GEMMs -----------------------------------------------------------
-// A workgroup (8 wavefronts) owns one tile (<= 32 pairs of one expert) and 256
-// weight rows: gate/up takes 128 width columns of gate (wavefronts 0-3) and
-// the same 128 of up (4-7); down takes 256 hidden columns.  Each wavefront
-// runs the full K for its own 32 rows (one 32x32 MFMA tile), so there is no
-// cross-wave reduction, and the workgroup shares every staged byte.
-// K advances in chunks of 4 Q4 blocks (128 k): the workgroup loads chunk
-// c + 2 with coalesced 16 B buffer loads into registers while chunk c, in
-// LDS, feeds the MFMAs and chunk c + 1 waits in the other register set; one
-// barrier per chunk flips the two LDS stages.  While staging, four adjacent
-// lanes sum each activation row's 32-element block, so the bias correction
-// -136 * sum_k a_k enters the MFMA as its accumulator input (no extra MFMA).
-// LDS images of a chunk (pitches padded so that MFMA fragment reads are free
-// of bank conflicts):
-//   weights  [row][pair p][half h][block of pair][8 B]   (64 B + 16 B pad): a
-//            lane's 16 B read for (row n, pair p, half h) is its B operand
-//            bytes of both blocks of the pair;
-//   scales   [octet][block][8 rows x f16]                (as in HBM);
-//   acts     [set][row][128 x bf16]                      (256 B + 16 B pad);
-//   xs       [block][half h][16] f32: -136 * block sum over all activation
-//            sets of row 8 (v / 4) + 4 h + v % 4 at position v, i.e. already in
-//            the D-register order of the lanes of half h (one 64 B read).
-constexpr int kChunk = 4;            // Q4 blocks per K chunk
-constexpr int kGemmThreads = 512;
-constexpr int kGemmWaves = kGemmThreads / kWave;
-constexpr int kImgRows = 32 * kGemmWaves;  // weight rows per workgroup
-constexpr int kWPitch = 80;
-constexpr int kAPitch = 272;
-constexpr int kGUCols = kImgRows / 2;      // gate/up: width columns per workgroup
-constexpr int kDnCols = kImgRows;          // down: hidden columns per workgroup
+// A workgroup of 4 wavefronts owns one tile (<= 32 pairs of one expert), a
+// wavefront two 16-row MFMA subtiles of weights (in gate/up the same 16 rows of
+// gate and up, so SwiGLU stays in registers) for the full K.
+//
+// B operands are 16 + q in bf16.  The zero point and that bias (24 together)
+// are cancelled by starting each block's MFMA from -24 times the block's
+// activation sum; the result is scaled by the block's f16 scale in fp32.
+//
+// Everything comes through LDS with direct copies (buffer_load ... lds), so no
+// register holds a byte on its way and every weight request is a whole 128-byte
+// line: K advances in steps of 8 Q4 blocks, in which a row's nibbles are 128
+// contiguous bytes.  (Loading 4 blocks of 16 rows per instruction straight to
+// registers took 64-byte requests; their second halves came after the line had
+// left the L1, and issuing one group's loads took 1,600-23,000 clocks against
+// 2,500-3,500 for its arithmetic.)  Each wavefront copies its own weights, one
+// step ahead of its arithmetic where its stage is free; the activations and
+// their sums are copied by all of them, one stage per step (two with h's two
+// sets), between two barriers.  Stages are single: three or four workgroups per
+// CU run through each other's waits, and hide them better than two with
+// double-buffered stages do.
+//
+// Per 16 x 16 x 32 unit the vector ALU has 4 fmas (16 clocks) and 9 / MS
+// instructions for the B operand and the scale (MS: 16-row subtiles of the
+// tile); an MFMA is 16 clocks of the matrix cores and takes 8 of vector issue
+// (measured; v_permlane*_swap takes 8 as well); the LDS reads are about 11
+// clocks of the CU's LDS.  So tiles of 16 rows are bound by the weight stream,
+// long lists of full tiles by vector issue and LDS together.
+// Tiles have up to 32 rows, up to 64 where experts average 32 pairs or more
+// (half the operand work and weight traffic per row, against more workgroups in
+// flight: 1024 even tokens 232 us, 512 Zipf tokens 152 us a layer).
+// Measured, gate/up and down kernels in one run each (rocprof, medians): 37
+// Zipf tokens 40.9 + 28.2 -> 32.4 + 20.5 us, 512 116 + 80 -> 89 + 56 us, 4096
+// even tokens 411 + 286 -> 374 + 274 us against 32-row tiles of 8 wavefronts
+// that staged weights through registers.  Tried on the way at 4096 tokens and
+// no faster: 64-row tiles of 8 wavefronts with 4 subtiles each and the next
+// step's weights in flight (334 + 265 us, but 38 us for a lone tile, which a
+// short prompt waits for), double-buffered stages at two workgroups per CU (439
+// + 305), K started at a step of the workgroup's own (no change).
+constexpr int kStepBlocks = 8;
+constexpr int kGemmWaves = 4;
+constexpr int kSub = 2;  // weight subtiles per wavefront
 
-template <int NA>
-struct GemmStage {
-    uint8_t w[kImgRows * kWPitch];
-    uint8_t sc[(kImgRows / 8) * kChunk * 16];
-    uint8_t a[NA][kTileM * kAPitch];
-    float xs[kChunk][2][16];
+struct Desc { u32x4 v; };  // a buffer descriptor in scalar registers; loads past `bytes` return zero
+__device__ __forceinline__ Desc make_desc(const void *p, uint32_t bytes) {
+    const uint64_t a = (uint64_t)p;
+    Desc d;
+    d.v = u32x4{(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)a),
+                (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(a >> 32)) & 0xFFFFu, bytes, 0x00020000u};
+    return d;
+}
+// 16 (4) bytes per lane from descriptor + voff + soff to LDS byte lds + 16 (4) x lane.
+__device__ __forceinline__ void copy16(const Desc &d, uint32_t voff, uint32_t soff, uint32_t lds) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(lds), "v"(voff), "s"(d.v),
+                 "s"(soff)
+                 : "memory", "m0");
+}
+__device__ __forceinline__ void copy4(const Desc &d, uint32_t voff, uint32_t soff, uint32_t lds) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dword %1, %2, %3 offen lds" ::"s"(lds), "v"(voff), "s"(d.v),
+                 "s"(soff)
+                 : "memory", "m0");
+}
+// This wavefront's LDS reads and writes are done, then the workgroup's; publish:
+// its copies too.
+__device__ __forceinline__ void rendezvous() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+__device__ __forceinline__ void publish() { asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+typedef __attribute__((address_space(3))) uint8_t lds_byte;
+template <typename T>
+__device__ __forceinline__ T lds_load(uint32_t at) {
+    return *(const __attribute__((address_space(3))) T *)(at);
+}
+
+struct GroupedArgs {
+    const uint8_t *const *mats;
+    MatrixDims dims;        // of this GEMM's matrices
+    uint32_t mat_bytes;
+    uint32_t K, N;          // dims.cols, and the output's columns
+    const uint8_t *act;     // permuted activations [act_rows][K]
+    const float *sums;      // [K / 32][act_rows]
+    uint32_t act_rows;
+    const int32_t *pair_of_pos;
+    const uint2 *tiles;
+    const int32_t *n_tiles;
+    uint8_t *h;             // gate/up: permuted h, its sums [N / 32][h_rows]
+    float *h_sums;
+    uint32_t h_rows;
+    float *out;             // down
 };
-template <int NA>
-constexpr size_t gemm_lds_bytes() { return 2 * sizeof(GemmStage<NA>); }
 
-__device__ __forceinline__ uint4 lds_u4(const uint8_t *p) { return *reinterpret_cast<const uint4 *>(p); }
-__device__ __forceinline__ bf16x8 lds_bf16x8(const uint8_t *p) {
-    return __builtin_bit_cast(bf16x8, *reinterpret_cast<const u32x4 *>(p));
-}
+// GATE_UP: matrices 0 and 1 of the expert against x rows (the pair's token);
+// else matrix 2 against h rows (the position).
+//
+// LDS.  Per wavefront a weight stage: 4 octets x [8 rows][8 blocks][16 B], where
+// slot c of row r of octet o holds block c ^ r ^ (o & 1) (fragment reads free of
+// bank conflicts), then 4 octets x [8 blocks][8 rows] f16 scales.  Then the
+// activation stage, [block pair (one set) or block][row octet] x 1 KiB of
+// [block of pair or set][4 pieces][8 rows][16 B], and the sums, [block][rows].
+template <bool GATE_UP, int MS>
+struct TileGemm {
+    static constexpr int NW = kGemmWaves, NS = kSub;
+    static constexpr int kMats = GATE_UP ? 2 : 1, kSets = GATE_UP ? 1 : 2;  // matrices; activation sets
+    static constexpr int kPerMat = NS / kMats;                              // subtiles per matrix
+    static constexpr int kCols = 16 * kPerMat;                              // output columns per wavefront
+    static constexpr int kParts = kSets;              // activation stages per step: 8 blocks of one set, 4 of two
+    static constexpr int kBlocks = kStepBlocks / kParts;
+    static constexpr int kOctets = 2 * MS;            // row octets
+    static constexpr int kRowSets = (kOctets + NW - 1) / NW;  // octets a wavefront copies
+    static constexpr int kFence = kSets == 1 ? 8 : 2;
+    static constexpr int kCopies = 4;                 // 1 KiB activation copies per octet and stage
+    static constexpr uint32_t kWStage = NS * (2048 + 256), kAStage = kCopies * kOctets * 1024, kSumStage = kBlocks * MS * 64;
+    static constexpr uint32_t kLds = NW * kWStage + kAStage + kSumStage;
 
-// Loads go through buffer descriptors (base and byte range in SGPRs): each
-// thread keeps a 32-bit offset per piece for the whole K loop and the chunk
-// advances a scalar offset.  A load outside the descriptor's range returns
-// zero instead of touching memory.
-typedef __amdgpu_buffer_rsrc_t Rsrc;
-__device__ __forceinline__ Rsrc make_rsrc(const void *p, uint32_t bytes) {
-    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(p), (short)0, (int)bytes, 0x00020000);
-}
-__device__ __forceinline__ uint4 buf_u4(Rsrc r, uint32_t voff, uint32_t soff) {
-    const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(r, voff, soff, 0);
-    return make_uint4(v.x, v.y, v.z, v.w);
-}
+    uint32_t w_lds, a_lds, sum_lds;  // this wavefront's weights; the workgroup's activations and sums
+    Desc ws[kMats], as, cs;
+    uint32_t wv[2], sv, row16;       // weight offsets by octet parity, scale offset; bytes of a row's nibbles
+    uint32_t av[kRowSets], cv, act_rows;
+    int wave, lane;
 
-// One chunk in registers.  Thread t stages weight pieces (row, block j) t and
-// t + 512 of the 1024, scale piece t % 128 (duplicates write identical bytes:
-// no divergent branch, so the pipeline stays in one basic block) and the 16 B
-// piece (row t / 16, elements 8 (t % 16) ..) of every activation set.
-template <int NA>
-struct Chunk {
-    uint4 q[2];
-    uint4 s;
-    uint4 a[NA];
-};
-// Per-thread offsets of those pieces at k = 0 (the chunk adds b0 * 16 bytes
-// to weights and scales, k0 * 2 bytes to activations).
-template <int NA>
-struct ChunkOffsets {
-    uint32_t q[2], s, a;
-    int s_mat;  // matrix of the scale piece (uniform per wavefront)
-};
-
-template <int MATS, int NA>
-__device__ __forceinline__ ChunkOffsets<NA> chunk_offsets(const MatrixDims &dm, uint32_t n0, uint32_t a_row_off,
-                                                          int tid) {
-    constexpr int kPerMat = kImgRows / MATS;
-    ChunkOffsets<NA> o;
+    __device__ __forceinline__ TileGemm(const GroupedArgs &p, uint32_t lds, uint32_t pos0, uint32_t e, uint32_t rows,
+                                        uint32_t col0, int wave_, int lane_)
+        : wave(wave_), lane(lane_) {
+        w_lds = lds + wave * kWStage;
+        a_lds = lds + NW * kWStage;
+        sum_lds = a_lds + kAStage;
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
-        const int f = i * kGemmThreads + tid, r = f / kChunk, j = f % kChunk;
-        o.q[i] = (uint32_t)nibble_offset(dm, n0 + r % kPerMat, j);
+        for (int k = 0; k < kMats; ++k) ws[k] = make_desc(load_global_ptr(p.mats + e * 3 + (GATE_UP ? k : 2)), p.mat_bytes);
+        act_rows = p.act_rows;
+        as = make_desc(p.act, act_rows * p.K * 2 * kSets);
+        cs = make_desc(p.sums, act_rows * (p.K / 32) * 4);
+        row16 = p.dims.blocks_padded * 16;
+        const uint32_t r = lane >> 3, c = lane & 7, oct0 = col0 >> 3;
+#pragma unroll
+        for (uint32_t o = 0; o < 2; ++o) wv[o] = (oct0 * 9 + r) * row16 + ((c ^ r ^ o) & 7) * 16;
+        sv = ((oct0 + r) * 9 + 8) * row16 + c * 16;
+        // tile rows past the last take the first: read, not used
+        auto act_row = [&](uint32_t m) {
+            const uint32_t pos = pos0 + (m < rows ? m : 0u);
+            return GATE_UP ? (uint32_t)p.pair_of_pos[pos] / kTopK : pos;
+        };
+#pragma unroll
+        for (int i = 0; i < kRowSets; ++i)
+            av[i] = act_row(((wave + i * NW) % kOctets) * 8 + (lane & 7)) * (p.K * 2 * kSets) + (lane >> 3) * 16;
+        cv = act_row(lane) * 4;
     }
-    const int sp = tid % ((kImgRows / 8) * kChunk), oct = sp / kChunk, j = sp % kChunk;
-    o.s = (uint32_t)scale_offset(dm, n0 + (8 * oct) % kPerMat, j);
-    o.s_mat = __builtin_amdgcn_readfirstlane((8 * oct) / kPerMat);
-    o.a = a_row_off + (tid % 16) * 16;
-    return o;
-}
 
-template <int MATS, int NA>
-__device__ __forceinline__ void chunk_load(Chunk<NA> &c, const Rsrc (&ws)[MATS], const Rsrc (&as)[NA],
-                                           const ChunkOffsets<NA> &o, uint32_t chunk) {
-    constexpr int kPerMat = kImgRows / MATS;
-    const uint32_t b0 = chunk * kChunk, k0 = b0 * 32;
+    __device__ __forceinline__ void copy_weights(uint32_t step) const {
+        const uint32_t at = step * (kStepBlocks * 16);
 #pragma unroll
-    for (int i = 0; i < 2; ++i) c.q[i] = buf_u4(ws[(kImgRows / 2 * i) / kPerMat], o.q[i], b0 * 16);
-    c.s = buf_u4(MATS == 1 || o.s_mat == 0 ? ws[0] : ws[MATS - 1], o.s, b0 * 16);
+        for (int o = 0; o < 2 * NS; ++o)
+            copy16(ws[o / (2 * kPerMat)], wv[o & 1], at + (o % (2 * kPerMat)) * 9 * row16, w_lds + o * 1024);
 #pragma unroll
-    for (int n = 0; n < NA; ++n) c.a[n] = buf_u4(as[n], o.a, k0 * 2);
-}
-
-__device__ __forceinline__ float bf16_lo(uint32_t w) { return __uint_as_float(w << 16); }
-__device__ __forceinline__ float bf16_hi(uint32_t w) { return __uint_as_float(w & 0xFFFF0000u); }
-
-template <int NA>
-__device__ __forceinline__ void chunk_store(const Chunk<NA> &c, GemmStage<NA> &st, int tid) {
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-        const int f = i * kGemmThreads + tid, r = f / kChunk, j = f % kChunk;
-        uint8_t *row = st.w + r * kWPitch + (j >> 1) * 32 + (j & 1) * 8;
-        *reinterpret_cast<uint2 *>(row) = make_uint2(c.q[i].x, c.q[i].y);        // half 0
-        *reinterpret_cast<uint2 *>(row + 16) = make_uint2(c.q[i].z, c.q[i].w);   // half 1
+        for (int m = 0; m < kMats; ++m)
+            if (lane < 16 * kPerMat) copy16(ws[m], sv, at, w_lds + NS * 2048 + m * (kPerMat * 256));
     }
-    *reinterpret_cast<uint4 *>(st.sc + (tid % ((kImgRows / 8) * kChunk)) * 16) = c.s;
-    const int m = tid / 16, u = tid % 16;
-    float sum = 0.0f;
+    // Activation stage `at` of K (kBlocks blocks): [block pair (one set) or
+    // block][row octet] x 1 KiB, and the blocks' sums.
+    __device__ __forceinline__ void copy_act(uint32_t at) const {
+        constexpr int kShare = NW / kOctets > 1 ? NW / kOctets : 1;  // wavefronts that share an octet
 #pragma unroll
-    for (int n = 0; n < NA; ++n) {
-        *reinterpret_cast<uint4 *>(st.a[n] + m * kAPitch + u * 16) = c.a[n];
-        const uint32_t w4[4] = {c.a[n].x, c.a[n].y, c.a[n].z, c.a[n].w};
+        for (int i = 0; i < kRowSets; ++i) {
+            const int octet = kShare == 1 ? wave + i * NW : wave % kOctets;
+            if (kShare == 1 && octet >= kOctets) break;
 #pragma unroll
-        for (int d = 0; d < 4; ++d) sum += bf16_lo(w4[d]) + bf16_hi(w4[d]);
+            for (int c = 0; c < kCopies; ++c)
+                if (kShare == 1 || c % kShare == wave / kOctets)
+                    copy16(as, av[i], at * (kCopies * 128) + c * 128, a_lds + (c * kOctets + octet) * 1024);
+        }
+#pragma unroll
+        for (int b = 0; b < kBlocks; b += NW)
+            if (lane < 16 * MS) copy4(cs, cv, (at * kBlocks + b + wave) * act_rows * 4, sum_lds + (b + wave) * (MS * 64));
     }
-    // the 4 lanes of one block (pieces 4j .. 4j + 3 of the row) are adjacent;
-    // all four store the same sum (no divergent branch in the pipeline)
-    sum += __shfl_xor(sum, 1);
-    sum += __shfl_xor(sum, 2);
-    st.xs[u >> 2][(m >> 2) & 1][4 * (m >> 3) + (m & 3)] = -136.0f * sum;
-}
-
-// A fragments of block b (0..3 of the chunk) of set n for this lane (row = lane
-// % 32, half h): k 0..15 and 16..31 of the block.
-__device__ __forceinline__ void a_block(const uint8_t *img, int col, int half, int b, bf16x8 &lo, bf16x8 &hi) {
-    const uint8_t *r = img + col * kAPitch + (32 * b + 8 * half) * 2;
-    lo = lds_bf16x8(r);
-    hi = lds_bf16x8(r + 32);
-}
-
-// The correction of every D row of this lane (rows of D[v] are
-// 8 (v / 4) + 4 h + v % 4): one contiguous 64 B LDS read into the MFMA's
-// accumulator input.
-__device__ __forceinline__ f32x16 correction(const float (&xs)[2][16], int half) {
-    return *reinterpret_cast<const f32x16 *>(&xs[half][0]);
-}
-
-// One chunk of this wavefront's 32-row tile: per block, B operands of its row
-// from the weight image, MFMAs over every activation set starting from the
-// correction, fp32 scaling by the block's scale.
-template <int RG, int NA>
-__device__ __forceinline__ void chunk_mma(const GemmStage<NA> &s, uint32_t row, int col, int half,
-                                          float (&acc)[4 * RG]) {
+    // This lane's dword and scale of block b and subtile k in a weight stage:
+    // row n = lane % 16 of the subtile, dword lane / 16.
+    __device__ __forceinline__ uint32_t weight(int b, int k) const {
+        const uint32_t o = (lane >> 3) & 1, r = lane & 7;
+        return lds_load<uint32_t>(((w_lds + o * 1024 + r * 128 + ((r ^ o) << 4) + (lane >> 4) * 4) ^ (b << 4)) + k * 2048);
+    }
+    __device__ __forceinline__ uint16_t scale(int b, int k) const {
+        return lds_load<uint16_t>(w_lds + NS * 2048 + ((lane >> 3) & 1) * 128 + (lane & 7) * 2 + b * 16 + k * 256);
+    }
+    // The blocks of activation stage `part` of a step.
+    __device__ __forceinline__ void compute(int part, uint32_t bit7, f32x4 (&acc)[MS][NS]) const {
+        const uint32_t grp = lane >> 4, o = (lane >> 3) & 1, r = lane & 7;
+        const uint32_t al = a_lds + o * 1024 + grp * 128 + r * 16, cl = sum_lds + grp * 16;
 #pragma unroll
-    for (int p = 0; p < kChunk / 2; ++p) {
-        const uint4 q = lds_u4(s.w + row * kWPitch + p * 32 + half * 16);
-        const uint16_t *scp = reinterpret_cast<const uint16_t *>(s.sc + ((row >> 3) * kChunk + 2 * p) * 16) + (row & 7);
-        const float s0 = f16_to_f32(scp[0]), s1 = f16_to_f32(scp[8]);
+        for (int j = 0; j < kBlocks; ++j) {
+            const int b = kBlocks * part + j;
+            bf16x8 af[kSets][MS];
+            f32x4 t0[MS];
 #pragma unroll
-        for (int bb = 0; bb < 2; ++bb) {
-            const int b = 2 * p + bb;
-            bf16x8 lo, hi;
-            biased_operands(bb ? q.z : q.x, bb ? q.w : q.y, lo, hi);
-            f32x16 t = correction(s.xs[b], half);
+            for (int i = 0; i < MS; ++i) {
+                t0[i] = lds_load<f32x4>(cl + j * (MS * 64) + i * 64);
 #pragma unroll
-            for (int n = 0; n < NA; ++n) {
-                bf16x8 alo, ahi;
-                a_block(s.a[n], col, half, b, alo, ahi);
-                t = mfma(alo, lo, t);
-                t = mfma(ahi, hi, t);
+                for (int a = 0; a < kSets; ++a) {
+                    const int at = kSets == 1 ? (j >> 1) * kOctets * 1024 + (j & 1) * 512 : j * kOctets * 1024 + a * 512;
+                    af[a][i] = __builtin_bit_cast(bf16x8, lds_load<u32x4>(al + at + i * 2048));
+                }
             }
-            const float sb = bb ? s1 : s0;
 #pragma unroll
-            for (int v = 0; v < 4 * RG; ++v) acc[v] = fmaf(sb, t[v], acc[v]);
-            __builtin_amdgcn_sched_barrier(0);  // one block's operands live at a time
+            for (int k = 0; k < NS; ++k) {
+                const bf16x8 bw = biased_operand(weight(b, k), bit7);
+                const float s = f16_to_f32(scale(b, k));
+                f32x4 t[MS];
+#pragma unroll
+                for (int i = 0; i < MS; ++i) t[i] = mfma(af[0][i], bw, t0[i]);
+                if (kSets == 2) {
+#pragma unroll
+                    for (int i = 0; i < MS; ++i) t[i] = mfma(af[kSets - 1][i], bw, t[i]);
+                }
+#pragma unroll
+                for (int i = 0; i < MS; ++i)
+#pragma unroll
+                    for (int v = 0; v < 4; ++v) acc[i][k][v] = fmaf(s, t[i][v], acc[i][k][v]);
+            }
+            if (j % kFence == kFence - 1) __builtin_amdgcn_sched_barrier(0);  // bounds the reads the compiler moves up
+        }
+        // the sums are values here: moved past the next branch, they would keep
+        // every MFMA result of the stage live
+#pragma unroll
+        for (int i = 0; i < MS; ++i)
+#pragma unroll
+            for (int k = 0; k < NS; ++k) asm volatile("" : "+v"(acc[i][k]));
+    }
+
+    __device__ __forceinline__ void run(uint32_t steps, f32x4 (&acc)[MS][NS]) const {
+        uint32_t bit7;
+        asm("v_mov_b32 %0, 0x80808080" : "=v"(bit7));
+#pragma unroll
+        for (int i = 0; i < MS; ++i)
+#pragma unroll
+            for (int k = 0; k < NS; ++k) acc[i][k] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+        copy_weights(0);
+        for (uint32_t s = 0; s < steps; ++s) {
+#pragma unroll
+            for (int part = 0; part < kParts; ++part) {
+                if (part > 0 || s > 0) rendezvous();  // every wavefront has read the last stage
+                copy_act(kParts * s + part);
+                publish();
+                compute(part, bit7, acc);
+            }
+            if (s + 1 < steps) {
+                asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the weights are read before they are overwritten
+                copy_weights(s + 1);
+            }
         }
     }
-}
+};
 
-// The pipelined K loop of one workgroup (chunks even: K is a multiple of 256).
-template <int RG, int MATS, int NA>
-__device__ __forceinline__ void gemm_tile(GemmStage<NA> *sm, const Rsrc (&ws)[MATS], const Rsrc (&as)[NA],
-                                          const ChunkOffsets<NA> &o, uint32_t chunks, uint32_t row,
-                                          int tid, int col, int half, float (&acc)[4 * RG]) {
+// SwiGLU of column col0 + n of rows 16 i + 4 grp + v (n = lane % 16, grp = lane
+// / 16) into the permuted h; even lanes store the hi parts of columns n, n + 1,
+// odd lanes the lo parts of n - 1, n.  A 32-column block spans two wavefronts,
+// whose halves of its sum meet in LDS (at ps, 64 floats per wavefront).
+template <int MS>
+__device__ __forceinline__ void store_h(const GroupedArgs &p, const f32x4 (&acc)[MS][kSub], uint32_t ps, uint32_t pos0,
+                                        uint32_t rows, uint32_t col0, int wave, int lane) {
+    const uint32_t n = lane & 15, grp = lane >> 4, blk = col0 >> 5;
+    const uint32_t in_block = (n & 1) * 64 + (n >> 2) * 16 + (wave & 1) * 8 + (n & 2) * 2;
+    rendezvous();  // every wavefront is done with the stages
 #pragma unroll
-    for (int v = 0; v < 4 * RG; ++v) acc[v] = 0.0f;
-    Chunk<NA> c0, c1;
-    chunk_load<MATS, NA>(c0, ws, as, o, 0);
-    chunk_store<NA>(c0, sm[0], tid);
-    __syncthreads();
-    chunk_load<MATS, NA>(c1, ws, as, o, 1);
-    for (uint32_t c = 0; c + 2 < chunks; c += 2) {
-        chunk_load<MATS, NA>(c0, ws, as, o, c + 2);
-        chunk_mma<RG, NA>(sm[0], row, col, half, acc);
-        chunk_store<NA>(c1, sm[1], tid);
-        __syncthreads();
-        chunk_load<MATS, NA>(c1, ws, as, o, c + 3);
-        chunk_mma<RG, NA>(sm[1], row, col, half, acc);
-        chunk_store<NA>(c0, sm[0], tid);
-        __syncthreads();
-    }
-    chunk_mma<RG, NA>(sm[0], row, col, half, acc);
-    chunk_store<NA>(c1, sm[1], tid);
-    __syncthreads();
-    chunk_mma<RG, NA>(sm[1], row, col, half, acc);
-}
-
-template <int MATS, int NA>
-__device__ __forceinline__ void gemm_dispatch(int rg, GemmStage<NA> *sm, const Rsrc (&ws)[MATS],
-                                              const Rsrc (&as)[NA], const ChunkOffsets<NA> &o,
-                                              uint32_t chunks, uint32_t row, int tid, int col, int half,
-                                              float (&acc)[16]) {
-    switch (rg) {
-        case 1: gemm_tile<1, MATS, NA>(sm, ws, as, o, chunks, row, tid, col, half,
-                                       *reinterpret_cast<float(*)[4]>(acc)); break;
-        case 2: gemm_tile<2, MATS, NA>(sm, ws, as, o, chunks, row, tid, col, half,
-                                       *reinterpret_cast<float(*)[8]>(acc)); break;
-        case 3: gemm_tile<3, MATS, NA>(sm, ws, as, o, chunks, row, tid, col, half,
-                                       *reinterpret_cast<float(*)[12]>(acc)); break;
-        default: gemm_tile<4, MATS, NA>(sm, ws, as, o, chunks, row, tid, col, half, acc); break;
-    }
-}
-
-// ---- gate/up + SwiGLU --------------------------------------------------------
-__global__ __launch_bounds__(kGemmThreads) __attribute__((amdgpu_waves_per_eu(4))) void gg_gate_up_kernel(
-    const uint8_t *const *__restrict__ mats, MatrixDims dg, uint32_t mat_bytes,
-    const uint16_t *__restrict__ x, uint32_t x_bytes, const int32_t *__restrict__ pair_of_pos,
-    const uint2 *__restrict__ tiles, const int32_t *__restrict__ n_tiles, uint32_t H, uint32_t F,
-    uint16_t *__restrict__ h_hi, uint16_t *__restrict__ h_lo) {
-    extern __shared__ uint4 gg_smem[];
-    GemmStage<1> *sm = reinterpret_cast<GemmStage<1> *>(gg_smem);
-    if ((int)blockIdx.y >= *n_tiles) return;
-    const int tid = threadIdx.x;
-    const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
-    const int lane = tid % kWave, half = lane >> 5, col = lane & 31;
-    const uint2 tl = tiles[blockIdx.y];
-    const uint32_t pos0 = tl.x, e = tl.y & 0xFFFFu, rows = tl.y >> 16;
-    const Rsrc ws[2] = {make_rsrc(load_global_ptr(mats + e * 3 + 0), mat_bytes),
-                        make_rsrc(load_global_ptr(mats + e * 3 + 1), mat_bytes)};
-    const Rsrc as[1] = {make_rsrc(x, x_bytes)};
-    const uint32_t n0 = blockIdx.x * kGUCols;
-    const uint32_t m = tid / 16;  // the activation row this thread stages (clamped to a real row)
-    const uint32_t tok = (uint32_t)pair_of_pos[pos0 + (m < rows ? m : 0u)] / kTopK;
-    const ChunkOffsets<1> o = chunk_offsets<2, 1>(dg, n0, tok * H * 2, tid);
-    const int rg = __builtin_amdgcn_readfirstlane((int)(rows + 7) / 8);
-    float acc[16];
-    gemm_dispatch<2, 1>(rg, sm, ws, as, o, H / 32 / kChunk, (uint32_t)(32 * wave + col), tid, col, half, acc);
-    // SwiGLU: the up wavefronts hand their tile to the gate wavefronts in LDS
-    __syncthreads();
-    float *xu = reinterpret_cast<float *>(gg_smem);  // [4 waves][16][64]
-    if (wave >= kGemmWaves / 2) {
+    for (int i = 0; i < MS; ++i)
 #pragma unroll
-        for (int v = 0; v < 16; ++v)
-            if (v < 4 * rg) xu[((wave - kGemmWaves / 2) * 16 + v) * kWave + lane] = acc[v];
-    }
-    __syncthreads();
-    if (wave >= kGemmWaves / 2) return;
-#pragma unroll
-    for (int v = 0; v < 16; ++v) {
-        if (v >= 4 * rg) break;
-        const uint32_t r = (uint32_t)d_row(v, half);
-        if (r < rows) {
-            const float g = acc[v], u = xu[(wave * 16 + v) * kWave + lane];
+        for (int v = 0; v < 4; ++v) {
+            const float g = acc[i][0][v], u = acc[i][1][v];
             const float hv = (g / (1.0f + expf(-g))) * u;
-            const __bf16 hb = (__bf16)hv;
-            const __bf16 lb = (__bf16)(hv - (float)hb);
-            const size_t off = (size_t)(pos0 + r) * F + n0 + 32 * wave + col;
-            h_hi[off] = __builtin_bit_cast(uint16_t, hb);
-            h_lo[off] = __builtin_bit_cast(uint16_t, lb);
+            const uint32_t hi = bf16_bits(hv), lo = bf16_bits(hv - bf16_lo(hi));
+            float sum = bf16_lo(hi) + bf16_lo(lo);
+            sum += dpp_f<kDppXor1>(sum);
+            sum += dpp_f<kDppXor2>(sum);
+            sum += dpp_f<kDppHalfMirror>(sum);
+            sum += dpp_f<kDppMirror>(sum);
+            const uint32_t hi1 = (uint32_t)dpp_i<kDppXor1>((int)hi), lo1 = (uint32_t)dpp_i<kDppXor1>((int)lo);
+            const uint32_t r = 16 * i + 4 * grp + v;
+            if (n == 0) *(__attribute__((address_space(3))) float *)(ps + (wave * 64 + r) * 4) = sum;
+            if (r < rows)
+                *reinterpret_cast<uint32_t *>(p.h + ((size_t)(pos0 + r) * (p.N >> 5) + blk) * 128 + in_block) =
+                    n & 1 ? lo1 | (lo << 16) : hi | (hi1 << 16);
         }
+    rendezvous();
+    const uint32_t q = wave, r = lane;  // the workgroup's block q, row r
+    if (q < kGemmWaves / 2 && r < rows) {
+        const float s = lds_load<float>(ps + (2 * q * 64 + r) * 4) + lds_load<float>(ps + ((2 * q + 1) * 64 + r) * 4);
+        p.h_sums[(size_t)(blk - (wave >> 1) + q) * p.h_rows + pos0 + r] = kBias * s;
     }
 }
-
-// ---- down ------------------------------------------------------------------
-__global__ __launch_bounds__(kGemmThreads) __attribute__((amdgpu_waves_per_eu(4))) void gg_down_kernel(
-    const uint8_t *const *__restrict__ mats, MatrixDims dd, uint32_t mat_bytes,
-    const uint16_t *__restrict__ h_hi, const uint16_t *__restrict__ h_lo, uint32_t h_bytes,
-    const uint2 *__restrict__ tiles, const int32_t *__restrict__ n_tiles, uint32_t H, uint32_t F,
-    float *__restrict__ out) {
-    extern __shared__ uint4 gg_smem[];
-    GemmStage<2> *sm = reinterpret_cast<GemmStage<2> *>(gg_smem);
-    if ((int)blockIdx.y >= *n_tiles) return;
-    const int tid = threadIdx.x;
-    const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
-    const int lane = tid % kWave, half = lane >> 5, col = lane & 31;
-    const uint2 tl = tiles[blockIdx.y];
-    const uint32_t pos0 = tl.x, e = tl.y & 0xFFFFu, rows = tl.y >> 16;
-    const Rsrc ws[1] = {make_rsrc(load_global_ptr(mats + e * 3 + 2), mat_bytes)};
-    const Rsrc as[2] = {make_rsrc(h_hi, h_bytes), make_rsrc(h_lo, h_bytes)};
-    const uint32_t n0 = blockIdx.x * kDnCols;
-    const uint32_t m = tid / 16;
-    const ChunkOffsets<2> o = chunk_offsets<1, 2>(dd, n0, (pos0 + (m < rows ? m : 0u)) * F * 2, tid);
-    const int rg = __builtin_amdgcn_readfirstlane((int)(rows + 7) / 8);
-    float acc[16];
-    gemm_dispatch<1, 2>(rg, sm, ws, as, o, F / 32 / kChunk, (uint32_t)(32 * wave + col), tid, col, half, acc);
+// Even lanes store subtile 0's columns n, n + 1, odd lanes subtile 1's n - 1, n.
+template <int MS>
+__device__ __forceinline__ void store_out(const GroupedArgs &p, const f32x4 (&acc)[MS][kSub], uint32_t pos0, uint32_t rows,
+                                          uint32_t col0, int lane) {
+    const uint32_t n = lane & 15, odd = n & 1;
 #pragma unroll
-    for (int v = 0; v < 16; ++v) {
-        if (v >= 4 * rg) break;
-        const uint32_t r = (uint32_t)d_row(v, half);
-        if (r < rows) out[(size_t)(pos0 + r) * H + n0 + 32 * wave + col] = acc[v];
-    }
+    for (int i = 0; i < MS; ++i)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            const float got = dpp_f<kDppXor1>(odd ? acc[i][0][v] : acc[i][1][v]);
+            const uint32_t r = 16 * i + 4 * (lane >> 4) + v;
+            if (r < rows)
+                *reinterpret_cast<float2 *>(p.out + (size_t)(pos0 + r) * p.N + col0 + odd * 16 + (n & 14)) =
+                    odd ? make_float2(got, acc[i][1][v]) : make_float2(acc[i][0][v], got);
+        }
+}
+
+template <bool GATE_UP, int MS>
+__device__ __forceinline__ void tile_pass(const GroupedArgs &p, uint32_t lds, uint32_t pos0, uint32_t e, uint32_t rows,
+                                          int wave, int lane) {
+    using G = TileGemm<GATE_UP, MS>;
+    const uint32_t col0 = (blockIdx.x * kGemmWaves + wave) * G::kCols;
+    const G g(p, lds, pos0, e, rows, col0, wave, lane);
+    f32x4 acc[MS][kSub];
+    g.run(p.K / (32 * kStepBlocks), acc);
+    if constexpr (GATE_UP) store_h<MS>(p, acc, g.a_lds, pos0, rows, col0, wave, lane);
+    else store_out<MS>(p, acc, pos0, rows, col0, lane);
+}
+
+template <bool GATE_UP, int MAX_MS>
+__global__ __launch_bounds__(kGemmWaves * kWave) __attribute__((amdgpu_waves_per_eu(MAX_MS == 2 ? 4 : 3,
+                                                                                  MAX_MS == 2 ? 4 : 3))) void
+gg_gemm_kernel(GroupedArgs p) {
+    extern __shared__ uint4 gg_smem[];
+    const uint32_t lds = (uint32_t)(uintptr_t)(lds_byte *)(uint8_t *)gg_smem;
+    if ((int)blockIdx.y >= *p.n_tiles) return;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x % kWave;
+    const uint2 tl = p.tiles[blockIdx.y];
+    const uint32_t pos0 = __builtin_amdgcn_readfirstlane(tl.x), er = __builtin_amdgcn_readfirstlane(tl.y);
+    const uint32_t e = er & 0xFFFFu, rows = er >> 16;
+    if (MAX_MS == 4 && rows > 48) tile_pass<GATE_UP, MAX_MS>(p, lds, pos0, e, rows, wave, lane);
+    else if (MAX_MS == 4 && rows > 32) tile_pass<GATE_UP, MAX_MS - 1>(p, lds, pos0, e, rows, wave, lane);
+    else if (rows > 16) tile_pass<GATE_UP, 2>(p, lds, pos0, e, rows, wave, lane);
+    else tile_pass<GATE_UP, 1>(p, lds, pos0, e, rows, wave, lane);
 }
 
 // ---- combine: y[t] = sum_k w[t,k] * out[pos(t,k)], k in route order ----------
@@ -537,69 +596,105 @@ __global__ __launch_bounds__(256) void gg_combine_kernel(const float *__restrict
 // ---- host side ----------------------------------------------------------------
 namespace {
 size_t round256(size_t v) { return (v + 255) / 256 * 256; }
+// Most rows of a tile: 64 where experts average at least 32 pairs.
+int tile_m_for(uint32_t T, uint32_t E) { return T * kTopK >= 32 * E ? 64 : 32; }
 uint32_t max_tiles_for(uint32_t T, uint32_t E) {
     const uint32_t P = T * kTopK;
-    return (P + kTileM - 1) / kTileM + (E < P ? E : P);
+    return P / tile_m_for(T, E) + (E < P ? E : P);
+}
+
+template <bool GATE_UP, int MAX_MS>
+hipError_t launch_tiles(hipStream_t s, const GroupedArgs &p, uint32_t tiles) {
+    using G = TileGemm<GATE_UP, MAX_MS>;
+    static const hipError_t attr = hipFuncSetAttribute((const void *)gg_gemm_kernel<GATE_UP, MAX_MS>,
+                                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)G::kLds);
+    if (attr != hipSuccess) return attr;
+    hipLaunchKernelGGL((gg_gemm_kernel<GATE_UP, MAX_MS>), dim3(p.N / (kGemmWaves * G::kCols), tiles), dim3(kGemmWaves * kWave),
+                       G::kLds, s, p);
+    return hipGetLastError();
+}
+
+template <bool GATE_UP>
+hipError_t launch_grouped_gemm(hipStream_t s, const LayerDev &L, const GroupedBuffers &g) {
+    const uint32_t P = g.tokens * kTopK;
+    GroupedArgs p;
+    p.mats = L.mats;
+    p.dims = GATE_UP ? matrix_dims(L.width, L.hidden) : matrix_dims(L.hidden, L.width);
+    p.mat_bytes = (uint32_t)layout_bytes(p.dims);
+    p.K = GATE_UP ? L.hidden : L.width;
+    p.N = GATE_UP ? L.width : L.hidden;
+    p.act = GATE_UP ? g.x : g.h;
+    p.act_rows = GATE_UP ? g.tokens : P;
+    p.sums = GATE_UP ? g.x_sums : g.h_sums;
+    p.pair_of_pos = g.pair_of_pos;
+    p.tiles = g.tiles;
+    p.n_tiles = g.n_tiles;
+    p.h = g.h;
+    p.h_sums = g.h_sums;
+    p.h_rows = P;
+    p.out = g.out;
+    return tile_m_for(g.tokens, L.n_experts) == 64 ? launch_tiles<GATE_UP, 4>(s, p, g.max_tiles)
+                                                   : launch_tiles<GATE_UP, 2>(s, p, g.max_tiles);
+}
+
+template <typename F>
+void carve(uint32_t T, uint32_t E, uint32_t H, uint32_t W, F take) {
+    const size_t P = (size_t)T * kTopK;
+    take(P * 4);                                                // pos_of_pair
+    take(P * 4);                                                // pair_of_pos
+    take((size_t)max_tiles_for(T, E) * 8);                      // tiles
+    take(256);                                                  // n_tiles
+    take((size_t)T * H * 2);                                    // x, permuted
+    take((size_t)T * H / 8);                                    // x_sums
+    take(P * W * 4);                                            // h, permuted
+    take(P * W / 8);                                            // h_sums
+    take(P * H * 4);                                            // out
 }
 }  // namespace
 
 size_t grouped_scratch_bytes(uint32_t T, uint32_t E, uint32_t H, uint32_t F) {
-    const size_t P = (size_t)T * kTopK;
-    return 2 * round256(P * 4) + round256((size_t)max_tiles_for(T, E) * 8) + 256 +
-           2 * round256(P * F * 2) + round256(P * H * 4);
+    size_t sum = 0;
+    carve(T, E, H, F, [&](size_t bytes) { sum += round256(bytes); });
+    return sum;
 }
 
 GroupedBuffers grouped_buffers(void *scratch, uint32_t T, uint32_t E, uint32_t H, uint32_t F) {
-    const size_t P = (size_t)T * kTopK;
-    uint8_t *p = static_cast<uint8_t *>(scratch);
-    auto take = [&](size_t bytes) {
-        uint8_t *r = p;
+    uint8_t *part[9], *p = static_cast<uint8_t *>(scratch);
+    int n = 0;
+    carve(T, E, H, F, [&](size_t bytes) {
+        part[n++] = p;
         p += round256(bytes);
-        return r;
-    };
+    });
     GroupedBuffers g;
-    g.pos_of_pair = reinterpret_cast<int32_t *>(take(P * 4));
-    g.pair_of_pos = reinterpret_cast<int32_t *>(take(P * 4));
     g.tokens = T;
     g.max_tiles = max_tiles_for(T, E);
-    g.tiles = reinterpret_cast<uint2 *>(take((size_t)g.max_tiles * 8));
-    g.n_tiles = reinterpret_cast<int32_t *>(take(256));
-    g.h_hi = reinterpret_cast<uint16_t *>(take(P * F * 2));
-    g.h_lo = reinterpret_cast<uint16_t *>(take(P * F * 2));
-    g.out = reinterpret_cast<float *>(take(P * H * 4));
+    g.pos_of_pair = reinterpret_cast<int32_t *>(part[0]);
+    g.pair_of_pos = reinterpret_cast<int32_t *>(part[1]);
+    g.tiles = reinterpret_cast<uint2 *>(part[2]);
+    g.n_tiles = reinterpret_cast<int32_t *>(part[3]);
+    g.x = part[4];
+    g.x_sums = reinterpret_cast<float *>(part[5]);
+    g.h = part[6];
+    g.h_sums = reinterpret_cast<float *>(part[7]);
+    g.out = reinterpret_cast<float *>(part[8]);
     return g;
 }
 
-hipError_t launch_grouped_plan(hipStream_t s, const uint16_t *ids, uint32_t T, uint32_t E,
+hipError_t launch_grouped_plan(hipStream_t s, const uint16_t *ids, const uint16_t *x, uint32_t T, uint32_t E, uint32_t H,
                                const GroupedBuffers &g, int32_t *status) {
-    hipLaunchKernelGGL(gg_plan_kernel, dim3((T * kTopK + kPlanThreads - 1) / kPlanThreads), dim3(kPlanThreads), 0, s, ids, T * kTopK, E,
-                       g.pos_of_pair, g.pair_of_pos, g.tiles, g.n_tiles, status);
+    const uint32_t pairs = T * kTopK, pieces = T * H / 8;
+    const uint32_t blocks = (pairs + kPlanThreads - 1) / kPlanThreads + (pieces + kPlanThreads - 1) / kPlanThreads;
+    hipLaunchKernelGGL(gg_plan_kernel, dim3(blocks), dim3(kPlanThreads), 0, s, ids, pairs, E, tile_m_for(T, E), g.pos_of_pair, g.pair_of_pos,
+                       g.tiles, g.n_tiles, status, x, H / 32, reinterpret_cast<uint4 *>(g.x), g.x_sums);
     return hipGetLastError();
 }
 
-hipError_t launch_grouped_gate_up(hipStream_t s, const LayerDev &L, const uint16_t *x,
-                                  const GroupedBuffers &g) {
-    static const hipError_t attr = hipFuncSetAttribute(
-        (const void *)gg_gate_up_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)gemm_lds_bytes<1>());
-    if (attr != hipSuccess) return attr;
-    const MatrixDims dg = matrix_dims(L.width, L.hidden);
-    hipLaunchKernelGGL(gg_gate_up_kernel, dim3(L.width / kGUCols, g.max_tiles), dim3(kGemmThreads),
-                       gemm_lds_bytes<1>(), s, L.mats, dg, (uint32_t)layout_bytes(dg), x,
-                       g.tokens * L.hidden * 2, g.pair_of_pos, g.tiles, g.n_tiles, L.hidden,
-                       L.width, g.h_hi, g.h_lo);
-    return hipGetLastError();
+hipError_t launch_grouped_gate_up(hipStream_t s, const LayerDev &L, const GroupedBuffers &g) {
+    return launch_grouped_gemm<true>(s, L, g);
 }
 
 hipError_t launch_grouped_down(hipStream_t s, const LayerDev &L, const GroupedBuffers &g) {
-    static const hipError_t attr = hipFuncSetAttribute(
-        (const void *)gg_down_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)gemm_lds_bytes<2>());
-    if (attr != hipSuccess) return attr;
-    const MatrixDims dd = matrix_dims(L.hidden, L.width);
-    hipLaunchKernelGGL(gg_down_kernel, dim3(L.hidden / kDnCols, g.max_tiles), dim3(kGemmThreads),
-                       gemm_lds_bytes<2>(), s, L.mats, dd, (uint32_t)layout_bytes(dd), g.h_hi,
-                       g.h_lo, g.tokens * kTopK * L.width * 2, g.tiles, g.n_tiles, L.hidden,
-                       L.width, g.out);
-    return hipGetLastError();
+    return launch_grouped_gemm<false>(s, L, g);
 }
 
 hipError_t launch_grouped_combine(hipStream_t s, const GroupedBuffers &g, const float *w,

@@ -541,24 +541,23 @@ hipError_t launch_q6k_q8k_gemv(hipStream_t s, const uint8_t *const *tables, uint
 
 // ---- grouped expert GEMM (tqf_grouped.hip) --------------------------------
 // Scratch views of one call over T tokens (P = 8 T pairs): the expert-sorted
-// positions, the tile list, h (bf16 hi and lo, [P x width]) and the
-// per-pair expert outputs ([P x hidden] f32).  Shapes: hidden and width
-// multiples of 256, at most 256 experts.
+// positions, the tile list, x [T x hidden] and h (bf16 hi and lo, [P x width]) in MFMA operand
+// order with their block sums, and the per-pair expert outputs ([P x hidden]
+// f32).  Shapes: hidden and width multiples of 256, at most 256 experts.
 struct GroupedBuffers {
     int32_t *pos_of_pair, *pair_of_pos, *n_tiles;
     uint2 *tiles;
-    uint16_t *h_hi, *h_lo;
-    float *out;
+    uint8_t *x, *h;
+    float *x_sums, *h_sums, *out;
     uint32_t tokens, max_tiles;
 };
 size_t grouped_scratch_bytes(uint32_t T, uint32_t E, uint32_t H, uint32_t F);
 GroupedBuffers grouped_buffers(void *scratch, uint32_t T, uint32_t E, uint32_t H, uint32_t F);
 // status (may be null) is set to TQF_HIP_ERR_INVALID when an id is >= E; the
 // later kernels then do nothing.
-hipError_t launch_grouped_plan(hipStream_t s, const uint16_t *ids, uint32_t T, uint32_t E,
-                               const GroupedBuffers &g, int32_t *status);
-hipError_t launch_grouped_gate_up(hipStream_t s, const LayerDev &L, const uint16_t *x_bf16,
-                                  const GroupedBuffers &g);
+hipError_t launch_grouped_plan(hipStream_t s, const uint16_t *ids, const uint16_t *x_bf16, uint32_t T, uint32_t E,
+                               uint32_t H, const GroupedBuffers &g, int32_t *status);
+hipError_t launch_grouped_gate_up(hipStream_t s, const LayerDev &L, const GroupedBuffers &g);
 hipError_t launch_grouped_down(hipStream_t s, const LayerDev &L, const GroupedBuffers &g);
 hipError_t launch_grouped_combine(hipStream_t s, const GroupedBuffers &g, const float *w,
                                   uint32_t T, uint32_t H, float *y);
