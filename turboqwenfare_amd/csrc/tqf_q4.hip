@@ -178,13 +178,24 @@ hipError_t launch_gemv(hipStream_t s, const uint8_t *const *d_tables, uint32_t c
 // descending top-8 with ties to the lower id, renormalise) and the pair
 // plan, and advances the launch count.  The poll is bounded in time; a
 // timeout writes a failed plan (TQF_HIP_ERR_DEVICE).
+// Bound by the chain of its latencies (loads, two block sums, the words' round
+// trip, softmax and top-8), not by its 2.1 MB: 7.7 / 10.4 us with the norm at 1
+// / 4 tokens (9.0 / 11.8 while the norm's weights were loaded behind the sum of
+// squares), 14.0 us at 8 (23.2 with 256 threads, which spilled 272 bytes a
+// thread building the records).
 // ---------------------------------------------------------------------------
 constexpr int kRouteRows = 2;
 constexpr int64_t kRouteSpinLimit = 2000000;  // wall-clock ticks (100 MHz): 20 ms
 constexpr int kRouteSeq = 1;                   // the launch count's counter slot
 
+// The first 256 threads hold the rows' elements.  For more than four tokens
+// there are 512: one wavefront per token in workgroup 0's routing, where four
+// took two each.
 template <int MT>
-__global__ __launch_bounds__(256) void route_kernel(LayerDev L, const float *__restrict__ h,
+constexpr int kRouteThreads = MT <= 4 ? 256 : 512;
+
+template <int MT>
+__global__ __launch_bounds__(kRouteThreads<MT>) void route_kernel(LayerDev L, const float *__restrict__ h,
                                                     const float *__restrict__ norm, uint32_t m,
                                                     uint32_t bp, uint32_t *__restrict__ xprep,
                                                     uint64_t *__restrict__ logits,
@@ -201,8 +212,10 @@ __global__ __launch_bounds__(256) void route_kernel(LayerDev L, const float *__r
     __shared__ int s_ids[kMaxTokens * kTopK];
     __shared__ float s_w[kMaxTokens * kTopK];
     __shared__ float s_gate[kMaxTokens];
+    __shared__ float s_blk[MT][32];
 
     const int tid = threadIdx.x;
+    const bool front = kRouteThreads<MT> == 256 || tid < 256;
     const uint32_t seq = __hip_atomic_load(&counter[kRouteSeq], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     const uint32_t tag = 0x80000000u | (seq & 0x7FFFFFFFu);
     const uint32_t H = L.hidden, E = L.n_experts;
@@ -213,9 +226,11 @@ __global__ __launch_bounds__(256) void route_kernel(LayerDev L, const float *__r
     // overlaps the activation loads and the records below
     // (the model geometry, hidden 2048, loads 8 contiguous floats per thread
     // as two 16-byte loads; other widths element by element)
-    float wv[kRouteRows][8];
-    float x[MT][8];
-    if (vpt == 8) {
+    float wv[kRouteRows][8] = {};
+    float x[MT][8] = {};
+    float nw[8] = {};  // the norm's weights: loaded here, not behind the sum of squares
+    if (!front) {
+    } else if (vpt == 8) {
 #pragma unroll
         for (int rr = 0; rr < kRouteRows; ++rr) {
             const uint32_t r = blockIdx.x * kRouteRows + rr;
@@ -233,6 +248,11 @@ __global__ __launch_bounds__(256) void route_kernel(LayerDev L, const float *__r
             x[t][0] = a.x; x[t][1] = a.y; x[t][2] = a.z; x[t][3] = a.w;
             x[t][4] = b.x; x[t][5] = b.y; x[t][6] = b.z; x[t][7] = b.w;
         }
+        if (norm != nullptr) {
+            const float4 a = *reinterpret_cast<const float4 *>(norm + col0), b = *reinterpret_cast<const float4 *>(norm + col0 + 4);
+            nw[0] = a.x; nw[1] = a.y; nw[2] = a.z; nw[3] = a.w;
+            nw[4] = b.x; nw[5] = b.y; nw[6] = b.z; nw[7] = b.w;
+        }
     } else {
 #pragma unroll
         for (int rr = 0; rr < kRouteRows; ++rr) {
@@ -246,6 +266,9 @@ __global__ __launch_bounds__(256) void route_kernel(LayerDev L, const float *__r
 #pragma unroll
             for (int v = 0; v < 8; ++v)
                 x[t][v] = (t < (int)m && v < vpt) ? h[(size_t)t * H + col0 + v] : 0.0f;
+        if (norm != nullptr)
+#pragma unroll
+            for (int v = 0; v < 8; ++v) nw[v] = v < vpt ? norm[col0 + v] : 0.0f;
     }
 
     if (norm != nullptr) {
@@ -257,14 +280,11 @@ __global__ __launch_bounds__(256) void route_kernel(LayerDev L, const float *__r
             for (int v = 0; v < 8; ++v) ss[t] += x[t][v] * x[t][v];
         }
         block_sum_256<MT>(ss, lds_norm);
-        float wv[8];
-#pragma unroll
-        for (int v = 0; v < 8; ++v) wv[v] = v < vpt ? norm[col0 + v] : 0.0f;
 #pragma unroll
         for (int t = 0; t < MT; ++t) {
             const float inv = 1.0f / sqrtf(ss[t] / (float)H + 1e-6f);
 #pragma unroll
-            for (int v = 0; v < 8; ++v) x[t][v] = x[t][v] * inv * wv[v];
+            for (int v = 0; v < 8; ++v) x[t][v] = x[t][v] * inv * nw[v];
         }
     }
 
@@ -292,36 +312,28 @@ __global__ __launch_bounds__(256) void route_kernel(LayerDev L, const float *__r
                                        __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
     }
-    // 3. xprep (when asked for) of block kb is held by threads [kb * 32/vpt,
-    //    (kb+1) * 32/vpt) of workgroup kb + 1 (workgroup 0 routes); records
-    //    are strided by the gate/up matrices' padded block count bp.  The
-    //    kernels that read them start after this one ends.
+    // 3. xprep (when asked for) of block kb is written by workgroup kb + 1
+    //    (workgroup 0 routes), one half-wavefront per token: the threads that
+    //    hold the block's elements leave them in LDS.  (Made by those threads
+    //    themselves, eight elements each and token after token, the records of
+    //    eight tokens took longer than the routing.)  Records are strided by
+    //    the gate/up matrices' padded block count bp.  The kernels that read
+    //    them start after this one ends.
     const uint32_t KB = xprep ? H / 32 : 0;
     for (uint32_t kb = blockIdx.x - 1; blockIdx.x > 0 && kb < KB; kb += gridDim.x - 1) {
-        const int lpb = 32 / vpt;
-        const int first = (int)kb * lpb;
-        if (tid >= first && tid < first + lpb) {
-            for (int t = 0; t < (int)m; ++t) {
-                uint32_t *rec = xprep + (size_t)t * bp * kXprepDwords;
-                if (vpt == 8) {
-                    float v8[8];
+        const int lpb = 32 / vpt, at = tid - (int)kb * lpb;
+        __syncthreads();
+        if (front && at >= 0 && at < lpb) {
 #pragma unroll
-                    for (int v = 0; v < 8; ++v) v8[v] = x[t][v];
-                    prep_block<8>(v8, tid - first, rec, bp, kb);
-                } else if (vpt == 4) {
-                    float v4[4];
+            for (int t = 0; t < MT; ++t)
 #pragma unroll
-                    for (int v = 0; v < 4; ++v) v4[v] = x[t][v];
-                    prep_block<4>(v4, tid - first, rec, bp, kb);
-                } else if (vpt == 2) {
-                    float v2[2] = {x[t][0], x[t][1]};
-                    prep_block<2>(v2, tid - first, rec, bp, kb);
-                } else {
-                    float v1[1] = {x[t][0]};
-                    prep_block<1>(v1, tid - first, rec, bp, kb);
-                }
-            }
+                for (int v = 0; v < 8; ++v)
+                    if (v < vpt) s_blk[t][at * vpt + v] = x[t][v];
         }
+        __syncthreads();
+        const int t = tid >> 5, j = tid & 31;
+        prep_block32(s_blk[t < MT ? t : 0][j], j, t < (int)m, xprep + (size_t)(t < MT ? t : 0) * bp * kXprepDwords, bp, kb,
+                     PlainStore());
     }
 
     // 4. Q8_K records (when asked for): chunk j < m * H / 256 (chunk c = j %
@@ -340,7 +352,7 @@ __global__ __launch_bounds__(256) void route_kernel(LayerDev L, const float *__r
 #pragma unroll
                 for (int v = 0; v < 8; ++v) {
                     const uint32_t e = col0 + (uint32_t)v;
-                    if (v < vpt && e >= 256 * c && e < 256 * c + 256) s_chunk[e - 256 * c] = x[tt][v];
+                    if (front && v < vpt && e >= 256 * c && e < 256 * c + 256) s_chunk[e - 256 * c] = x[tt][v];
                 }
         __syncthreads();
         if (tid < kWave) {
@@ -361,7 +373,7 @@ __global__ __launch_bounds__(256) void route_kernel(LayerDev L, const float *__r
         s_last = 0;  // 1: the poll timed out
     }
     __syncthreads();
-    for (int t = wave; t < (int)m; t += 4) {
+    for (int t = wave; t < (int)m; t += kRouteThreads<MT> / kWave) {
         // this token's E + 1 words: lane l takes experts l + 64 i, lane 0 also
         // the gate word; until every word carries this launch's tag
         const uint64_t *lt = logits + (size_t)t * (E + 1);
@@ -524,7 +536,7 @@ hipError_t launch_route(hipStream_t s, const LayerDev &L, const float *h, const 
     const uint32_t bp = padded_blocks(L.hidden / 32);
     uint32_t *counter = sc.counters;
 #define TQF_ROUTE(MT)                                                                        \
-    hipLaunchKernelGGL(route_kernel<MT>, dim3(grid), dim3(256), 0, s, L, h, norm, m, bp,          \
+    hipLaunchKernelGGL(route_kernel<MT>, dim3(grid), dim3(kRouteThreads<MT>), 0, s, L, h, norm, m, bp,          \
                        records ? sc.xprep : nullptr,                                               \
                        sc.logits, sc.plan, counter, ids_out, w_out, status_out, q8, bp8)
     if (m <= 1) TQF_ROUTE(1);
