@@ -548,17 +548,19 @@ hipError_t launch_route(hipStream_t s, const LayerDev &L, const float *h, const 
 }
 
 // ---------------------------------------------------------------------------
-// Gate/up kernel.  Grid (width / (64 G) row groups, pair slots), eight
-// wavefronts per workgroup; G = 64 / LPR lane groups per wavefront, LPR =
+// Gate/up kernel.  Grid (width / (32 G) row groups, pair slots), four
+// wavefronts per workgroup (with eight, one token's 9 slots made 72 workgroups
+// for 256 CUs, and at 8 tokens one workgroup was resident per CU: 8.6 and 22.2
+// us, 6.7 and 16.7 with four); G = 64 / LPR lane groups per wavefront, LPR =
 // the gate/up matrices' padded block count (hidden / 32 <= 64).  Lane group
 // j of a wavefront owns 8 rows of both matrices: lane b loads block b of each
 // row (16 nibble loads), the scales of its block for the 8 rows (one 16-byte
 // load per matrix) and the activation record of block b of the slot's token,
 // then reduces the 16 block products across the group (value 2n + u: row n,
 // u = 0 gate, 1 up).  h = silu(gate) * up (weights.rs:241-259) meets in LDS
-// and the first G wavefronts write it as xprep records for the down kernel.
+// and a half-wavefront per block writes it as xprep records for the down kernel.
 // ---------------------------------------------------------------------------
-constexpr int kGateUpWaves = 8;
+constexpr int kGateUpWaves = 4;
 constexpr int kGateUpRows = 8;  // rows per lane group per matrix
 
 template <int LPR>
@@ -605,13 +607,12 @@ __global__ __launch_bounds__(kGateUpWaves * kWave) void gate_up_kernel(
             s_h[wave * RW + j * kGateUpRows + q / (2 * R)] = (gate / (1.0f + expf(-gate))) * up;
     }
     __syncthreads();
-    if (wave < G) {
-        const uint32_t blk = blockIdx.x * (2 * G) + 2 * wave + (uint32_t)(lane >> 5);
-        if (blk < L.width / 32) {
-            float hv[1] = {s_h[(2 * wave + (lane >> 5)) * 32 + (lane & 31)]};
-            prep_block<1>(hv, lane & 31, hprep + (size_t)slot * bp_down * kXprepDwords, bp_down,
-                          blk);
-        }
+    constexpr int kBlocks = kGateUpWaves * RW / 32;  // blocks of h per workgroup, one per half-wavefront
+    if (2 * wave < kBlocks) {
+        const int q = 2 * wave + (lane >> 5);
+        const uint32_t blk = blockIdx.x * kBlocks + (uint32_t)q;
+        prep_block32(s_h[(q < kBlocks ? q : 0) * 32 + (lane & 31)], lane & 31, q < kBlocks && blk < L.width / 32,
+                     hprep + (size_t)slot * bp_down * kXprepDwords, bp_down, blk, PlainStore());
     }
 }
 
@@ -635,18 +636,21 @@ hipError_t launch_gate_up(hipStream_t s, const LayerDev &L, uint32_t slots, cons
 }
 
 // ---------------------------------------------------------------------------
-// Down kernel.  Grid (hidden / (16 G) row groups, slot groups of four pair
-// slots), one wavefront per slot.  Lane group j owns 16 consecutive rows of
+// Down kernel.  Grid (hidden / (8 G) row groups, slot groups of four pair
+// slots), one wavefront per slot.  Lane group j owns 8 consecutive rows of
 // the slot's down matrix; lane b reads block b of each (LPR = the padded
 // block count of the width, <= 64) against block b of the slot's h records.
 // The workgroup weights each slot by its coefficient (shared: sigmoid gate;
 // routed: route weight; experts/mod.rs:1609-1630) and sums per token in slot
 // order; the last workgroup of a row group sums the slot groups in order and
-// adds the residual (runtime.rs:802) when given.  8 tokens: 15.0 us, 22.3 while
-// the last workgroup loaded the 18 slot groups one after another.
+// adds the residual (runtime.rs:802) when given.  While the last
+// workgroup loaded the slot groups (18 at 8 tokens) one after another, 8 tokens
+// took 22.3 us; loaded eight at a time, 15.0.
 // ---------------------------------------------------------------------------
 constexpr int kDownSlots = 4;
-constexpr int kDownRows = 16;  // rows per lane group
+// Rows per lane group: one octet.  With two, one token's 9 slots made 96
+// workgroups for 256 CUs (7.2 us, 6.1 with one; 8 tokens 15.0 and 14.1).
+constexpr int kDownRows = 8;
 
 template <int LPR>
 __global__ __launch_bounds__(kDownSlots * kWave) void down_kernel(
@@ -676,7 +680,7 @@ __global__ __launch_bounds__(kDownSlots * kWave) void down_kernel(
         uint4 nib[kDownRows];
 #pragma unroll
         for (int n = 0; n < kDownRows; ++n) nib[n] = q4_signed(load_nibbles(W, rl + n, b));
-        const uint4 s0 = load_scales(W, rl / 8, b), s1 = load_scales(W, rl / 8 + 1, b);
+        const uint4 sc = load_scales(W, rl / 8, b);
         uint32_t x[28];
         load_xrec(hprep + (size_t)slot * LPR * kXprepDwords, LPR, b, x);
         if (b >= L.width / 32) x[24] = 0;  // padding block: contributes exactly 0
@@ -684,7 +688,7 @@ __global__ __launch_bounds__(kDownSlots * kWave) void down_kernel(
         float a[kDownRows];
 #pragma unroll
         for (int n = 0; n < kDownRows; ++n)
-            a[n] = octet_scale(n < 8 ? s0 : s1, n % 8) * q4_block_dot(nib[n], x);
+            a[n] = octet_scale(sc, n) * q4_block_dot(nib[n], x);
         v = coef * transpose_reduce<LPR, kDownRows>(a);
     }
     if (reduced_first_copy<LPR, kDownRows>(lane))
