@@ -214,6 +214,33 @@ def test_moe_layer_parity(backend, layer, m):
     print(f"m={m} rel err {rel_err(y, yc):.3e} union {len(mtp.routes_union(ids))}")
 
 
+@pytest.mark.parametrize("F", [256, 1024, 2048])
+def test_moe_layer_kernels_over_widths_and_rows(backend, F):
+    """The layer kernels at the block counts of the down matrices (16, 32 and
+    64 per lane group), at row counts on both sides of the route kernel's
+    instantiations (4 | 5 rows: one routing wavefront per row from there on)
+    and at the most rows; with the norm through a one-layer stack."""
+    L = Layer(backend, 40 + F // 256, F=F)
+    norm = (1.0 + 0.1 * synth.normal((2048,), seed=970)).astype(np.float32)
+    st = backend.prepare_stack([L.dev], [backend.upload_f32(norm)])
+    try:
+        for m in (1, 4, 5, 8):
+            x = synth.normal((m, 2048), seed=980 + m)
+            y, ids, w = backend.moe_forward_batch(L.dev, x)
+            yc, idc, wc = L.host.forward_batch(x)
+            assert np.array_equal(ids, idc) and rel_err(w, wc) < 1e-5 and rel_err(y, yc) < FFN_TOL, (F, m)
+            with backend.variant(_lib.VARIANT_PERSISTENT, False):
+                dh = backend.to_device(x)
+                backend.stack_forward_device(st, dh, m)
+                h = backend.read(dh, np.float32, (m, 2048))
+                backend.free(dh)
+            hc, _ = oracle_stack([L], [norm], x)
+            assert rel_err(h, hc) < FFN_TOL, (F, m)
+    finally:
+        backend.free_stack(st)
+        backend.free_moe_layer(L.dev)
+
+
 def test_moe_layer_bf16_input(backend, layer):
     x = synth.normal((4, 2048), seed=7)
     xb = (x.view(np.uint32) >> 16).astype(np.uint16)

@@ -173,24 +173,20 @@ int32_t ensure_moe_scratch(tqf_hip_ctx *ctx, uint32_t hidden, uint32_t width, ui
     (void)hipFree(sc.hprep);
     (void)hipFree(sc.logits);
     (void)hipFree(sc.plan);
-    (void)hipFree(sc.partial);
     (void)hipFree(sc.counters);
     sc.xprep = sc.hprep = sc.counters = nullptr;
     sc.logits = nullptr;
-    sc.partial = nullptr;
     sc.plan = nullptr;
     sc.hidden = sc.width = sc.experts = 0;
     // padding records stay zero: kernels only write real blocks
     const size_t xprep = (size_t)kMaxTokens * padded_blocks(hidden / 32) * kXprepDwords * 4;
     const size_t hprep = (size_t)kMaxSlots * padded_blocks(width / 32) * kXprepDwords * 4;
     const size_t logits = (size_t)kMaxTokens * (experts + 1) * 8;
-    const size_t partial = (size_t)kMaxSlots * kMaxTokens * hidden * 4;
     const size_t counters = counter_count(hidden) * 4;
     TQF_HIP(ctx, hipMalloc(&sc.xprep, xprep));
     TQF_HIP(ctx, hipMalloc(&sc.hprep, hprep));
     TQF_HIP(ctx, hipMalloc(&sc.logits, logits));
     TQF_HIP(ctx, hipMalloc(&sc.plan, sizeof(Plan)));
-    TQF_HIP(ctx, hipMalloc(&sc.partial, partial));
     TQF_HIP(ctx, hipMalloc(&sc.counters, counters));
     TQF_HIP(ctx, hipMemset(sc.xprep, 0, xprep));
     TQF_HIP(ctx, hipMemset(sc.hprep, 0, hprep));
@@ -356,7 +352,7 @@ int32_t enqueue_layer(tqf_hip_ctx *ctx, const LayerDev &L, const float *h, const
     }
     {
         Prof p(ctx);
-        hipError_t e = launch_down(ctx->stream, L, m, m * (kTopK + 1), sc, sc.plan, sc.hprep, resid, out);
+        hipError_t e = launch_down(ctx->stream, L, m, kTopK + 1, sc.plan, sc.hprep, resid, out);
         if (e != hipSuccess) return hip_fail(ctx, "down kernel launch", e);
         p.end(TQF_HIP_KERNEL_DOWN, pairs * F * 4 + m * H * 4 * (resid ? 2 : 1),
               q4_bytes(L.hidden, L.width), sc.plan);
@@ -428,7 +424,7 @@ int32_t enqueue_layer_q4k(tqf_hip_ctx *ctx, const LayerDev &L, const float *h, c
     {
         Prof p(ctx);
         e = fold ? launch_q4k_q8k_slots(ctx->stream, sc.plan, S, true, dd, nullptr, b.dn, b.gu, out, resid,
-                                        sc.counters + counter_fold_offset(H))
+                                        sc.counters + kCounterFold)
                  : launch_q4k_q8k_slots(ctx->stream, sc.plan, S, true, dd, nullptr, b.dn, b.gu);
         if (e != hipSuccess) return hip_fail(ctx, "Q4_K down kernel launch", e);
         p.end(TQF_HIP_KERNEL_Q4K_MATVEC, S * ((double)F * H / 256 * kQ4KBlock + H * 4.0), 0, nullptr);
@@ -722,7 +718,6 @@ extern "C" int32_t tqf_hip_destroy(tqf_hip_ctx *ctx) {
     (void)hipFree(sc.hprep);
     (void)hipFree(sc.logits);
     (void)hipFree(sc.plan);
-    (void)hipFree(sc.partial);
     (void)hipFree(sc.counters);
     (void)hipFree(sc.accept);
     (void)hipFree(ctx->stack.sync);
@@ -1566,6 +1561,7 @@ extern "C" int32_t tqf_hip_expert_forward(tqf_hip_ctx *ctx, const tqf_hip_weight
     plan.m = (int32_t)m;
     for (uint32_t t = 0; t < m; ++t) {
         plan.slots[t] = SlotRec{{gate->tiles, up->tiles, down->tiles}, (int32_t)t, 1.0f};
+        plan.down[t][0] = DownRec{down->tiles, (int32_t)t, 1.0f};
         plan.slot_expert[t] = 0;
     }
     TQF_HIP(ctx, hipStreamSynchronize(ctx->stream));
@@ -1579,7 +1575,7 @@ extern "C" int32_t tqf_hip_expert_forward(tqf_hip_ctx *ctx, const tqf_hip_weight
     if (e == hipSuccess)
         e = launch_gate_up(ctx->stream, L, m, ctx->d_adhoc_plan, sc.xprep, sc.hprep);
     if (e == hipSuccess)
-        e = launch_down(ctx->stream, L, m, m, sc, ctx->d_adhoc_plan, sc.hprep, nullptr, dy);
+        e = launch_down(ctx->stream, L, m, 1, ctx->d_adhoc_plan, sc.hprep, nullptr, dy);
     if (e != hipSuccess) return hip_fail(ctx, "expert kernels", e);
     TQF_HIP(ctx, hipMemcpyAsync(y, dy, xb, hipMemcpyDeviceToHost, ctx->stream));
     TQF_HIP(ctx, hipStreamSynchronize(ctx->stream));

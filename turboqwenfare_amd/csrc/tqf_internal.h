@@ -194,6 +194,20 @@ __device__ __forceinline__ SlotRec load_slot(const SlotRec *p) {
     return __builtin_bit_cast(SlotRec, v);
 }
 
+// One of the nine down matvecs of a token, as the down kernels read it: the
+// matrix, the pair slot whose h it takes (< 0: no work), the coefficient.
+struct DownRec {
+    const uint8_t *mat;
+    int32_t slot;
+    float coef;
+};
+static_assert(sizeof(DownRec) == 16, "down record is one s_load_dwordx4");
+__device__ __forceinline__ DownRec load_down(const DownRec *p) {
+    typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+    const u32x4 v = *reinterpret_cast<const u32x4 *>(p);
+    return __builtin_bit_cast(DownRec, v);
+}
+
 struct Plan {
     int32_t n_slots;  // 9 * M when routing succeeded, 0 otherwise
     int32_t status;   // 0 or TQF_HIP_ERR_ROUTER
@@ -201,6 +215,7 @@ struct Plan {
     int32_t m;
     int32_t pad[4];
     SlotRec slots[kMaxSlots];
+    DownRec down[kMaxTokens][kTopK + 1];  // the shared expert, then the routes in order
     int32_t slot_expert[kMaxSlots];  // expert index; n_experts = shared
     uint16_t ids[kMaxTokens][kTopK];
     float weights[kMaxTokens][kTopK];
@@ -223,8 +238,7 @@ struct Scratch {
     uint32_t *hprep = nullptr;   // [kMaxSlots x padded(width/32) x 32]
     uint64_t *logits = nullptr;  // [kMaxTokens x (n_experts + 1)] tagged words (tag << 32 | f32 bits)
     Plan *plan = nullptr;
-    float *partial = nullptr;    // [slot groups x kMaxTokens x hidden]
-    uint32_t *counters = nullptr;  // last-arriver counters (see kCounter*)
+    uint32_t *counters = nullptr;  // see kCounterFold
     void *accept = nullptr;      // acceptance partials
     size_t accept_bytes = 0;
     uint32_t hidden = 0, width = 0, experts = 0;
@@ -418,17 +432,12 @@ struct tqf_hip_ctx {
 
 namespace tqf {
 
-// Counter array layout: [route launch count (slot 1) | pad | down (one per
-// row group, at most hidden / 16)].  The down counters return to zero in the
-// workgroup that finishes its kernel; the route kernel's launch count only
-// grows (it tags that launch's logit words).
-constexpr int kCounterDown = 64;
-// [0, 64) route; [64, 64 + hidden / 16) the Q4_0 down kernel; then the Q4_K
-// down launch's combine fold, kMaxTokens x (hidden / 64) (token, row tile)
-inline size_t counter_fold_offset(uint32_t hidden) { return kCounterDown + hidden / 16; }
-inline size_t counter_count(uint32_t hidden) {
-    return counter_fold_offset(hidden) + (size_t)kMaxTokens * (hidden / 64);
-}
+// Counter array layout: [route launch count (slot 1) | pad | the Q4_K down
+// launch's combine fold, kMaxTokens x (hidden / 32) (token, row tile)].  The
+// fold's counters return to zero in the workgroup that finishes its tile; the
+// route kernel's launch count only grows (it tags that launch's logit words).
+constexpr size_t kCounterFold = 64;
+inline size_t counter_count(uint32_t hidden) { return kCounterFold + (size_t)kMaxTokens * (hidden / 32); }
 
 // ---- launchers (defined in the .hip translation units) -------------------
 // All are asynchronous on ctx->stream and return a hipError_t.
@@ -457,8 +466,9 @@ hipError_t launch_route(hipStream_t s, const LayerDev &L, const float *h, const 
 // a slot whose record has token < 0 does no work.
 hipError_t launch_gate_up(hipStream_t s, const LayerDev &L, uint32_t slots, const Plan *plan,
                           const uint32_t *xprep, uint32_t *hprep);
-hipError_t launch_down(hipStream_t s, const LayerDev &L, uint32_t m, uint32_t slots, Scratch &sc,
-                       const Plan *plan, const uint32_t *hprep, const float *resid, float *out);
+// per_token: the down records each token has (9 for a MoE layer).
+hipError_t launch_down(hipStream_t s, const LayerDev &L, uint32_t m, uint32_t per_token, const Plan *plan,
+                       const uint32_t *hprep, const float *resid, float *out);
 size_t accept_scratch_bytes(uint32_t k, uint32_t vocab);
 void accept_warm();
 hipError_t launch_embed_rows(hipStream_t s, const uint8_t *tiles, const MatrixDims &d, const int32_t *tokens,

@@ -455,7 +455,10 @@ __global__ __launch_bounds__(kRouteThreads<MT>) void route_kernel(LayerDev L, co
     if (s_bad || s_last) {
         const int32_t err = s_last ? TQF_HIP_ERR_DEVICE : TQF_HIP_ERR_ROUTER;
         if (wave == 0)
-            for (int i = lane; i < (int)m * (kTopK + 1); i += kWave) plan->slots[i].token = -1;
+            for (int i = lane; i < (int)m * (kTopK + 1); i += kWave) {
+                plan->slots[i].token = -1;
+                plan->down[i / (kTopK + 1)][i % (kTopK + 1)].slot = -1;
+            }
         if (tid == 0) {
             plan->n_slots = 0;
             plan->n_union = 0;
@@ -498,6 +501,7 @@ __global__ __launch_bounds__(kRouteThreads<MT>) void route_kernel(LayerDev L, co
             rec.token = t;
             rec.coef = wv;
             plan->slots[slot] = rec;
+            plan->down[t][1 + k] = DownRec{rec.mat[2], slot, wv};
             plan->slot_expert[slot] = e_i;
             plan->pair_slot[lane] = slot;
             plan->ids[t][k] = (uint16_t)e_i;
@@ -516,6 +520,7 @@ __global__ __launch_bounds__(kRouteThreads<MT>) void route_kernel(LayerDev L, co
             rec.token = lane;
             rec.coef = 1.0f / (1.0f + expf(-gl));
             plan->slots[lane] = rec;
+            plan->down[lane][0] = DownRec{rec.mat[2], lane, rec.coef};
             plan->slot_expert[lane] = (int)E;
         }
         if (lane == 0) {
@@ -636,111 +641,63 @@ hipError_t launch_gate_up(hipStream_t s, const LayerDev &L, uint32_t slots, cons
 }
 
 // ---------------------------------------------------------------------------
-// Down kernel.  Grid (hidden / (8 G) row groups, slot groups of four pair
-// slots), one wavefront per slot.  Lane group j owns 8 consecutive rows of
-// the slot's down matrix; lane b reads block b of each (LPR = the padded
+// Down kernel.  Grid (hidden / (8 G) row groups, tokens), one wavefront per
+// down record of the token (nine in a layer).  Lane group j owns 8 consecutive
+// rows of the record's matrix; lane b reads block b of each (LPR = the padded
 // block count of the width, <= 64) against block b of the slot's h records.
-// The workgroup weights each slot by its coefficient (shared: sigmoid gate;
-// routed: route weight; experts/mod.rs:1609-1630) and sums per token in slot
-// order; the last workgroup of a row group sums the slot groups in order and
-// adds the residual (runtime.rs:802) when given.  While the last
-// workgroup loaded the slot groups (18 at 8 tokens) one after another, 8 tokens
-// took 22.3 us; loaded eight at a time, 15.0.
+// The workgroup weights each by its coefficient (shared: sigmoid gate; routed:
+// route weight) and adds them in the reference's order, shared expert first
+// (experts/mod.rs:1609-1630), then the residual (runtime.rs:802) when given.
+// Bound by its latencies (records, weights, records of h, dot, sum).  All of a
+// token's records in one workgroup need no hand-off between workgroups: with
+// four slots a workgroup, whose partials the last one of a row group added up,
+// it took 6.1 / 14.1 us at 1 / 8 tokens, now 5.5 / 10.6.
 // ---------------------------------------------------------------------------
-constexpr int kDownSlots = 4;
-// Rows per lane group: one octet.  With two, one token's 9 slots made 96
-// workgroups for 256 CUs (7.2 us, 6.1 with one; 8 tokens 15.0 and 14.1).
-constexpr int kDownRows = 8;
+constexpr int kDownRows = 8;  // rows per lane group
 
 template <int LPR>
-__global__ __launch_bounds__(kDownSlots * kWave) void down_kernel(
-    LayerDev L, const Plan *__restrict__ plan, const uint32_t *__restrict__ hprep,
-    uint32_t rows_padded, float *__restrict__ partial, uint32_t *__restrict__ counters,
-    const float *resid, float *out, uint32_t m, int n_slots) {
-    constexpr int G = kWave / LPR;
-    constexpr int RW = kDownRows * G;  // rows per workgroup
-    __shared__ float red[kDownSlots][RW];
-    __shared__ int s_tok[kDownSlots];
-    __shared__ int s_last;
-    const int n_sg = gridDim.y;  // every workgroup arrives, with or without work
-    const int sg = blockIdx.y;
+__global__ __launch_bounds__((kTopK + 1) * kWave) void down_kernel(LayerDev L, const Plan *__restrict__ plan,
+                                                                   const uint32_t *__restrict__ hprep,
+                                                                   const float *resid, float *out) {
+    constexpr int RW = kDownRows * (kWave / LPR);  // rows per workgroup
+    __shared__ float red[kTopK + 1][RW];
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
     const int lane = threadIdx.x % kWave;
     const uint32_t j = (uint32_t)lane / LPR, b = (uint32_t)lane % LPR;
-    const int slot = sg * kDownSlots + wave;
-    const uint32_t r0 = blockIdx.x * RW;
-    const uint32_t H = L.hidden;
-    float v = 0.0f;
-    const SlotRec rec = load_slot(&plan->slots[slot < n_slots ? slot : 0]);
-    const int tok = slot < n_slots ? rec.token : -1;
-    if (tok >= 0) {
-        const float coef = rec.coef;
-        const RowLane W = row_lane(rec.mat[2], LPR);
-        const uint32_t rl = r0 + j * kDownRows;
-        uint4 nib[kDownRows];
+    const uint32_t t = blockIdx.y, r0 = blockIdx.x * RW, H = L.hidden;
+    const DownRec rec = load_down(&plan->down[t][wave]);
+    if (rec.slot < 0) return;  // routing failed: every wavefront leaves
+    const uint32_t r = threadIdx.x;
+    const float res = resid && r < RW && r0 + r < H ? resid[(size_t)t * H + r0 + r] : 0.0f;
+    const RowLane W = row_lane(rec.mat, LPR);
+    const uint32_t rl = r0 + j * kDownRows;
+    uint4 nib[kDownRows];
 #pragma unroll
-        for (int n = 0; n < kDownRows; ++n) nib[n] = q4_signed(load_nibbles(W, rl + n, b));
-        const uint4 sc = load_scales(W, rl / 8, b);
-        uint32_t x[28];
-        load_xrec(hprep + (size_t)slot * LPR * kXprepDwords, LPR, b, x);
-        if (b >= L.width / 32) x[24] = 0;  // padding block: contributes exactly 0
-        __builtin_amdgcn_sched_barrier(0);  // every load in flight before any math
-        float a[kDownRows];
+    for (int n = 0; n < kDownRows; ++n) nib[n] = q4_signed(load_nibbles(W, rl + n, b));
+    const uint4 sc = load_scales(W, rl / 8, b);
+    uint32_t x[28];
+    load_xrec(hprep + (size_t)rec.slot * LPR * kXprepDwords, LPR, b, x);
+    if (b >= L.width / 32) x[24] = 0;  // padding block: contributes exactly 0
+    __builtin_amdgcn_sched_barrier(0);  // every load in flight before any math
+    float a[kDownRows];
 #pragma unroll
-        for (int n = 0; n < kDownRows; ++n)
-            a[n] = octet_scale(sc, n) * q4_block_dot(nib[n], x);
-        v = coef * transpose_reduce<LPR, kDownRows>(a);
-    }
-    if (reduced_first_copy<LPR, kDownRows>(lane))
-        red[wave][j * kDownRows + reduced_index<LPR, kDownRows>(lane)] = v;
-    if (lane == 0) s_tok[wave] = tok;
+    for (int n = 0; n < kDownRows; ++n) a[n] = octet_scale(sc, n) * q4_block_dot(nib[n], x);
+    const float v = rec.coef * transpose_reduce<LPR, kDownRows>(a);
+    if (reduced_first_copy<LPR, kDownRows>(lane)) red[wave][j * kDownRows + reduced_index<LPR, kDownRows>(lane)] = v;
     __syncthreads();
-    for (int i = threadIdx.x; i < (int)m * RW; i += kDownSlots * kWave) {
-        const int t = i / RW, r = i % RW;
-        float p = 0.0f;
-#pragma unroll
-        for (int w = 0; w < kDownSlots; ++w)
-            if (s_tok[w] == t) p += red[w][r];
-        if (r0 + r < H) store_coherent(&partial[((size_t)sg * kMaxTokens + t) * H + r0 + r], p);
+    if (r < RW && r0 + r < H) {
+        float sum = red[0][r];
+        for (uint32_t w = 1; w < blockDim.x / kWave; ++w) sum += red[w][r];
+        out[(size_t)t * H + r0 + r] = resid ? res + sum : sum;
     }
-    wait_own_stores();
-    __syncthreads();
-    if (threadIdx.x == 0)
-        s_last = (counter_arrive(&counters[blockIdx.x]) == (uint32_t)n_sg - 1) ? 1 : 0;
-    __syncthreads();
-    if (!s_last) return;
-    for (int i = threadIdx.x; i < (int)m * RW; i += kDownSlots * kWave) {
-        const int t = i / RW, r = i % RW;
-        if (r0 + r >= H) continue;
-        // eight loads in flight: one after another, a slot group's partial
-        // was a round trip, 18 of them with eight tokens
-        float sum = 0.0f;
-        for (int q0 = 0; q0 < n_sg; q0 += 8) {
-            float p[8];
-#pragma unroll
-            for (int q = 0; q < 8; ++q)
-                p[q] = q0 + q < n_sg ? load_coherent(&partial[((size_t)(q0 + q) * kMaxTokens + t) * H + r0 + r]) : 0.0f;
-#pragma unroll
-            for (int q = 0; q < 8; ++q)
-                if (q0 + q < n_sg) sum += p[q];
-        }
-        const size_t o = (size_t)t * H + r0 + r;
-        out[o] = resid ? resid[o] + sum : sum;
-    }
-    if (threadIdx.x == 0) counter_reset(&counters[blockIdx.x]);
 }
 
-hipError_t launch_down(hipStream_t s, const LayerDev &L, uint32_t m, uint32_t slots, Scratch &sc,
-                       const Plan *plan, const uint32_t *hprep, const float *resid, float *out) {
+hipError_t launch_down(hipStream_t s, const LayerDev &L, uint32_t m, uint32_t per_token, const Plan *plan,
+                       const uint32_t *hprep, const float *resid, float *out) {
     const MatrixDims dn = matrix_dims(L.hidden, L.width);
-    const uint32_t G = kWave / dn.lpr;
-    const uint32_t rows_per_group = kDownRows * G;
-    const uint32_t n_sg = (slots + kDownSlots - 1) / kDownSlots;
-    dim3 grid((dn.rows_padded + rows_per_group - 1) / rows_per_group, n_sg);
-    dim3 block(kDownSlots * kWave);
-#define TQF_DOWN(LPR)                                                                      \
-    hipLaunchKernelGGL(down_kernel<LPR>, grid, block, 0, s, L, plan, hprep, dn.rows_padded, \
-                       sc.partial, sc.counters + kCounterDown, resid, out, m, (int)slots)
+    const uint32_t rows = kDownRows * (kWave / dn.lpr);
+    const dim3 grid((dn.rows_padded + rows - 1) / rows, m), block(per_token * kWave);
+#define TQF_DOWN(LPR) hipLaunchKernelGGL(down_kernel<LPR>, grid, block, 0, s, L, plan, hprep, resid, out)
     if (dn.blocks_padded == 16) TQF_DOWN(16);
     else if (dn.blocks_padded == 32) TQF_DOWN(32);
     else if (dn.blocks_padded == 64) TQF_DOWN(64);
