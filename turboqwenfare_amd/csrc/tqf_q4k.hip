@@ -399,54 +399,52 @@ struct Fold {
     uint32_t *counters;     // [M x tiles], zero between launches
 };
 
+// The slot forms take workgroups of four wavefronts: with eight, one token's 9
+// slots made 144 gate/up and 72 down workgroups for 256 CUs.  Gate/up and down
+// 12.9 + 10.9 -> 12.2 + 10.5 us at 4 tokens, 6.8 + 8.7 -> 6.6 + 8.2 at 1, with
+// the down form's weights loaded ahead of its records and the fold's view of
+// the plan ahead of its stores.  (Two wavefronts a workgroup: 12.0 + 11.4 and
+// 7.2 + 8.3.  All nine down records of a token in one workgroup, with no
+// hand-off: 10.8 and 9.6 for the down form; its integer work then sits on 64
+// CUs at one token.)
+constexpr int kSlotWaves = 4;
+template <int SRC>
+constexpr int kQ8KWaves = SRC == kSrcTables ? kQ4KWaves : kSlotWaves;
+
 template <int LPR, int TG, int SRC>
-__global__ __launch_bounds__(kQ4KWaves * kWave) void q4k_q8k_gemv_kernel(
+__global__ __launch_bounds__(kQ8KWaves<SRC> * kWave) void q4k_q8k_gemv_kernel(
     const uint8_t *const *__restrict__ tables, const Plan *__restrict__ plan, MatrixDims d,
     const uint32_t *__restrict__ q8, uint32_t m, float *__restrict__ y, const float *__restrict__ gu,
     Fold fold) {
+    constexpr int NW = kQ8KWaves<SRC>;
+    constexpr bool kDownSwiglu = SRC == kSrcSlotDownSwiglu;
     constexpr int G = kWave / LPR;         // row octets per wavefront
     constexpr int SB = LPR / 8;            // super-blocks per lane group and chunk
     constexpr int NCH = (9 + SB - 1) / SB; // running sums per lane
-    __shared__ float lds[kQ4KWaves][kWave][9];
-    __shared__ uint4 s_rec[SRC == kSrcSlotDownSwiglu ? 3 * kMaxRecBp : 1];
+    __shared__ float lds[NW][kWave][9];
+    __shared__ uint4 s_rec[kDownSwiglu ? 3 * kMaxRecBp : 1];
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
     const int lane = threadIdx.x % kWave;
     const int jg = lane / LPR, b = lane % LPR, k = b & 7, g = b >> 3;
     const uint32_t mat = blockIdx.y;
-    if constexpr (SRC == kSrcSlotDownSwiglu) {
-        // before any wavefront can leave: every wavefront reaches the barrier
-        if (plan->slots[mat].token >= 0) {
-            const uint32_t cols = d.cols, S = gridDim.y;
-            const int kk = lane >> 3, cc = lane & 7;
-            for (uint32_t ch = (uint32_t)wave; ch < cols / 256; ch += kQ4KWaves) {
-                const size_t e0 = (size_t)mat * cols + (size_t)ch * 256 + 32 * kk + cc;
-                float v[4];
-#pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    const float gv = gu[e0 + 8 * i], uv = gu[(size_t)S * cols + e0 + 8 * i];
-                    v[i] = __fmul_rn(__fdiv_rn(gv, __fadd_rn(1.0f, expf(-gv))), uv);
-                }
-                q8k_quantize_values(v, reinterpret_cast<uint32_t *>(s_rec), d.blocks_padded, ch);
-            }
-        }
-        __syncthreads();
-    }
-    const uint32_t r0 = (blockIdx.x * kQ4KWaves + wave) * 8 * G;
-    if (r0 >= d.rows_padded) return;  // no workgroup barrier below
+    const uint32_t r0 = (blockIdx.x * NW + wave) * 8 * G;
     const uint8_t *base;
+    int token = 0;
     if constexpr (SRC == kSrcTables) {
         base = tables[mat];
     } else {
         const uint32_t S = SRC == kSrcSlotGateUp ? gridDim.y / 2 : gridDim.y;
         const uint32_t slot = mat % S;
         const SlotRec rec = load_slot(&plan->slots[slot]);
-        if (rec.token < 0) return;  // routing failed: no work
+        if (rec.token < 0) return;  // routing failed: no work for the whole workgroup
+        token = rec.token;
         // a select, not an index: a dynamic index would move the record to LDS
         base = SRC == kSrcSlotGateUp ? (mat < S ? rec.mat[0] : rec.mat[1]) : rec.mat[2];
-        if constexpr (SRC != kSrcSlotDownSwiglu)
+        if constexpr (!kDownSwiglu)
             q8 += (size_t)(SRC == kSrcSlotGateUp ? (uint32_t)rec.token : slot) * d.blocks_padded *
                   kQ8KRecDwords;
     }
+    const bool has_rows = r0 < d.rows_padded;
     const RowLane W = row_lane(base, d.blocks_padded);
     const uint32_t rl = r0 + jg * 8;
     const uint32_t nb = d.blocks >> 3;
@@ -456,6 +454,44 @@ __global__ __launch_bounds__(kQ4KWaves * kWave) void q4k_q8k_gemv_kernel(
     const uint8_t *dm_row = base + q4k_dm_offset(d, rl + k, 0);
     float(*my)[9] = lds[wave];
     const int gbase = jg * LPR;
+    uint4 nib[8], scm;
+    uint32_t dmw;
+    auto load_weights = [&](uint32_t blk) {
+#pragma unroll
+        for (int p = 0; p < 8; ++p) nib[p] = load_nibbles(W, rl + p, blk);  // row rl + (p ^ k)
+        scm = load_scales(W, rl / 8, blk);
+        dmw = *(const __attribute__((address_space(1))) uint32_t *)(dm_row + (size_t)(blk >> 3) * 32);
+    };
+    float coef = 0.0f, weight[kTopK];
+    int pair[kTopK];
+    if constexpr (kDownSwiglu) {
+        // the first chunk's weights are on their way while the records are
+        // made, and so is what the fold reads of the plan
+        if (has_rows) load_weights(b);
+        if (fold.out) {
+            coef = plan->slots[token].coef;
+#pragma unroll
+            for (int kk = 0; kk < kTopK; ++kk) {
+                pair[kk] = plan->pair_slot[token * kTopK + kk];
+                weight[kk] = plan->weights[token][kk];
+            }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        const uint32_t cols = d.cols, S = gridDim.y;
+        const int kk = lane >> 3, cc = lane & 7;
+        for (uint32_t ch = (uint32_t)wave; ch < cols / 256; ch += NW) {
+            const size_t e0 = (size_t)mat * cols + (size_t)ch * 256 + 32 * kk + cc;
+            float v[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const float gv = gu[e0 + 8 * i], uv = gu[(size_t)S * cols + e0 + 8 * i];
+                v[i] = __fmul_rn(__fdiv_rn(gv, __fadd_rn(1.0f, expf(-gv))), uv);
+            }
+            q8k_quantize_values(v, reinterpret_cast<uint32_t *>(s_rec), d.blocks_padded, ch);
+        }
+        __syncthreads();
+    }
+    if (!has_rows) return;  // no workgroup barrier below but the fold's, whose workgroups have rows throughout
     for (uint32_t t0 = 0; t0 < m; t0 += TG) {
         float acc[TG][NCH];
 #pragma unroll
@@ -464,15 +500,11 @@ __global__ __launch_bounds__(kQ4KWaves * kWave) void q4k_q8k_gemv_kernel(
             for (int q = 0; q < NCH; ++q) acc[t][q] = 0.0f;
         for (uint32_t c = 0; c < chunks; ++c) {
             const uint32_t blk = c * LPR + b;
-            uint4 nib[8];
-#pragma unroll
-            for (int p = 0; p < 8; ++p) nib[p] = load_nibbles(W, rl + p, blk);  // row rl + (p ^ k)
-            const uint4 scm = load_scales(W, rl / 8, blk);
-            const uint32_t dmw = *(const __attribute__((address_space(1))) uint32_t *)(dm_row + (size_t)(blk >> 3) * 32);
+            if (!kDownSwiglu || c > 0) load_weights(blk);
             uint4 xa[TG], xb[TG], xc[TG];
 #pragma unroll
             for (int t = 0; t < TG; ++t) {
-                if constexpr (SRC == kSrcSlotDownSwiglu) {
+                if constexpr (kDownSwiglu) {
                     xa[t] = s_rec[blk];
                     xb[t] = s_rec[bp + blk];
                     xc[t] = s_rec[2 * bp + blk];
@@ -555,17 +587,16 @@ __global__ __launch_bounds__(kQ4KWaves * kWave) void q4k_q8k_gemv_kernel(
                 for (int ch = 0; ch < 8; ++ch) total = __fadd_rn(total, my[gbase + 8 * (ch % SB) + k][ch / SB]);
                 const float minimum = my[gbase + 8 * (8 % SB) + k][8 / SB];
                 float *dst = &y[((size_t)mat * m + t0 + t) * d.rows + rl + k];
-                if (SRC == kSrcSlotDownSwiglu && fold.out) store_coherent(dst, __fadd_rn(minimum, total));
+                if (kDownSwiglu && fold.out) store_coherent(dst, __fadd_rn(minimum, total));
                 else *dst = __fadd_rn(minimum, total);
             }
             wave_sync();
         }
     }
-    if constexpr (SRC == kSrcSlotDownSwiglu) {
+    if constexpr (kDownSwiglu) {
         if (!fold.out) return;
         __shared__ int s_last;
         const uint32_t tile = blockIdx.x, tiles = gridDim.x;
-        const int token = plan->slots[mat].token;  // >= 0: slots without work left above
         wait_own_stores();
         __syncthreads();
         if (threadIdx.x == 0)
@@ -573,16 +604,16 @@ __global__ __launch_bounds__(kQ4KWaves * kWave) void q4k_q8k_gemv_kernel(
         __syncthreads();
         if (!s_last) return;
         const uint32_t H = d.rows, rows_per_tile = H / tiles;
-        const float coef = plan->slots[token].coef;
         for (uint32_t r = threadIdx.x; r < rows_per_tile; r += blockDim.x) {
             const uint32_t c = tile * rows_per_tile + r;
-            float o = __fmul_rn(load_coherent(&y[(size_t)token * H + c]), coef);
-#pragma unroll
-            for (int kk = 0; kk < kTopK; ++kk) {
-                const int slot = plan->pair_slot[token * kTopK + kk];
-                o = __fadd_rn(o, __fmul_rn(load_coherent(&y[(size_t)slot * H + c]), plan->weights[token][kk]));
-            }
             const size_t i = (size_t)token * H + c;
+            const float shared = load_coherent(&y[i]);
+            float v[kTopK];
+#pragma unroll
+            for (int kk = 0; kk < kTopK; ++kk) v[kk] = load_coherent(&y[(size_t)pair[kk] * H + c]);
+            float o = __fmul_rn(shared, coef);
+#pragma unroll
+            for (int kk = 0; kk < kTopK; ++kk) o = __fadd_rn(o, __fmul_rn(v[kk], weight[kk]));
             if (fold.resid) o = __fadd_rn(fold.resid[i], o);
             fold.out[i] = o;
         }
@@ -611,9 +642,9 @@ template <int LPR>
 hipError_t launch_q4k_q8k_slots_lpr(hipStream_t s, const Plan *plan, uint32_t n_slots, bool down,
                                     const MatrixDims &d, const uint32_t *q8, float *y, const float *gu,
                                     const Fold &fold) {
-    constexpr uint32_t rows_per_group = kQ4KWaves * 8 * (kWave / LPR);
+    constexpr uint32_t rows_per_group = kSlotWaves * 8 * (kWave / LPR);
     const dim3 grid((d.rows_padded + rows_per_group - 1) / rows_per_group, down ? n_slots : 2 * n_slots);
-    const dim3 block(kQ4KWaves * kWave);
+    const dim3 block(kSlotWaves * kWave);
     const uint8_t *const *none = nullptr;
     // the fold needs every wavefront of every workgroup to own rows
     if (fold.out && (!down || !gu || d.rows % rows_per_group || d.rows_padded != d.rows)) return hipErrorInvalidValue;
@@ -649,14 +680,14 @@ hipError_t launch_q4k_q8k_slots(hipStream_t s, const Plan *plan, uint32_t n_slot
 }
 
 uint32_t q4k_fold_tiles(const MatrixDims &d) {
-    const uint32_t rows_per_group = kQ4KWaves * 8 * (kWave / d.lpr);
+    const uint32_t rows_per_group = kSlotWaves * 8 * (kWave / d.lpr);
     return (d.rows_padded + rows_per_group - 1) / rows_per_group;
 }
 
 bool q4k_fold_ok(const MatrixDims &d) {
-    const uint32_t rows_per_group = kQ4KWaves * 8 * (kWave / d.lpr);
+    const uint32_t rows_per_group = kSlotWaves * 8 * (kWave / d.lpr);
     return d.rows % rows_per_group == 0 && d.rows_padded == d.rows && d.blocks_padded <= (uint32_t)kMaxRecBp &&
-           d.cols % 256 == 0 && q4k_fold_tiles(d) <= d.rows / 64;
+           d.cols % 256 == 0 && q4k_fold_tiles(d) <= d.rows / 32;
 }
 
 // ---------------------------------------------------------------------------
