@@ -241,6 +241,46 @@ def test_moe_layer_kernels_over_widths_and_rows(backend, F):
         backend.free_moe_layer(L.dev)
 
 
+@pytest.mark.parametrize("fmt", ["q4_0", "q4_k"])
+@pytest.mark.parametrize("m", [1, 4, 8])
+def test_moe_router_error_in_any_row(backend, layer, fmt, m):
+    """The gate/up kernels make the routes, each workgroup its own token's:
+    one row whose logits are not finite, whichever it is, fails the call for
+    every row, and neither y nor the routes of any row are written; the call
+    after it is served."""
+    if fmt == "q4_k":
+        from test_gpu_q4k_moe import Q4KLayer
+        L = Q4KLayer(backend, 5)
+    else:
+        L = layer
+    x = synth.normal((m, 2048), seed=71 + m)
+    want = backend.moe_forward_batch(L.dev, x)
+    dy, dids = backend.alloc(m * 2048 * 4), backend.alloc(m * 8 * 2)
+    dst = backend.to_device(np.zeros(1, np.int32))
+    for bad in range(m):
+        for value in (np.inf, np.nan):
+            xb = x.copy()
+            xb[bad, 100 + bad] = value
+            dx = backend.to_device(xb)
+            dy0, di0 = backend.to_device(np.full((m, 2048), 7.0, np.float32)), backend.to_device(np.full((m, 8), 999, np.uint16))
+            backend.moe_layer_device(L.dev, dx, m, dy0, di0, None, dst)
+            assert int(backend.read(dst, np.int32, (1,))[0]) == ERR_ROUTER, (bad, value)
+            assert np.all(backend.read(dy0, np.float32, (m, 2048)) == 7.0)
+            assert np.all(backend.read(di0, np.uint16, (m, 8)) == 999)
+            for b in (dx, dy0, di0, dst):
+                backend.free(b)
+            dst = backend.to_device(np.zeros(1, np.int32))
+    dx = backend.to_device(x)
+    backend.moe_layer_device(L.dev, dx, m, dy, dids, None, dst)
+    assert int(backend.read(dst, np.int32, (1,))[0]) == 0
+    assert np.array_equal(backend.read(dy, np.float32, (m, 2048)), want[0])
+    assert np.array_equal(backend.read(dids, np.uint16, (m, 8)), want[1])
+    for b in (dx, dy, dids, dst):
+        backend.free(b)
+    if fmt == "q4_k":
+        backend.free_moe_layer(L.dev)
+
+
 def test_moe_layer_bf16_input(backend, layer):
     x = synth.normal((4, 2048), seed=7)
     xb = (x.view(np.uint32) >> 16).astype(np.uint16)

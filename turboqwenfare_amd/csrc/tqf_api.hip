@@ -181,7 +181,7 @@ int32_t ensure_moe_scratch(tqf_hip_ctx *ctx, uint32_t hidden, uint32_t width, ui
     // padding records stay zero: kernels only write real blocks
     const size_t xprep = (size_t)kMaxTokens * padded_blocks(hidden / 32) * kXprepDwords * 4;
     const size_t hprep = (size_t)kMaxSlots * padded_blocks(width / 32) * kXprepDwords * 4;
-    const size_t logits = (size_t)kMaxTokens * (experts + 1) * 8;
+    const size_t logits = (size_t)kMaxTokens * (experts + 1) * 4;
     const size_t counters = counter_count(hidden) * 4;
     TQF_HIP(ctx, hipMalloc(&sc.xprep, xprep));
     TQF_HIP(ctx, hipMalloc(&sc.hprep, hprep));
@@ -192,7 +192,6 @@ int32_t ensure_moe_scratch(tqf_hip_ctx *ctx, uint32_t hidden, uint32_t width, ui
     TQF_HIP(ctx, hipMemset(sc.hprep, 0, hprep));
     TQF_HIP(ctx, hipMemset(sc.plan, 0, sizeof(Plan)));
     TQF_HIP(ctx, hipMemset(sc.counters, 0, counters));
-    TQF_HIP(ctx, hipMemset(sc.logits, 0, logits));  // zero carries no launch's tag
     sc.hidden = hidden;
     sc.width = width;
     sc.experts = experts;
@@ -299,7 +298,7 @@ struct Prof {
     }
     // per_slot_bytes > 0 is charged once per distinct expert of the launch
     // just made: (plan->n_union + 1) including the shared expert.
-    void end(int kind, double fixed_bytes, double per_slot_bytes, const Plan *plan) {
+    void end(int kind, double fixed_bytes, double per_slot_bytes, Plan *plan, uint32_t m = 0) {
         if (!start) return;
         hipEvent_t stop = take_event(ctx);
         if (!stop) return;
@@ -307,6 +306,7 @@ struct Prof {
         int ring = -1;
         if (per_slot_bytes > 0 && plan) {
             ring = ctx->prof_ring_next++;
+            (void)launch_count_union(ctx->stream, plan, m);
             (void)hipMemcpyAsync(&ctx->prof_ring[ring], &plan->n_union, sizeof(int32_t),
                                  hipMemcpyDeviceToHost, ctx->stream);
         }
@@ -338,24 +338,25 @@ int32_t enqueue_layer(tqf_hip_ctx *ctx, const LayerDev &L, const float *h, const
     const double pairs = (double)m * (kTopK + 1);
     {
         Prof p(ctx);
-        hipError_t e = launch_route(ctx->stream, L, h, norm, m, sc, ids, w, status);
+        hipError_t e = launch_route(ctx->stream, L, h, norm, m, sc.logits, sc.xprep);
         if (e != hipSuccess) return hip_fail(ctx, "route kernel launch", e);
         p.end(TQF_HIP_KERNEL_ROUTE, (L.n_experts + 1) * H * 4 + m * H * 4 + (norm ? H * 4 : 0), 0,
               nullptr);
     }
     {
         Prof p(ctx);
-        hipError_t e = launch_gate_up(ctx->stream, L, m * (kTopK + 1), sc.plan, sc.xprep, sc.hprep);
+        hipError_t e = launch_gate_up(ctx->stream, L, m * (kTopK + 1), sc.plan, sc.xprep, sc.hprep,
+                                      RouteArgs{L, sc.logits, m, ids, w, status});
         if (e != hipSuccess) return hip_fail(ctx, "gate/up kernel launch", e);
         p.end(TQF_HIP_KERNEL_GATE_UP, m * H * 4 + pairs * F * 4, 2 * q4_bytes(L.width, L.hidden),
-              sc.plan);
+              sc.plan, m);
     }
     {
         Prof p(ctx);
         hipError_t e = launch_down(ctx->stream, L, m, kTopK + 1, sc.plan, sc.hprep, resid, out);
         if (e != hipSuccess) return hip_fail(ctx, "down kernel launch", e);
         p.end(TQF_HIP_KERNEL_DOWN, pairs * F * 4 + m * H * 4 * (resid ? 2 : 1),
-              q4_bytes(L.hidden, L.width), sc.plan);
+              q4_bytes(L.hidden, L.width), sc.plan, m);
     }
     return TQF_HIP_OK;
 }
@@ -408,13 +409,13 @@ int32_t enqueue_layer_q4k(tqf_hip_ctx *ctx, const LayerDev &L, const float *h, c
     hipError_t e = hipSuccess;
     {
         Prof p(ctx);
-        e = launch_route(ctx->stream, L, h, norm, m, sc, ids, w, status, false, b.q8x, dgu.blocks_padded);
+        e = launch_route(ctx->stream, L, h, norm, m, sc.logits, nullptr, b.q8x, dgu.blocks_padded);
         if (e != hipSuccess) return hip_fail(ctx, "route kernel launch", e);
         p.end(TQF_HIP_KERNEL_ROUTE, (L.n_experts + 1) * (double)H * 4 + m * (double)H * 4, 0, nullptr);
     }
     {
         Prof p(ctx);
-        e = launch_q4k_q8k_slots(ctx->stream, sc.plan, S, false, dgu, b.q8x, b.gu);
+        e = launch_q4k_gate_up(ctx->stream, dgu, RouteArgs{L, sc.logits, m, ids, w, status}, b.q8x, sc.plan, b.gu);
         if (e != hipSuccess) return hip_fail(ctx, "Q4_K gate/up kernel launch", e);
         p.end(TQF_HIP_KERNEL_Q4K_MATVEC, 2.0 * S * ((double)F * H / 256 * kQ4KBlock + F * 4.0), 0, nullptr);
     }
@@ -423,9 +424,8 @@ int32_t enqueue_layer_q4k(tqf_hip_ctx *ctx, const LayerDev &L, const float *h, c
     const bool fold = ctx->variant[TQF_HIP_VARIANT_Q4K_FOLD] != 0 && q4k_fold_ok(dd);
     {
         Prof p(ctx);
-        e = fold ? launch_q4k_q8k_slots(ctx->stream, sc.plan, S, true, dd, nullptr, b.dn, b.gu, out, resid,
-                                        sc.counters + kCounterFold)
-                 : launch_q4k_q8k_slots(ctx->stream, sc.plan, S, true, dd, nullptr, b.dn, b.gu);
+        e = fold ? launch_q4k_down(ctx->stream, dd, m, sc.plan, b.gu, b.dn, out, resid, sc.counters)
+                 : launch_q4k_down(ctx->stream, dd, m, sc.plan, b.gu, b.dn);
         if (e != hipSuccess) return hip_fail(ctx, "Q4_K down kernel launch", e);
         p.end(TQF_HIP_KERNEL_Q4K_MATVEC, S * ((double)F * H / 256 * kQ4KBlock + H * 4.0), 0, nullptr);
     }
@@ -1556,14 +1556,7 @@ extern "C" int32_t tqf_hip_expert_forward(tqf_hip_ctx *ctx, const tqf_hip_weight
     const uint8_t *mats[3] = {gate->tiles, up->tiles, down->tiles};
     Plan plan;
     std::memset(&plan, 0, sizeof plan);
-    plan.n_slots = (int32_t)m;
-    plan.n_union = 0;
-    plan.m = (int32_t)m;
-    for (uint32_t t = 0; t < m; ++t) {
-        plan.slots[t] = SlotRec{{gate->tiles, up->tiles, down->tiles}, (int32_t)t, 1.0f};
-        plan.down[t][0] = DownRec{down->tiles, (int32_t)t, 1.0f};
-        plan.slot_expert[t] = 0;
-    }
+    for (uint32_t t = 0; t < m; ++t) plan.down[t][0] = DownRec{down->tiles, (int32_t)t, 1.0f};
     TQF_HIP(ctx, hipStreamSynchronize(ctx->stream));
     drop_graphs(ctx);
     TQF_HIP(ctx, hipMemcpy(ctx->d_adhoc_mats, mats, sizeof mats, hipMemcpyHostToDevice));

@@ -100,7 +100,7 @@ __device__ __forceinline__ float wave_max4(const float (&v)[4]) {
 // four keys, then 8 rounds take the largest lane head.  Every lane of the
 // wavefront must be active; psel / idsel are uniform.
 __device__ __forceinline__ void top8_by_probability(const float (&p)[4], int lane, uint32_t E, float (&psel)[8],
-                                                    int (&idsel)[8]) {
+                                                    int (&idsel)[8], int rounds = 8) {
     uint32_t q[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i)
@@ -117,6 +117,7 @@ __device__ __forceinline__ void top8_by_probability(const float (&p)[4], int lan
     order(1, 2);
 #pragma unroll
     for (int k = 0; k < 8; ++k) {
+        if (k >= rounds) break;
         const uint32_t best = wave_umax(q[0]);
         const int l_win = (int)__builtin_ctzll(__ballot(q[0] == best));
         psel[k] = __uint_as_float((best >> 2) - 1u);

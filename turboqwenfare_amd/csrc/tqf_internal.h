@@ -171,31 +171,14 @@ inline size_t q6k_layout_bytes(const MatrixDims &d) {
     return q6k_d_base(d) + (size_t)(d.rows_padded >> 3) * (d.blocks_padded >> 3) * 16;
 }
 
-// Route plan written by the route kernel and read by the expert kernels.
-// Work is planned per (expert, token) pair so that every workgroup carries
-// the same arithmetic: slots [0, M) are the shared expert for tokens 0..M-1
-// (coefficient sigmoid(shared gate logit), experts/mod.rs:1614-1615); then,
-// for each distinct routed expert in first-demand order (the union of
-// experts/mod.rs:268-275 BatchExpertPlan), one slot per token routed to it
-// (coefficient = that token's route weight).  Slots of one expert are
-// adjacent, so its second reads come from L2 / Infinity Cache.
-// One pair slot as the expert kernels read it: a single 32-byte scalar load.
-struct SlotRec {
-    const uint8_t *mat[3];  // gate, up, down matrices of the slot's expert
-    int32_t token;          // < 0: no work (routing failed)
-    float coef;
-};
-static_assert(sizeof(SlotRec) == 32, "slot record is one s_load_dwordx8");
-
-// Reads a slot record with one 32-byte load, ahead of any use of its fields.
-__device__ __forceinline__ SlotRec load_slot(const SlotRec *p) {
-    typedef uint32_t u32x8 __attribute__((ext_vector_type(8)));
-    const u32x8 v = *reinterpret_cast<const u32x8 *>(p);
-    return __builtin_bit_cast(SlotRec, v);
-}
-
+// Work is planned per (token, expert) pair so that every workgroup carries
+// the same arithmetic: slot 9 t is the shared expert for token t (coefficient
+// sigmoid(shared gate logit), experts/mod.rs:1614-1615), slot 9 t + 1 + k its
+// route's expert k (coefficient = the route weight).  Tokens that share an
+// expert read its matrices in workgroups of one XCD (a row group's index is
+// the workgroup index modulo the row groups), so the second read is from L2.
 // One of the nine down matvecs of a token, as the down kernels read it: the
-// matrix, the pair slot whose h it takes (< 0: no work), the coefficient.
+// matrix, the slot whose h it takes (< 0: no work), the coefficient.
 struct DownRec {
     const uint8_t *mat;
     int32_t slot;
@@ -209,19 +192,8 @@ __device__ __forceinline__ DownRec load_down(const DownRec *p) {
 }
 
 struct Plan {
-    int32_t n_slots;  // 9 * M when routing succeeded, 0 otherwise
-    int32_t status;   // 0 or TQF_HIP_ERR_ROUTER
-    int32_t n_union;  // distinct routed experts (HBM bytes = (n_union + 1) experts)
-    int32_t m;
-    int32_t pad[4];
-    SlotRec slots[kMaxSlots];
     DownRec down[kMaxTokens][kTopK + 1];  // the shared expert, then the routes in order
-    int32_t slot_expert[kMaxSlots];  // expert index; n_experts = shared
-    uint16_t ids[kMaxTokens][kTopK];
-    float weights[kMaxTokens][kTopK];
-    float gate_logit[kMaxTokens];
-    int32_t union_ids[kMaxTokens * kTopK];
-    int32_t pair_slot[kMaxTokens * kTopK];  // slot of route (t, k) at index t * kTopK + k
+    int32_t n_union;                      // distinct routed experts (count_union; profiling only)
 };
 
 // Device-side description of one MoE layer (passed by value to kernels).
@@ -232,13 +204,26 @@ struct LayerDev {
     uint32_t n_experts, hidden, width;
 };
 
+// What a gate/up kernel needs to make the routes (tqf_route.h), and where it
+// records them.  m == 0: no routing.
+// status is set to TQF_HIP_ERR_ROUTER when a logit is not finite and left
+// untouched otherwise (a sticky flag the caller zeroes).
+struct RouteArgs {
+    LayerDev L{};
+    const float *logits = nullptr;  // [m x (n_experts + 1)]: the router's, then the gate's
+    uint32_t m = 0;
+    uint16_t *ids = nullptr;        // optional outputs
+    float *w = nullptr;
+    int32_t *status = nullptr;
+};
+
 // Per-context device scratch (allocated once, grown on demand).
 struct Scratch {
     uint32_t *xprep = nullptr;   // [kMaxTokens x padded(hidden/32) x 32]
     uint32_t *hprep = nullptr;   // [kMaxSlots x padded(width/32) x 32]
-    uint64_t *logits = nullptr;  // [kMaxTokens x (n_experts + 1)] tagged words (tag << 32 | f32 bits)
+    float *logits = nullptr;     // [kMaxTokens x (n_experts + 1)]
     Plan *plan = nullptr;
-    uint32_t *counters = nullptr;  // see kCounterFold
+    uint32_t *counters = nullptr;  // see counter_count
     void *accept = nullptr;      // acceptance partials
     size_t accept_bytes = 0;
     uint32_t hidden = 0, width = 0, experts = 0;
@@ -432,12 +417,9 @@ struct tqf_hip_ctx {
 
 namespace tqf {
 
-// Counter array layout: [route launch count (slot 1) | pad | the Q4_K down
-// launch's combine fold, kMaxTokens x (hidden / 32) (token, row tile)].  The
-// fold's counters return to zero in the workgroup that finishes its tile; the
-// route kernel's launch count only grows (it tags that launch's logit words).
-constexpr size_t kCounterFold = 64;
-inline size_t counter_count(uint32_t hidden) { return kCounterFold + (size_t)kMaxTokens * (hidden / 32); }
+// The Q4_K down launch's combine fold: one counter per (token, row tile); each
+// returns to zero in the workgroup that finishes its tile.
+inline size_t counter_count(uint32_t hidden) { return (size_t)kMaxTokens * (hidden / 32); }
 
 // ---- launchers (defined in the .hip translation units) -------------------
 // All are asynchronous on ctx->stream and return a hipError_t.
@@ -449,23 +431,22 @@ hipError_t launch_prep(hipStream_t s, const float *x, uint32_t m, uint32_t cols,
                        uint32_t blocks_padded, uint32_t *xprep);
 hipError_t launch_gemv(hipStream_t s, const uint8_t *const *d_tiles, uint32_t count,
                        const MatrixDims &d, const uint32_t *xprep, uint32_t m, float *y);
-// status_out (may be null) is set to TQF_HIP_ERR_ROUTER when routing fails and
-// left untouched otherwise (a sticky flag the caller zeroes).
-// records = false skips the Q4_0 activation records (xprep), which only the
-// Q4_0 gate/up kernel reads; q8 (with its record stride bp8 = the gate/up
-// matrices' padded block count) asks for the Q8_K records of the (normed)
-// rows as well, which the Q4_K gate/up reads.
-hipError_t launch_route(hipStream_t s, const LayerDev &L, const float *h, const float *norm,
-                        uint32_t m, Scratch &sc, uint16_t *ids_out, float *w_out,
-                        int32_t *status_out, bool records = true, uint32_t *q8 = nullptr,
-                        uint32_t bp8 = 0);
+// The router's and the shared gate's logits of the (normed) rows; xprep (may
+// be null) asks for the Q4_0 activation records, which the Q4_0 gate/up kernel
+// reads, q8 (with its record stride bp8 = the gate/up matrices' padded block
+// count) for the Q8_K records, which the Q4_K gate/up reads.
+hipError_t launch_route(hipStream_t s, const LayerDev &L, const float *h, const float *norm, uint32_t m,
+                        float *logits, uint32_t *xprep, uint32_t *q8 = nullptr, uint32_t bp8 = 0);
+// The distinct routed experts of the plan's m tokens, into plan->n_union.
+hipError_t launch_count_union(hipStream_t s, Plan *plan, uint32_t m);
 // gate/up needs the gate/up matrices' padded block count (hidden / 32) and the
 // down matrix's (width / 32) in {16, 32, 64}; other shapes return
 // hipErrorInvalidValue (callers validate first).
-// `slots` is the number of pair slots the grid covers (9 M for a MoE layer);
-// a slot whose record has token < 0 does no work.
-hipError_t launch_gate_up(hipStream_t s, const LayerDev &L, uint32_t slots, const Plan *plan,
-                          const uint32_t *xprep, uint32_t *hprep);
+// Nine matvecs per token, which make their routes from rt.logits and record
+// them in the plan; with rt.m == 0, matvec s < slots is L.mats[0] and [1] on
+// token s.
+hipError_t launch_gate_up(hipStream_t s, const LayerDev &L, uint32_t slots, Plan *plan,
+                          const uint32_t *xprep, uint32_t *hprep, const RouteArgs &rt = RouteArgs{});
 // per_token: the down records each token has (9 for a MoE layer).
 hipError_t launch_down(hipStream_t s, const LayerDev &L, uint32_t m, uint32_t per_token, const Plan *plan,
                        const uint32_t *hprep, const float *resid, float *out);
@@ -518,19 +499,18 @@ hipError_t launch_q4k_q8k_gemv(hipStream_t s, const uint8_t *const *tables, uint
 // rows] ([2 x m x cols]).
 hipError_t launch_q8k_swiglu_quantize(hipStream_t s, const float *gu, uint32_t m, uint32_t cols,
                                       uint32_t bp, uint32_t *q8);
-// The Q4_K MoE layer over a route plan (n_slots = 9 M slots of launch_route):
-// gate and up of every slot (y [2 x n_slots x rows]: gate rows, then up rows;
-// the records of the slot's token, q8 [M x 12 Bp]), or down of every slot
-// (records of the slot's own h, q8 [n_slots x 12 Bp]; y [n_slots x rows]).
-// Down with gu (the gate/up output, [2 x n_slots x cols]) makes each slot's
-// records of h = silu_mul(gate, up) in the workgroup instead (q8 unused).
-// With out (and counters [M x q4k_fold_tiles(d)], zero between launches),
+// The Q4_K MoE layer's matvecs, S = 9 m of them (token t's at 9 t: the shared
+// expert, then its route).  Gate and up (y [2 x S x rows]: gate rows, then up
+// rows; q8 [m x 12 Bp], the tokens' records) make the routes and record them
+// in the plan.  Down (y [S x rows]) makes the records of h = silu_mul(gate,
+// up) from gu, the gate/up output, in each workgroup.
+// With out (and counters [m x q4k_fold_tiles(d)], zero between launches),
 // the down form also folds in launch_q4k_moe_combine's work (+ resid), so
 // out receives the layer output without a combine launch.
-hipError_t launch_q4k_q8k_slots(hipStream_t s, const Plan *plan, uint32_t n_slots, bool down,
-                                const MatrixDims &d, const uint32_t *q8, float *y,
-                                const float *gu = nullptr, float *out = nullptr,
-                                const float *resid = nullptr, uint32_t *counters = nullptr);
+hipError_t launch_q4k_gate_up(hipStream_t s, const MatrixDims &d, const RouteArgs &rt, const uint32_t *q8, Plan *plan,
+                              float *y);
+hipError_t launch_q4k_down(hipStream_t s, const MatrixDims &d, uint32_t m, Plan *plan, const float *gu, float *y,
+                           float *out = nullptr, const float *resid = nullptr, uint32_t *counters = nullptr);
 uint32_t q4k_fold_tiles(const MatrixDims &d);
 bool q4k_fold_ok(const MatrixDims &d);  // the down matrix's shape allows the fold
 // y[t] = resid[t] (if given) + (shared slot t's down x its coefficient, then

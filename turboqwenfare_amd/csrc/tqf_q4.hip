@@ -11,6 +11,7 @@
 
 #include "tqf_device.h"
 #include "tqf_internal.h"
+#include "tqf_route.h"
 
 namespace tqf {
 
@@ -153,71 +154,31 @@ hipError_t launch_gemv(hipStream_t s, const uint8_t *const *d_tables, uint32_t c
 }
 
 // ---------------------------------------------------------------------------
-// Cross-workgroup hand-off without whole-L2 write-back/invalidate fences.
-// Values that another workgroup will read are stored with agent-scope
-// atomic stores (coherent at device scope, i.e. not left dirty in one XCD's
-// L2), each thread waits for its stores to complete, and only then is the
-// device-scope counter incremented; the workgroup that sees the final count
-// reads the values back with agent-scope atomic loads (store_coherent,
-// load_coherent, wait_own_stores, counter_arrive in tqf_device.h).
-// ---------------------------------------------------------------------------
-
-// ---------------------------------------------------------------------------
 // Route kernel.  One workgroup per two router rows (row n_experts is the
 // shared-expert input gate, experts/mod.rs:1614).  Each workgroup
 //   1. loads h [m x hidden], applies RMSNorm when `norm` is given
 //      (weights.rs:216-239: x * (1/sqrt(mean(x^2) + 1e-6)) * w),
-//   2. computes its router logits (experts/mod.rs:1491 router matvec) and
-//      stores them as tagged words (tag << 32 | f32 bits; the tag is the
-//      launch count with the high bit set, so a word of an earlier launch,
-//      or the zeroed allocation, never matches),
-//   3. writes the xprep / Q8_K records of the blocks assigned to it
-//      (workgroups 1..).
-// Workgroup 0 polls every logit word of this launch, turns the logits into
-// routes (RouterResult::from_logits, experts/mod.rs:134-167: softmax, stable
-// descending top-8 with ties to the lower id, renormalise) and the pair
-// plan, and advances the launch count.  The poll is bounded in time; a
-// timeout writes a failed plan (TQF_HIP_ERR_DEVICE).
-// Bound by the chain of its latencies (loads, two block sums, the words' round
-// trip, softmax and top-8), not by its 2.1 MB: 7.7 / 10.4 us with the norm at 1
-// / 4 tokens (9.0 / 11.8 while the norm's weights were loaded behind the sum of
-// squares), 14.0 us at 8 (23.2 with 256 threads, which spilled 272 bytes a
-// thread building the records).
+//   2. computes its router logits (experts/mod.rs:1491 router matvec),
+//   3. writes the xprep / Q8_K records of the blocks assigned to it.
+// The routes themselves are made from the logits by the gate/up kernels
+// (tqf_route.h).  Bound by its latencies (loads, two block sums), not by its
+// 2.1 MB: 3.9 / 6.0 / 7.8 us with the norm at 1 / 4 / 8 tokens (with the routing
+// behind a poll of every workgroup's logits 7.7 / 10.4 / 14.0).
 // ---------------------------------------------------------------------------
 constexpr int kRouteRows = 2;
-constexpr int64_t kRouteSpinLimit = 2000000;  // wall-clock ticks (100 MHz): 20 ms
-constexpr int kRouteSeq = 1;                   // the launch count's counter slot
-
-// The first 256 threads hold the rows' elements.  For more than four tokens
-// there are 512: one wavefront per token in workgroup 0's routing, where four
-// took two each.
-template <int MT>
-constexpr int kRouteThreads = MT <= 4 ? 256 : 512;
+constexpr int kRouteThreads = 256;
 
 template <int MT>
-__global__ __launch_bounds__(kRouteThreads<MT>) void route_kernel(LayerDev L, const float *__restrict__ h,
-                                                    const float *__restrict__ norm, uint32_t m,
-                                                    uint32_t bp, uint32_t *__restrict__ xprep,
-                                                    uint64_t *__restrict__ logits,
-                                                    Plan *__restrict__ plan,
-                                                    uint32_t *__restrict__ counter,
-                                                    uint16_t *__restrict__ ids_out,
-                                                    float *__restrict__ w_out,
-                                                    int32_t *__restrict__ status_out,
-                                                    uint32_t *__restrict__ q8, uint32_t bp8) {
+__global__ __launch_bounds__(kRouteThreads) void route_kernel(LayerDev L, const float *__restrict__ h,
+                                                              const float *__restrict__ norm, uint32_t m,
+                                                              uint32_t bp, uint32_t *__restrict__ xprep,
+                                                              float *__restrict__ logits,
+                                                              uint32_t *__restrict__ q8, uint32_t bp8) {
     __shared__ float lds_red[4][MT * kRouteRows];
     __shared__ float lds_norm[4][MT];
-    __shared__ int s_last;
-    __shared__ int s_bad;
-    __shared__ int s_ids[kMaxTokens * kTopK];
-    __shared__ float s_w[kMaxTokens * kTopK];
-    __shared__ float s_gate[kMaxTokens];
     __shared__ float s_blk[MT][32];
 
     const int tid = threadIdx.x;
-    const bool front = kRouteThreads<MT> == 256 || tid < 256;
-    const uint32_t seq = __hip_atomic_load(&counter[kRouteSeq], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    const uint32_t tag = 0x80000000u | (seq & 0x7FFFFFFFu);
     const uint32_t H = L.hidden, E = L.n_experts;
     const int vpt = (int)(H / 256);  // 1..8 elements per thread
     const uint32_t col0 = (uint32_t)tid * vpt;
@@ -229,8 +190,7 @@ __global__ __launch_bounds__(kRouteThreads<MT>) void route_kernel(LayerDev L, co
     float wv[kRouteRows][8] = {};
     float x[MT][8] = {};
     float nw[8] = {};  // the norm's weights: loaded here, not behind the sum of squares
-    if (!front) {
-    } else if (vpt == 8) {
+    if (vpt == 8) {
 #pragma unroll
         for (int rr = 0; rr < kRouteRows; ++rr) {
             const uint32_t r = blockIdx.x * kRouteRows + rr;
@@ -306,24 +266,20 @@ __global__ __launch_bounds__(kRouteThreads<MT>) void route_kernel(LayerDev L, co
         for (int rr = 0; rr < kRouteRows; ++rr) {
             const uint32_t r = blockIdx.x * kRouteRows + rr;
             if (r <= E)
-                for (int t = 0; t < (int)m; ++t)
-                    __hip_atomic_store(&logits[(size_t)t * (E + 1) + r],
-                                       ((uint64_t)tag << 32) | __float_as_uint(dots[rr * MT + t]),
-                                       __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                for (int t = 0; t < (int)m; ++t) logits[(size_t)t * (E + 1) + r] = dots[rr * MT + t];
         }
     }
-    // 3. xprep (when asked for) of block kb is written by workgroup kb + 1
-    //    (workgroup 0 routes), one half-wavefront per token: the threads that
-    //    hold the block's elements leave them in LDS.  (Made by those threads
-    //    themselves, eight elements each and token after token, the records of
-    //    eight tokens took longer than the routing.)  Records are strided by
-    //    the gate/up matrices' padded block count bp.  The kernels that read
-    //    them start after this one ends.
+    // 3. xprep (when asked for) of block kb is written by workgroup kb, one
+    //    half-wavefront per token: the threads that hold the block's elements
+    //    leave them in LDS.  (Made by those threads themselves, eight elements
+    //    each and token after token, the records of eight tokens took longer
+    //    than the rest.)  Records are strided by the gate/up matrices' padded
+    //    block count bp.
     const uint32_t KB = xprep ? H / 32 : 0;
-    for (uint32_t kb = blockIdx.x - 1; blockIdx.x > 0 && kb < KB; kb += gridDim.x - 1) {
+    for (uint32_t kb = blockIdx.x; kb < KB; kb += gridDim.x) {
         const int lpb = 32 / vpt, at = tid - (int)kb * lpb;
         __syncthreads();
-        if (front && at >= 0 && at < lpb) {
+        if (at >= 0 && at < lpb) {
 #pragma unroll
             for (int t = 0; t < MT; ++t)
 #pragma unroll
@@ -337,12 +293,10 @@ __global__ __launch_bounds__(kRouteThreads<MT>) void route_kernel(LayerDev L, co
     }
 
     // 4. Q8_K records (when asked for): chunk j < m * H / 256 (chunk c = j %
-    //    (H / 256) of row t = j / (H / 256)) by workgroup (j + 1) % grid, so
-    //    that workgroup 0, which routes, has one only when the grid has no
-    //    other workgroup left for it; staged in LDS in the quantizer's lane
-    //    order.
+    //    (H / 256) of row t = j / (H / 256)) by workgroup j; staged in LDS in
+    //    the quantizer's lane order.
     const uint32_t cpr = H / 256;
-    const uint32_t jq = blockIdx.x == 0 ? gridDim.x - 1 : blockIdx.x - 1;
+    const uint32_t jq = blockIdx.x;
     if (q8 != nullptr && jq < m * cpr) {
         __shared__ float s_chunk[256];
         const uint32_t t = jq / cpr, c = jq % cpr;
@@ -352,7 +306,7 @@ __global__ __launch_bounds__(kRouteThreads<MT>) void route_kernel(LayerDev L, co
 #pragma unroll
                 for (int v = 0; v < 8; ++v) {
                     const uint32_t e = col0 + (uint32_t)v;
-                    if (front && v < vpt && e >= 256 * c && e < 256 * c + 256) s_chunk[e - 256 * c] = x[tt][v];
+                    if (v < vpt && e >= 256 * c && e < 256 * c + 256) s_chunk[e - 256 * c] = x[tt][v];
                 }
         __syncthreads();
         if (tid < kWave) {
@@ -363,187 +317,16 @@ __global__ __launch_bounds__(kRouteThreads<MT>) void route_kernel(LayerDev L, co
             q8k_quantize_values(v4, q8 + (size_t)t * bp8 * kQ8KRecDwords, bp8, c);
         }
     }
-
-    if (blockIdx.x != 0) return;
-
-    // ---- workgroup 0: routes and the pair plan ------------------------------
-    const int wave = tid / kWave, lane = tid % kWave;
-    if (tid == 0) {
-        s_bad = 0;
-        s_last = 0;  // 1: the poll timed out
-    }
-    __syncthreads();
-    for (int t = wave; t < (int)m; t += kRouteThreads<MT> / kWave) {
-        // this token's E + 1 words: lane l takes experts l + 64 i, lane 0 also
-        // the gate word; until every word carries this launch's tag
-        const uint64_t *lt = logits + (size_t)t * (E + 1);
-        uint64_t w[5];
-        uint32_t need = 0;
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-            if ((uint32_t)lane + 64u * i < E) need |= 1u << i;
-        if (lane == 0) need |= 1u << 4;
-        int64_t t0 = 0;
-        for (uint32_t spin = 1;; ++spin) {
-#pragma unroll
-            for (int i = 0; i < 5; ++i) {
-                if ((need >> i) & 1u) {
-                    const uint32_t e = i < 4 ? (uint32_t)lane + 64u * i : E;
-                    w[i] = __hip_atomic_load(const_cast<uint64_t *>(lt + e), __ATOMIC_RELAXED,
-                                             __HIP_MEMORY_SCOPE_AGENT);
-                    if ((uint32_t)(w[i] >> 32) == tag) need &= ~(1u << i);
-                }
-            }
-            if (__all(need == 0)) break;
-            if ((spin & 63) == 0) {
-                const int64_t now = wall_clock64();
-                if (t0 == 0) {
-                    t0 = now;
-                } else if (now - t0 > kRouteSpinLimit) {
-                    if (lane == 0) s_last = 1;
-                    break;
-                }
-            }
-            __builtin_amdgcn_s_sleep(1);
-        }
-        if (s_last) continue;
-        float lv[4];
-        bool fin = true;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const uint32_t e = (uint32_t)lane + 64u * i;
-            lv[i] = e < E ? __uint_as_float((uint32_t)w[i]) : -INFINITY;
-            if (e < E && !(fabsf(lv[i]) <= 3.402823466e38f)) fin = false;
-        }
-        if (lane == 0) s_gate[t] = __uint_as_float((uint32_t)w[4]);
-        if (__any(!fin)) {
-            if (lane == 0) s_bad = 1;
-            continue;
-        }
-        const float mx = wave_max4(lv);
-        float p[4], ssum = 0.0f;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const uint32_t e = (uint32_t)lane + 64u * i;
-            p[i] = e < E ? expf(lv[i] - mx) : 0.0f;
-            ssum += p[i];
-        }
-        ssum = group_reduce<64>(ssum, AddOp());
-#pragma unroll
-        for (int i = 0; i < 4; ++i) p[i] = ((uint32_t)lane + 64u * i < E) ? p[i] / ssum : -1.0f;
-        // top-8 by (probability descending, id ascending)
-        float psel[kTopK];
-        int idsel[kTopK];
-        top8_by_probability(p, lane, E, psel, idsel);
-        if (lane == 0) {
-            float total = -0.0f;
-            for (int k = 0; k < kTopK; ++k) total += psel[k];
-            float wsum = 0.0f;
-            for (int k = 0; k < kTopK; ++k) {
-                const float wk = psel[k] / total;
-                s_ids[t * kTopK + k] = idsel[k];
-                s_w[t * kTopK + k] = wk;
-                wsum += wk;
-            }
-            if (!(fabsf(wsum - 1.0f) <= 1e-4f)) s_bad = 1;
-        }
-    }
-    __syncthreads();
-    const int n = (int)m * kTopK;
-    if (tid == 0)  // every word of this launch has been read
-        __hip_atomic_store(&counter[kRouteSeq], seq + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    if (s_bad || s_last) {
-        const int32_t err = s_last ? TQF_HIP_ERR_DEVICE : TQF_HIP_ERR_ROUTER;
-        if (wave == 0)
-            for (int i = lane; i < (int)m * (kTopK + 1); i += kWave) {
-                plan->slots[i].token = -1;
-                plan->down[i / (kTopK + 1)][i % (kTopK + 1)].slot = -1;
-            }
-        if (tid == 0) {
-            plan->n_slots = 0;
-            plan->n_union = 0;
-            plan->status = err;
-            plan->m = (int)m;
-            if (status_out) *status_out = err;
-        }
-        return;
-    }
-    // Pair plan, one route entry i = (t, k) per lane of wave 0 (n <= 64).
-    // The entries of one expert as the bits of one mask (broadcast LDS reads):
-    // a group starts at its lowest entry; base = the entries of the groups
-    // that start earlier, upos = those groups' count.
-    if (wave == 0) {
-        __shared__ int s_first[kMaxTokens * kTopK];
-        const int e_i = lane < n ? s_ids[lane] : -1;
-        uint64_t eq = 0;
-#pragma unroll
-        for (int j = 0; j < MT * kTopK; ++j) eq |= (j < n && s_ids[j] == e_i) ? (1ull << j) : 0ull;
-        const int rank = __builtin_popcountll(eq & ((1ull << lane) - 1ull));
-        const int first = lane < n ? (int)__builtin_ctzll(eq) : lane;
-        const bool flag = lane < n && first == lane;
-        const uint64_t F = __ballot(flag);
-        const int upos = __builtin_popcountll(F & ((1ull << first) - 1ull));
-        s_first[lane] = first;
-        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        int base = 0;
-#pragma unroll
-        for (int j = 0; j < MT * kTopK; ++j) base += (j < n && s_first[j] < first) ? 1 : 0;
-        const int nu = __builtin_popcountll(F);
-        if (lane < n) {
-            const int slot = (int)m + base + rank;
-            const int t = lane / kTopK, k = lane % kTopK;
-            const float wv = s_w[lane];
-            SlotRec rec;
-            rec.mat[0] = L.mats[e_i * 3 + 0];
-            rec.mat[1] = L.mats[e_i * 3 + 1];
-            rec.mat[2] = L.mats[e_i * 3 + 2];
-            rec.token = t;
-            rec.coef = wv;
-            plan->slots[slot] = rec;
-            plan->down[t][1 + k] = DownRec{rec.mat[2], slot, wv};
-            plan->slot_expert[slot] = e_i;
-            plan->pair_slot[lane] = slot;
-            plan->ids[t][k] = (uint16_t)e_i;
-            plan->weights[t][k] = wv;
-            if (flag) plan->union_ids[upos] = e_i;
-            if (ids_out) ids_out[lane] = (uint16_t)e_i;
-            if (w_out) w_out[lane] = wv;
-        }
-        if (lane < (int)m) {
-            const float gl = s_gate[lane];
-            plan->gate_logit[lane] = gl;
-            SlotRec rec;
-            rec.mat[0] = L.mats[E * 3 + 0];
-            rec.mat[1] = L.mats[E * 3 + 1];
-            rec.mat[2] = L.mats[E * 3 + 2];
-            rec.token = lane;
-            rec.coef = 1.0f / (1.0f + expf(-gl));
-            plan->slots[lane] = rec;
-            plan->down[lane][0] = DownRec{rec.mat[2], lane, rec.coef};
-            plan->slot_expert[lane] = (int)E;
-        }
-        if (lane == 0) {
-            plan->n_union = nu;
-            plan->n_slots = (int)m * (kTopK + 1);
-            plan->status = 0;
-            plan->m = (int)m;
-        }
-    }
 }
 
 hipError_t launch_route(hipStream_t s, const LayerDev &L, const float *h, const float *norm,
-                        uint32_t m, Scratch &sc, uint16_t *ids_out, float *w_out,
-                        int32_t *status_out, bool records, uint32_t *q8, uint32_t bp8) {
+                        uint32_t m, float *logits, uint32_t *xprep, uint32_t *q8, uint32_t bp8) {
     if (q8 && (m * (L.hidden / 256) > (L.n_experts + 1 + kRouteRows - 1) / kRouteRows || bp8 < L.hidden / 32))
         return hipErrorInvalidValue;
     const uint32_t grid = (L.n_experts + 1 + kRouteRows - 1) / kRouteRows;
     const uint32_t bp = padded_blocks(L.hidden / 32);
-    uint32_t *counter = sc.counters;
-#define TQF_ROUTE(MT)                                                                        \
-    hipLaunchKernelGGL(route_kernel<MT>, dim3(grid), dim3(kRouteThreads<MT>), 0, s, L, h, norm, m, bp,          \
-                       records ? sc.xprep : nullptr,                                               \
-                       sc.logits, sc.plan, counter, ids_out, w_out, status_out, q8, bp8)
+#define TQF_ROUTE(MT) \
+    hipLaunchKernelGGL(route_kernel<MT>, dim3(grid), dim3(kRouteThreads), 0, s, L, h, norm, m, bp, xprep, logits, q8, bp8)
     if (m <= 1) TQF_ROUTE(1);
     else if (m <= 2) TQF_ROUTE(2);
     else if (m <= 4) TQF_ROUTE(4);
@@ -552,11 +335,32 @@ hipError_t launch_route(hipStream_t s, const LayerDev &L, const float *h, const 
     return hipGetLastError();
 }
 
+// The distinct down matrices among the tokens' routes: a lane counts when no
+// lower one holds its matrix.
+__global__ __launch_bounds__(kWave) void count_union_kernel(Plan *plan, uint32_t m) {
+    const uint32_t n = m * kTopK, i = threadIdx.x;
+    bool first = i < n;
+    if (first) {
+        const DownRec mine = plan->down[i / kTopK][1 + i % kTopK];
+        if (mine.slot < 0) first = false;
+        for (uint32_t j = 0; j < i; ++j)
+            if (plan->down[j / kTopK][1 + j % kTopK].mat == mine.mat) first = false;
+    }
+    const uint64_t held = __ballot(first);
+    if (i == 0) plan->n_union = __builtin_popcountll(held);
+}
+
+hipError_t launch_count_union(hipStream_t s, Plan *plan, uint32_t m) {
+    hipLaunchKernelGGL(count_union_kernel, dim3(1), dim3(kWave), 0, s, plan, m);
+    return hipGetLastError();
+}
+
 // ---------------------------------------------------------------------------
 // Gate/up kernel.  Grid (width / (32 G) row groups, pair slots), four
 // wavefronts per workgroup (with eight, one token's 9 slots made 72 workgroups
 // for 256 CUs, and at 8 tokens one workgroup was resident per CU: 8.6 and 22.2
-// us, 6.7 and 16.7 with four); G = 64 / LPR lane groups per wavefront, LPR =
+// us, 6.7 and 16.7 with four; 7.7 and 19.8 since the workgroups make their own
+// routes, for which the route kernel takes 3.8 and 6.2 less); G = 64 / LPR lane groups per wavefront, LPR =
 // the gate/up matrices' padded block count (hidden / 32 <= 64).  Lane group
 // j of a wavefront owns 8 rows of both matrices: lane b loads block b of each
 // row (16 nibble loads), the scales of its block for the 8 rows (one 16-byte
@@ -568,25 +372,42 @@ hipError_t launch_route(hipStream_t s, const LayerDev &L, const float *h, const 
 constexpr int kGateUpWaves = 4;
 constexpr int kGateUpRows = 8;  // rows per lane group per matrix
 
-template <int LPR>
+template <int LPR, bool ROUTED>
 __global__ __launch_bounds__(kGateUpWaves * kWave) void gate_up_kernel(
-    LayerDev L, const Plan *__restrict__ plan, const uint32_t *__restrict__ xprep,
-    uint32_t *__restrict__ hprep, uint32_t rows_padded, uint32_t bp_down) {
+    LayerDev L, Plan *__restrict__ plan, const uint32_t *__restrict__ xprep, uint32_t *__restrict__ hprep,
+    uint32_t rows_padded, uint32_t bp_down, RouteArgs rt) {
     constexpr int G = kWave / LPR;
     constexpr int RW = kGateUpRows * G;  // rows per wavefront per matrix
     constexpr int R = LPR / 16;          // copies of each reduced value
     __shared__ float s_h[kGateUpWaves * RW];
     const int slot = blockIdx.y;
-    const SlotRec rec = load_slot(&plan->slots[slot]);
-    if (rec.token < 0) return;  // routing failed: no work
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
     const int lane = threadIdx.x % kWave;
     const uint32_t j = (uint32_t)lane / LPR, b = (uint32_t)lane % LPR;
-    const int tok = rec.token;
     const uint32_t r0 = (blockIdx.x * kGateUpWaves + wave) * RW;
+    const uint8_t *mat_gate, *mat_up;
+    uint32_t x[28];
+    if constexpr (ROUTED) {
+        __shared__ const uint8_t *s_mat[2];
+        if (slot >= (int)rt.m * (kTopK + 1)) {  // below the matvecs: the routes' record
+            const uint32_t t = (slot - rt.m * (kTopK + 1)) * gridDim.x + blockIdx.x;
+            if (t < rt.m) route_record(L, rt.logits, rt.m, (int)t, wave, lane, plan, rt.ids, rt.w, rt.status);
+            return;
+        }
+        const int tok = slot / (kTopK + 1), k = slot % (kTopK + 1);
+        load_xrec(xprep + (size_t)tok * LPR * kXprepDwords, LPR, b, x);
+        if (wave == 0) route_slot(L, rt.logits + (size_t)tok * (L.n_experts + 1), k, lane, s_mat);
+        __syncthreads();
+        mat_gate = uniform_ptr(s_mat[0]);
+        mat_up = uniform_ptr(s_mat[1]);
+    } else {
+        load_xrec(xprep + (size_t)slot * LPR * kXprepDwords, LPR, b, x);
+        mat_gate = L.mats[0];
+        mat_up = L.mats[1];
+    }
     if (r0 < rows_padded) {
-        const RowLane Wg = row_lane(rec.mat[0], LPR);
-        const RowLane Wu = row_lane(rec.mat[1], LPR);
+        const RowLane Wg = row_lane(mat_gate, LPR);
+        const RowLane Wu = row_lane(mat_up, LPR);
         const uint32_t rl = r0 + j * kGateUpRows;
         uint4 ng[kGateUpRows], nu[kGateUpRows];
 #pragma unroll
@@ -595,8 +416,6 @@ __global__ __launch_bounds__(kGateUpWaves * kWave) void gate_up_kernel(
             nu[n] = q4_signed(load_nibbles(Wu, rl + n, b));
         }
         const uint4 sg = load_scales(Wg, rl / 8, b), su = load_scales(Wu, rl / 8, b);
-        uint32_t x[28];
-        load_xrec(xprep + (size_t)tok * LPR * kXprepDwords, LPR, b, x);
         if (b >= L.hidden / 32) x[24] = 0;  // padding block: contributes exactly 0
         __builtin_amdgcn_sched_barrier(0);  // every load in flight before any math
         float v[2 * kGateUpRows];
@@ -621,20 +440,27 @@ __global__ __launch_bounds__(kGateUpWaves * kWave) void gate_up_kernel(
     }
 }
 
-hipError_t launch_gate_up(hipStream_t s, const LayerDev &L, uint32_t slots, const Plan *plan,
-                          const uint32_t *xprep, uint32_t *hprep) {
+hipError_t launch_gate_up(hipStream_t s, const LayerDev &L, uint32_t slots, Plan *plan,
+                          const uint32_t *xprep, uint32_t *hprep, const RouteArgs &rt) {
     const MatrixDims g = matrix_dims(L.width, L.hidden);
     const MatrixDims dn = matrix_dims(L.hidden, L.width);
     const uint32_t G = kWave / g.lpr;
     const uint32_t rows_per_group = kGateUpWaves * kGateUpRows * G;
     dim3 grid((g.rows_padded + rows_per_group - 1) / rows_per_group, slots);
+    grid.y += route_record_rows(rt.m, grid.x);
     dim3 block(kGateUpWaves * kWave);
-#define TQF_GU(LPR)                                                                         \
-    hipLaunchKernelGGL(gate_up_kernel<LPR>, grid, block, 0, s, L, plan, xprep, hprep,          \
-                       g.rows_padded, dn.blocks_padded)
-    if (g.blocks_padded == 16) TQF_GU(16);
-    else if (g.blocks_padded == 32) TQF_GU(32);
-    else if (g.blocks_padded == 64) TQF_GU(64);
+#define TQF_GU(LPR)                                                                                              \
+    {                                                                                                            \
+        if (rt.m)                                                                                                \
+            hipLaunchKernelGGL((gate_up_kernel<LPR, true>), grid, block, 0, s, L, plan, xprep, hprep, g.rows_padded, \
+                               dn.blocks_padded, rt);                                                            \
+        else                                                                                                     \
+            hipLaunchKernelGGL((gate_up_kernel<LPR, false>), grid, block, 0, s, L, plan, xprep, hprep, g.rows_padded, \
+                               dn.blocks_padded, rt);                                                            \
+    }
+    if (g.blocks_padded == 16) TQF_GU(16)
+    else if (g.blocks_padded == 32) TQF_GU(32)
+    else if (g.blocks_padded == 64) TQF_GU(64)
     else return hipErrorInvalidValue;
 #undef TQF_GU
     return hipGetLastError();

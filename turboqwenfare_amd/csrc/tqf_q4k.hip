@@ -21,6 +21,7 @@
 
 #include "tqf_device.h"
 #include "tqf_internal.h"
+#include "tqf_route.h"
 
 namespace tqf {
 
@@ -375,12 +376,12 @@ hipError_t launch_q8k_swiglu_quantize(hipStream_t s, const float *gu, uint32_t m
 //
 // SRC says where workgroup row blockIdx.y takes its matrix and records:
 // kSrcTables -- tables[blockIdx.y], the m rows of q8; kSrcSlotGateUp --
-// matrix blockIdx.y / S (0 gate, 1 up) of plan slot blockIdx.y % S (S =
-// gridDim.y / 2), the records of the slot's token; kSrcSlotDown -- the down
-// matrix of slot blockIdx.y, the slot's own records.  The slot forms run one
-// row of records (m = 1) and skip slots without work (routing failed).
-// kSrcSlotDownSwiglu -- as kSrcSlotDown, but the workgroup first makes the
-// slot's records itself, in LDS: quantize_q8_k of h = silu_mul(gate, up) from
+// matrix blockIdx.y / S (0 gate, 1 up) of slot blockIdx.y % S (S = 9 M), whose
+// expert the workgroup finds from the logits (tqf_route.h), the records of the
+// slot's token; kSrcSlotDownSwiglu -- the down matrix of slot blockIdx.y as the
+// plan records it, and records the workgroup first makes itself, in LDS.  The
+// slot forms run one row of records (m = 1); the down form skips slots without
+// work (routing failed).  Its records are quantize_q8_k of h = silu_mul(gate, up) from
 // gu ([gate rows | up rows] of every slot, gridDim.y slots, d.cols each),
 // the arithmetic of q8k_swiglu_quantize_kernel.
 // With fold.out set (kSrcSlotDownSwiglu only; every wavefront of a
@@ -390,7 +391,7 @@ hipError_t launch_q8k_swiglu_quantize(hipStream_t s, const float *gu, uint32_t m
 // slots to arrive sums them for the tile in q4k_moe_combine_kernel's order
 // and arithmetic, adds the residual, writes fold.out, and resets the counter.
 // ---------------------------------------------------------------------------
-constexpr int kSrcTables = 0, kSrcSlotGateUp = 1, kSrcSlotDown = 2, kSrcSlotDownSwiglu = 3;
+constexpr int kSrcTables = 0, kSrcSlotGateUp = 1, kSrcSlotDownSwiglu = 2;
 constexpr int kMaxRecBp = 64;  // padded sub-blocks of a record row made in LDS (cols <= 2048)
 
 struct Fold {
@@ -413,9 +414,9 @@ constexpr int kQ8KWaves = SRC == kSrcTables ? kQ4KWaves : kSlotWaves;
 
 template <int LPR, int TG, int SRC>
 __global__ __launch_bounds__(kQ8KWaves<SRC> * kWave) void q4k_q8k_gemv_kernel(
-    const uint8_t *const *__restrict__ tables, const Plan *__restrict__ plan, MatrixDims d,
+    const uint8_t *const *__restrict__ tables, Plan *__restrict__ plan, MatrixDims d,
     const uint32_t *__restrict__ q8, uint32_t m, float *__restrict__ y, const float *__restrict__ gu,
-    Fold fold) {
+    Fold fold, RouteArgs rt) {
     constexpr int NW = kQ8KWaves<SRC>;
     constexpr bool kDownSwiglu = SRC == kSrcSlotDownSwiglu;
     constexpr int G = kWave / LPR;         // row octets per wavefront
@@ -432,17 +433,28 @@ __global__ __launch_bounds__(kQ8KWaves<SRC> * kWave) void q4k_q8k_gemv_kernel(
     int token = 0;
     if constexpr (SRC == kSrcTables) {
         base = tables[mat];
+    } else if constexpr (SRC == kSrcSlotGateUp) {
+        // matrix mat of 2 S: the gates of the S = 9 M matvecs, then the ups,
+        // then the workgroups that record the routes
+        __shared__ const uint8_t *s_mat[2];
+        const uint32_t S = rt.m * (kTopK + 1);
+        if (mat >= 2 * S) {
+            const uint32_t t = (mat - 2 * S) * gridDim.x + blockIdx.x;
+            if (t < rt.m) route_record(rt.L, rt.logits, rt.m, (int)t, wave, lane, plan, rt.ids, rt.w, rt.status);
+            return;
+        }
+        const uint32_t slot = mat < S ? mat : mat - S;
+        token = (int)(slot / (kTopK + 1));
+        if (wave == 0)
+            route_slot(rt.L, rt.logits + (size_t)token * (rt.L.n_experts + 1), (int)(slot % (kTopK + 1)), lane, s_mat);
+        __syncthreads();
+        base = uniform_ptr(s_mat[mat < S ? 0 : 1]);
+        q8 += (size_t)token * d.blocks_padded * kQ8KRecDwords;
     } else {
-        const uint32_t S = SRC == kSrcSlotGateUp ? gridDim.y / 2 : gridDim.y;
-        const uint32_t slot = mat % S;
-        const SlotRec rec = load_slot(&plan->slots[slot]);
-        if (rec.token < 0) return;  // routing failed: no work for the whole workgroup
-        token = rec.token;
-        // a select, not an index: a dynamic index would move the record to LDS
-        base = SRC == kSrcSlotGateUp ? (mat < S ? rec.mat[0] : rec.mat[1]) : rec.mat[2];
-        if constexpr (!kDownSwiglu)
-            q8 += (size_t)(SRC == kSrcSlotGateUp ? (uint32_t)rec.token : slot) * d.blocks_padded *
-                  kQ8KRecDwords;
+        token = (int)(mat / (kTopK + 1));
+        const DownRec rec = load_down(&plan->down[token][mat % (kTopK + 1)]);
+        if (rec.slot < 0) return;  // routing failed: no work for the whole workgroup
+        base = rec.mat;
     }
     const bool has_rows = r0 < d.rows_padded;
     const RowLane W = row_lane(base, d.blocks_padded);
@@ -462,19 +474,14 @@ __global__ __launch_bounds__(kQ8KWaves<SRC> * kWave) void q4k_q8k_gemv_kernel(
         scm = load_scales(W, rl / 8, blk);
         dmw = *(const __attribute__((address_space(1))) uint32_t *)(dm_row + (size_t)(blk >> 3) * 32);
     };
-    float coef = 0.0f, weight[kTopK];
-    int pair[kTopK];
+    float weight[kTopK + 1];
     if constexpr (kDownSwiglu) {
         // the first chunk's weights are on their way while the records are
         // made, and so is what the fold reads of the plan
         if (has_rows) load_weights(b);
         if (fold.out) {
-            coef = plan->slots[token].coef;
 #pragma unroll
-            for (int kk = 0; kk < kTopK; ++kk) {
-                pair[kk] = plan->pair_slot[token * kTopK + kk];
-                weight[kk] = plan->weights[token][kk];
-            }
+            for (int kk = 0; kk <= kTopK; ++kk) weight[kk] = plan->down[token][kk].coef;
         }
         __builtin_amdgcn_sched_barrier(0);
         const uint32_t cols = d.cols, S = gridDim.y;
@@ -607,13 +614,13 @@ __global__ __launch_bounds__(kQ8KWaves<SRC> * kWave) void q4k_q8k_gemv_kernel(
         for (uint32_t r = threadIdx.x; r < rows_per_tile; r += blockDim.x) {
             const uint32_t c = tile * rows_per_tile + r;
             const size_t i = (size_t)token * H + c;
-            const float shared = load_coherent(&y[i]);
+            const float shared = load_coherent(&y[(size_t)token * (kTopK + 1) * H + c]);
             float v[kTopK];
 #pragma unroll
-            for (int kk = 0; kk < kTopK; ++kk) v[kk] = load_coherent(&y[(size_t)pair[kk] * H + c]);
-            float o = __fmul_rn(shared, coef);
+            for (int kk = 0; kk < kTopK; ++kk) v[kk] = load_coherent(&y[(size_t)(token * (kTopK + 1) + 1 + kk) * H + c]);
+            float o = __fmul_rn(shared, weight[0]);
 #pragma unroll
-            for (int kk = 0; kk < kTopK; ++kk) o = __fadd_rn(o, __fmul_rn(v[kk], weight[kk]));
+            for (int kk = 0; kk < kTopK; ++kk) o = __fadd_rn(o, __fmul_rn(v[kk], weight[1 + kk]));
             if (fold.resid) o = __fadd_rn(fold.resid[i], o);
             fold.out[i] = o;
         }
@@ -627,36 +634,34 @@ hipError_t launch_q4k_q8k_lpr(hipStream_t s, const uint8_t *const *tables, uint3
     constexpr uint32_t rows_per_group = kQ4KWaves * 8 * (kWave / LPR);
     const dim3 grid((d.rows_padded + rows_per_group - 1) / rows_per_group, count);
     const dim3 block(kQ4KWaves * kWave);
-    const Plan *none = nullptr;
+    Plan *none = nullptr;
     const float *nogu = nullptr;
     if (m <= 1)
-        hipLaunchKernelGGL((q4k_q8k_gemv_kernel<LPR, 1, kSrcTables>), grid, block, 0, s, tables, none, d, q8, m, y, nogu, Fold{});
+        hipLaunchKernelGGL((q4k_q8k_gemv_kernel<LPR, 1, kSrcTables>), grid, block, 0, s, tables, none, d, q8, m, y, nogu, Fold{}, RouteArgs{});
     else if (m <= 2)
-        hipLaunchKernelGGL((q4k_q8k_gemv_kernel<LPR, 2, kSrcTables>), grid, block, 0, s, tables, none, d, q8, m, y, nogu, Fold{});
+        hipLaunchKernelGGL((q4k_q8k_gemv_kernel<LPR, 2, kSrcTables>), grid, block, 0, s, tables, none, d, q8, m, y, nogu, Fold{}, RouteArgs{});
     else
-        hipLaunchKernelGGL((q4k_q8k_gemv_kernel<LPR, 4, kSrcTables>), grid, block, 0, s, tables, none, d, q8, m, y, nogu, Fold{});
+        hipLaunchKernelGGL((q4k_q8k_gemv_kernel<LPR, 4, kSrcTables>), grid, block, 0, s, tables, none, d, q8, m, y, nogu, Fold{}, RouteArgs{});
     return hipGetLastError();
 }
 
 template <int LPR>
-hipError_t launch_q4k_q8k_slots_lpr(hipStream_t s, const Plan *plan, uint32_t n_slots, bool down,
-                                    const MatrixDims &d, const uint32_t *q8, float *y, const float *gu,
-                                    const Fold &fold) {
+hipError_t launch_q4k_q8k_slots_lpr(hipStream_t s, Plan *plan, uint32_t n_slots, const MatrixDims &d,
+                                    const uint32_t *q8, float *y, const float *gu, const Fold &fold,
+                                    const RouteArgs &rt) {
     constexpr uint32_t rows_per_group = kSlotWaves * 8 * (kWave / LPR);
-    const dim3 grid((d.rows_padded + rows_per_group - 1) / rows_per_group, down ? n_slots : 2 * n_slots);
+    const uint32_t gx = (d.rows_padded + rows_per_group - 1) / rows_per_group;
+    const dim3 grid(gx, gu ? n_slots : 2 * n_slots + route_record_rows(rt.m, gx));
     const dim3 block(kSlotWaves * kWave);
     const uint8_t *const *none = nullptr;
     // the fold needs every wavefront of every workgroup to own rows
-    if (fold.out && (!down || !gu || d.rows % rows_per_group || d.rows_padded != d.rows)) return hipErrorInvalidValue;
-    if (down && gu)
+    if (fold.out && (!gu || d.rows % rows_per_group || d.rows_padded != d.rows)) return hipErrorInvalidValue;
+    if (gu)
         hipLaunchKernelGGL((q4k_q8k_gemv_kernel<LPR, 1, kSrcSlotDownSwiglu>), grid, block, 0, s, none, plan, d,
-                           q8, 1u, y, gu, fold);
-    else if (down)
-        hipLaunchKernelGGL((q4k_q8k_gemv_kernel<LPR, 1, kSrcSlotDown>), grid, block, 0, s, none, plan, d, q8, 1u, y,
-                           gu, Fold{});
+                           q8, 1u, y, gu, fold, rt);
     else
         hipLaunchKernelGGL((q4k_q8k_gemv_kernel<LPR, 1, kSrcSlotGateUp>), grid, block, 0, s, none, plan, d, q8, 1u,
-                           y, gu, Fold{});
+                           y, gu, fold, rt);
     return hipGetLastError();
 }
 
@@ -667,16 +672,25 @@ hipError_t launch_q4k_q8k_gemv(hipStream_t s, const uint8_t *const *tables, uint
     return launch_q4k_q8k_lpr<64>(s, tables, count, d, q8, m, y);
 }
 
-hipError_t launch_q4k_q8k_slots(hipStream_t s, const Plan *plan, uint32_t n_slots, bool down,
-                                const MatrixDims &d, const uint32_t *q8, float *y, const float *gu,
-                                float *out, const float *resid, uint32_t *counters) {
+static hipError_t launch_q4k_q8k_slots(hipStream_t s, Plan *plan, uint32_t n_slots, const MatrixDims &d,
+                                       const uint32_t *q8, float *y, const float *gu, const Fold &fold,
+                                       const RouteArgs &rt) {
     if (n_slots == 0 || n_slots > (uint32_t)kMaxSlots) return hipErrorInvalidValue;
-    if (gu && (!down || d.blocks_padded > (uint32_t)kMaxRecBp || d.cols % 256)) return hipErrorInvalidValue;
-    if (out && (!counters || n_slots % (kTopK + 1))) return hipErrorInvalidValue;
-    const Fold fold{out, resid, counters};
-    if (d.lpr == 16) return launch_q4k_q8k_slots_lpr<16>(s, plan, n_slots, down, d, q8, y, gu, fold);
-    if (d.lpr == 32) return launch_q4k_q8k_slots_lpr<32>(s, plan, n_slots, down, d, q8, y, gu, fold);
-    return launch_q4k_q8k_slots_lpr<64>(s, plan, n_slots, down, d, q8, y, gu, fold);
+    if (d.lpr == 16) return launch_q4k_q8k_slots_lpr<16>(s, plan, n_slots, d, q8, y, gu, fold, rt);
+    if (d.lpr == 32) return launch_q4k_q8k_slots_lpr<32>(s, plan, n_slots, d, q8, y, gu, fold, rt);
+    return launch_q4k_q8k_slots_lpr<64>(s, plan, n_slots, d, q8, y, gu, fold, rt);
+}
+
+hipError_t launch_q4k_gate_up(hipStream_t s, const MatrixDims &d, const RouteArgs &rt, const uint32_t *q8, Plan *plan,
+                              float *y) {
+    return launch_q4k_q8k_slots(s, plan, rt.m * (kTopK + 1), d, q8, y, nullptr, Fold{}, rt);
+}
+
+hipError_t launch_q4k_down(hipStream_t s, const MatrixDims &d, uint32_t m, Plan *plan, const float *gu, float *y,
+                           float *out, const float *resid, uint32_t *counters) {
+    if (!gu || d.blocks_padded > (uint32_t)kMaxRecBp || d.cols % 256) return hipErrorInvalidValue;
+    if (out && !counters) return hipErrorInvalidValue;
+    return launch_q4k_q8k_slots(s, plan, m * (kTopK + 1), d, nullptr, y, gu, Fold{out, resid, counters}, RouteArgs{});
 }
 
 uint32_t q4k_fold_tiles(const MatrixDims &d) {
@@ -703,14 +717,13 @@ __global__ __launch_bounds__(256) void q4k_moe_combine_kernel(const Plan *__rest
                                                               uint32_t m, uint32_t H,
                                                               const float *resid, float *y) {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= m * H || plan->status != 0) return;
+    if (i >= m * H) return;
     const uint32_t t = i / H, c = i % H;
-    float o = __fmul_rn(dn[(size_t)t * H + c], plan->slots[t].coef);
+    if (plan->down[t][0].slot < 0) return;  // routing failed
+    const float *row = dn + (size_t)t * (kTopK + 1) * H + c;
+    float o = __fmul_rn(row[0], plan->down[t][0].coef);
 #pragma unroll
-    for (int k = 0; k < kTopK; ++k) {
-        const int slot = plan->pair_slot[t * kTopK + k];
-        o = __fadd_rn(o, __fmul_rn(dn[(size_t)slot * H + c], plan->weights[t][k]));
-    }
+    for (int k = 1; k <= kTopK; ++k) o = __fadd_rn(o, __fmul_rn(row[(size_t)k * H], plan->down[t][k].coef));
     if (resid) o = __fadd_rn(resid[i], o);
     y[i] = o;
 }
