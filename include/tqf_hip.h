@@ -179,9 +179,10 @@ int32_t tqf_hip_stack_free(tqf_hip_ctx *ctx, tqf_hip_stack *stack);
  * equal d_h to update d_h in place.  d_ids/d_w ([n_layers x m x 8], may be
  * NULL) receive every layer's route; *d_status (may be NULL, zeroed by the
  * caller) is set to TQF_HIP_ERR_ROUTER if any layer's routing fails.
- * Every layer of a stack has one expert format.  For Q4_0 layers with
- * m <= 4 on the model geometry (hidden 2048, width <= 2048, <= 256
- * experts) the whole stack runs as one persistent launch of one workgroup
+ * Every layer of a stack has one expert format.  Q4_0 layers with m <= 4 on
+ * the model geometry (hidden 2048, width <= 2048, <= 256 experts) run the
+ * per-layer kernels as plain launches or, with TQF_HIP_VARIANT_PERSISTENT set
+ * to 1, the whole stack as one persistent launch of one workgroup
  * per CU, which needs every workgroup resident at once.  If other work on
  * the device keeps it from being co-scheduled, its waits time out after
  * 20 ms; with TQF_HIP_VARIANT_RECOVER (the default) the call then re-runs the
@@ -488,11 +489,14 @@ int32_t tqf_hip_verify_step_device(tqf_hip_ctx *ctx, const tqf_hip_stack *stack,
  *      GpuExecutionState::kernel_kind (backend/metal/expert.rs:56-92).  Each
  *      selector starts from the environment when the context is created
  *      (TQF_HIP_PERSISTENT, TQF_HIP_Q4K_FOLD, TQF_HIP_GRAPHS,
- *      TQF_HIP_RECOVER: "0" selects 0, anything else or unset 1) and is
- *      changed per context here; a change drops the context's captured
- *      graphs, so no replay keeps an old choice. ------------------------- */
+ *      TQF_HIP_RECOVER: "0" selects 0, anything else 1, unset the library's
+ *      choice, reported as 1) and is changed per context here, from
+ *      when on it holds; a change drops the context's captured graphs, so
+ *      no replay keeps an old choice. ------------------------- */
 #define TQF_HIP_VARIANT_PERSISTENT 0 /* 1: the persistent stack kernel where it applies;
-                                        0: per-layer kernels (graph-replayed)          */
+                                        0: per-layer kernels (graph-replayed); unset:
+                                        the faster, which are the per-layer kernels,
+                                        plain launches where the other would apply     */
 #define TQF_HIP_VARIANT_Q4K_FOLD 1   /* 1: a Q4_K layer's combine folded into its down
                                         launch; 0: the separate combine launch          */
 #define TQF_HIP_VARIANT_GRAPHS 2     /* 1: multi-launch paths replay HIP graphs;

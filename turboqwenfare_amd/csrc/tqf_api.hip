@@ -463,14 +463,29 @@ int32_t enqueue_stack(tqf_hip_ctx *ctx, const tqf_hip_stack *st, const float *d_
     return TQF_HIP_OK;
 }
 
-// The persistent path: model geometry, m <= kStackMT, a device that can
-// co-schedule one workgroup per CU.
+// The geometry of the persistent kernel: it reads Q4_0, m <= kStackMT.
+bool stack_small(const tqf_hip_stack *st, uint32_t m) {
+    return st->format == TQF_HIP_FORMAT_Q4_0 && st->d_layers && m <= (uint32_t)kStackMT &&
+           st->hidden == (uint32_t)kStackHidden && st->experts > 0 && st->experts <= 256 && st->width % 256 == 0 &&
+           st->width <= 2048;
+}
+
+// Such a stack left to the library runs the per-layer kernels as plain
+// launches, not as a graph per set of buffers: 692 us for 40 layers at one row
+// either way once captured, 29.8 against 35.3 for two, and nothing to capture
+// when the buffers are new.  The host takes 475 us for 40 layers.
+bool stack_direct(const tqf_hip_ctx *ctx, const tqf_hip_stack *st, uint32_t m) {
+    return ctx->variant[TQF_HIP_VARIANT_PERSISTENT] == kVariantAuto && stack_small(st, m);
+}
+
+// The persistent path: asked for, its geometry, a device that can co-schedule
+// one workgroup per CU.  Left to the library (kVariantAuto) a
+// stack runs the per-layer kernels: 692 / 798 / 900 / 994 us for 40 layers at
+// 1 / 2 / 3 / 4 rows and 30 / 35 / 40 / 45 for two, against the persistent
+// kernel's 841 / 946 / 1111 / 1051 and 59 / 64 / 70 / 70.
 bool stack_persistent_ok(tqf_hip_ctx *ctx, const tqf_hip_stack *st, uint32_t m) {
-    if (!ctx->variant[TQF_HIP_VARIANT_PERSISTENT]) return false;
-    if (st->format != TQF_HIP_FORMAT_Q4_0) return false;  // the persistent kernel reads Q4_0
-    if (!st->d_layers || m > (uint32_t)kStackMT || st->hidden != (uint32_t)kStackHidden ||
-        st->experts == 0 || st->experts > 256 || st->width % 256 || st->width > 2048)
-        return false;
+    if (ctx->variant[TQF_HIP_VARIANT_PERSISTENT] != 1) return false;
+    if (!stack_small(st, m)) return false;
     const uint32_t bp_down = padded_blocks(st->width / 32);
     if (ctx->stack_grid == 0) ctx->stack_grid = stack_grid(ctx->device, bp_down);
     // phase A writes the activation records of block q from workgroup q / 2
@@ -545,8 +560,8 @@ int32_t enqueue_accept(tqf_hip_ctx *ctx, const float *t, const float *d, const i
 // variant TQF_HIP_VARIANT_GRAPHS = 0 disables capture (eager launches of the
 // same kernels), e.g. under tracing tools that do not follow graphs.
 template <typename F>
-int32_t run_graphed(tqf_hip_ctx *ctx, const std::vector<uint64_t> &key, F enqueue) {
-    if (ctx->profiling || !ctx->variant[TQF_HIP_VARIANT_GRAPHS]) return enqueue();
+int32_t run_graphed(tqf_hip_ctx *ctx, const std::vector<uint64_t> &key, F enqueue, bool direct = false) {
+    if (direct || ctx->profiling || !ctx->variant[TQF_HIP_VARIANT_GRAPHS]) return enqueue();
     GraphEntry *g = find_graph(ctx, key);
     if (!g) {
         if (ctx->graphs.size() >= kMaxGraphs) {
@@ -678,7 +693,7 @@ extern "C" int32_t tqf_hip_create(int32_t device, tqf_hip_ctx **out) {
                                                               "TQF_HIP_GRAPHS", "TQF_HIP_RECOVER"};
     for (int i = 0; i < TQF_HIP_VARIANTS; ++i) {
         const char *v = std::getenv(kVariantEnv[i]);
-        ctx->variant[i] = (v && v[0] == '0') ? 0 : 1;
+        ctx->variant[i] = v ? (v[0] == '0' ? 0 : 1) : i == TQF_HIP_VARIANT_PERSISTENT ? kVariantAuto : 1;
     }
     *out = ctx;
     return TQF_HIP_OK;
@@ -699,7 +714,7 @@ extern "C" int32_t tqf_hip_get_variant(tqf_hip_ctx *ctx, int32_t variant, int32_
     TQF_ENTER(ctx);
     if (variant < 0 || variant >= TQF_HIP_VARIANTS || !value)
         return fail(ctx, TQF_HIP_ERR_INVALID, "unknown variant or null pointer");
-    *value = ctx->variant[variant];
+    *value = ctx->variant[variant] ? 1 : 0;
     return TQF_HIP_OK;
 }
 
@@ -1776,7 +1791,7 @@ extern "C" int32_t tqf_hip_stack_forward_device(tqf_hip_ctx *ctx, const tqf_hip_
                                  k64(d_status)};
     return run_graphed(ctx, key, [&]() {
         return enqueue_stack(ctx, stack, d_h_in, d_h, m, d_ids, d_w, d_status);
-    });
+    }, stack_direct(ctx, stack, m));
 }
 
 // ===========================================================================
@@ -2118,7 +2133,7 @@ extern "C" int32_t tqf_hip_verify_step_device(tqf_hip_ctx *ctx, const tqf_hip_st
                 if (int32_t rc = enqueue_stack(ctx, stack, d_h_in, d_h, m, nullptr, nullptr, d_status)) return rc;
                 return enqueue_accept(ctx, d_target, d_draft, d_dtok, k, vocab, temperature, greedy, d_u,
                                       d_ures, d_accepted, d_tokens, rec_accept);
-            }))
+            }, stack_direct(ctx, stack, m)))
             return rc;
     }
     if (!rec_stack && !rec_accept) return TQF_HIP_OK;

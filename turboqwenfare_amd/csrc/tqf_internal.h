@@ -356,6 +356,9 @@ struct tqf_hip_stack {
 
 namespace tqf {
 struct GraphEntry;
+// The persistent stack kernel where it is the faster one, which is nowhere at
+// present; tqf_hip_get_variant reports it as 1.
+constexpr int32_t kVariantAuto = 2;
 }
 
 struct tqf_hip_ctx {
@@ -406,7 +409,7 @@ struct tqf_hip_ctx {
     void *noalloc_scratch = nullptr;
     // kernel variant selectors (TQF_HIP_VARIANT_*), from the environment at
     // creation, changed by tqf_hip_set_variant
-    int32_t variant[TQF_HIP_VARIANTS] = {1, 1, 1, 1};
+    int32_t variant[TQF_HIP_VARIANTS] = {};
     // recovery from a timed-out cross-workgroup wait: pinned host words the
     // kernels report an abort in ([0] the persistent stack, [1] the one-launch
     // acceptance), their device addresses, and the reruns so far
