@@ -241,6 +241,29 @@ def test_moe_layer_kernels_over_widths_and_rows(backend, F):
         backend.free_moe_layer(L.dev)
 
 
+@pytest.mark.parametrize("hidden,width", [(256, 256), (768, 512), (1280, 256), (1792, 768)])
+def test_moe_layer_other_hidden_sizes(backend, hidden, width):
+    """Hidden sizes whose elements per thread of the route kernel do and do not
+    divide a 32-element activation block."""
+    mats = [(backend.synth_q4_0(width, hidden, 3 * e, 91), backend.synth_q4_0(width, hidden, 3 * e + 1, 91),
+             backend.synth_q4_0(hidden, width, 3 * e + 2, 91)) for e in range(257)]
+    router = synth.normal((256, hidden), seed=9101, std=hidden ** -0.5)
+    gate = synth.normal((hidden,), seed=9102, std=hidden ** -0.5)
+    cols = list(zip(*mats[:256]))
+    dev = backend.prepare_moe_layer(backend.upload_f32(router), backend.upload_f32(gate), mats[256], *map(list, cols))
+    host = [[backend.download_q4_0(t) for t in m3] for m3 in mats]
+    L = orc.MoeLayerHost(router, gate, *host[256], *map(list, zip(*host[:256])), hidden=hidden, width=width)
+    for m in (1, 3, 8):
+        x = synth.normal((m, hidden), seed=9110 + m)
+        y, ids, w = backend.moe_forward_batch(dev, x)
+        yc, idc, wc = L.forward_batch(x)
+        assert np.array_equal(ids, idc) and rel_err(w, wc) < 1e-5 and rel_err(y, yc) < FFN_TOL, (hidden, m)
+    backend.free_moe_layer(dev)
+    for m3 in mats:
+        for t in m3:
+            backend.free_weights(t)
+
+
 @pytest.mark.parametrize("fmt", ["q4_0", "q4_k"])
 @pytest.mark.parametrize("m", [1, 4, 8])
 def test_moe_router_error_in_any_row(backend, layer, fmt, m):

@@ -277,14 +277,14 @@ __global__ __launch_bounds__(kRouteThreads) void route_kernel(LayerDev L, const 
     //    block count bp.
     const uint32_t KB = xprep ? H / 32 : 0;
     for (uint32_t kb = blockIdx.x; kb < KB; kb += gridDim.x) {
-        const int lpb = 32 / vpt, at = tid - (int)kb * lpb;
+        const int at = (int)col0 - (int)kb * 32;  // vpt need not divide 32
         __syncthreads();
-        if (at >= 0 && at < lpb) {
+        if (at > -vpt && at < 32) {
 #pragma unroll
             for (int t = 0; t < MT; ++t)
 #pragma unroll
                 for (int v = 0; v < 8; ++v)
-                    if (v < vpt) s_blk[t][at * vpt + v] = x[t][v];
+                    if (v < vpt && (uint32_t)(at + v) < 32u) s_blk[t][at + v] = x[t][v];
         }
         __syncthreads();
         const int t = tid >> 5, j = tid & 31;
