@@ -368,12 +368,16 @@ hipError_t launch_count_union(hipStream_t s, Plan *plan, uint32_t m) {
 // then reduces the 16 block products across the group (value 2n + u: row n,
 // u = 0 gate, 1 up).  h = silu(gate) * up (weights.rs:241-259) meets in LDS
 // and a half-wavefront per block writes it as xprep records for the down kernel.
+// Held to 128 registers at LPR = 64 (136 without the bound), so that four
+// workgroups are resident per CU instead of three: the 1152 of eight tokens take
+// 1.1 rounds instead of 1.5; 40-layer verify step 1587 -> 1560 us there, 1045 ->
+// 1027 at four tokens.  At LPR = 16 and 32 the bound would spill.
 // ---------------------------------------------------------------------------
 constexpr int kGateUpWaves = 4;
 constexpr int kGateUpRows = 8;  // rows per lane group per matrix
 
 template <int LPR, bool ROUTED>
-__global__ __launch_bounds__(kGateUpWaves * kWave) void gate_up_kernel(
+__global__ __launch_bounds__(kGateUpWaves * kWave, LPR == 64 ? 4 : 1) void gate_up_kernel(
     LayerDev L, Plan *__restrict__ plan, const uint32_t *__restrict__ xprep, uint32_t *__restrict__ hprep,
     uint32_t rows_padded, uint32_t bp_down, RouteArgs rt) {
     constexpr int G = kWave / LPR;
