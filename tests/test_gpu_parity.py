@@ -241,10 +241,11 @@ def test_moe_layer_kernels_over_widths_and_rows(backend, F):
         backend.free_moe_layer(L.dev)
 
 
-@pytest.mark.parametrize("hidden,width", [(256, 256), (768, 512), (1280, 256), (1792, 768)])
+@pytest.mark.parametrize("hidden,width", [(256, 256), (256, 2048), (512, 1024), (768, 512), (1280, 256), (1792, 768)])
 def test_moe_layer_other_hidden_sizes(backend, hidden, width):
     """Hidden sizes whose elements per thread of the route kernel do and do not
-    divide a 32-element activation block."""
+    divide a 32-element activation block; the down kernel's parts of an octet
+    (2, 4 or 8 rows a lane group) at each lane count of a row."""
     mats = [(backend.synth_q4_0(width, hidden, 3 * e, 91), backend.synth_q4_0(width, hidden, 3 * e + 1, 91),
              backend.synth_q4_0(hidden, width, 3 * e + 2, 91)) for e in range(257)]
     router = synth.normal((256, hidden), seed=9101, std=hidden ** -0.5)

@@ -481,15 +481,15 @@ hipError_t launch_gate_up(hipStream_t s, const LayerDev &L, uint32_t slots, Plan
 // Bound by its latencies (records, weights, records of h, dot, sum).  All of a
 // token's records in one workgroup need no hand-off between workgroups: with
 // four slots a workgroup, whose partials the last one of a row group added up,
-// it took 6.1 / 14.1 us at 1 / 8 tokens, now 5.5 / 10.6.
+// it took 6.1 / 14.1 us at 1 / 8 tokens, with all of them in one 5.5 / 10.6,
+// and 1.3 us less at one token with the parts of octets that launch_down takes.
 // ---------------------------------------------------------------------------
-constexpr int kDownRows = 8;  // rows per lane group
-
-template <int LPR>
+// ROWS: rows per lane group, an octet or a part of one (see launch_down).
+template <int LPR, int ROWS>
 __global__ __launch_bounds__((kTopK + 1) * kWave) void down_kernel(LayerDev L, const Plan *__restrict__ plan,
                                                                    const uint32_t *__restrict__ hprep,
                                                                    const float *resid, float *out) {
-    constexpr int RW = kDownRows * (kWave / LPR);  // rows per workgroup
+    constexpr int RW = ROWS * (kWave / LPR);  // rows per workgroup
     __shared__ float red[kTopK + 1][RW];
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
     const int lane = threadIdx.x % kWave;
@@ -500,20 +500,27 @@ __global__ __launch_bounds__((kTopK + 1) * kWave) void down_kernel(LayerDev L, c
     const uint32_t r = threadIdx.x;
     const float res = resid && r < RW && r0 + r < H ? resid[(size_t)t * H + r0 + r] : 0.0f;
     const RowLane W = row_lane(rec.mat, LPR);
-    const uint32_t rl = r0 + j * kDownRows;
-    uint4 nib[kDownRows];
+    const uint32_t rl = r0 + j * ROWS;
+    uint4 nib[ROWS];
 #pragma unroll
-    for (int n = 0; n < kDownRows; ++n) nib[n] = q4_signed(load_nibbles(W, rl + n, b));
-    const uint4 sc = load_scales(W, rl / 8, b);
+    for (int n = 0; n < ROWS; ++n) nib[n] = q4_signed(load_nibbles(W, rl + n, b));
+    uint4 sc = {};  // the scales of rows rl .. rl + ROWS - 1
+    if constexpr (ROWS == 8) {
+        sc = load_scales(W, rl / 8, b);
+    } else {
+        const auto *p = (const __attribute__((address_space(1))) uint32_t *)(W.base + (((size_t)(rl / 8) * 9 + 8) * LPR + b) * 16) + (rl & 7) / 2;
+        sc.x = p[0];
+        if constexpr (ROWS == 4) sc.y = p[1];
+    }
     uint32_t x[28];
     load_xrec(hprep + (size_t)rec.slot * LPR * kXprepDwords, LPR, b, x);
     if (b >= L.width / 32) x[24] = 0;  // padding block: contributes exactly 0
     __builtin_amdgcn_sched_barrier(0);  // every load in flight before any math
-    float a[kDownRows];
+    float a[ROWS];
 #pragma unroll
-    for (int n = 0; n < kDownRows; ++n) a[n] = octet_scale(sc, n) * q4_block_dot(nib[n], x);
-    const float v = rec.coef * transpose_reduce<LPR, kDownRows>(a);
-    if (reduced_first_copy<LPR, kDownRows>(lane)) red[wave][j * kDownRows + reduced_index<LPR, kDownRows>(lane)] = v;
+    for (int n = 0; n < ROWS; ++n) a[n] = octet_scale(sc, n) * q4_block_dot(nib[n], x);
+    const float v = rec.coef * transpose_reduce<LPR, ROWS>(a);
+    if (reduced_first_copy<LPR, ROWS>(lane)) red[wave][j * ROWS + reduced_index<LPR, ROWS>(lane)] = v;
     __syncthreads();
     if (r < RW && r0 + r < H) {
         float sum = red[0][r];
@@ -525,12 +532,27 @@ __global__ __launch_bounds__((kTopK + 1) * kWave) void down_kernel(LayerDev L, c
 hipError_t launch_down(hipStream_t s, const LayerDev &L, uint32_t m, uint32_t per_token, const Plan *plan,
                        const uint32_t *hprep, const float *resid, float *out) {
     const MatrixDims dn = matrix_dims(L.hidden, L.width);
-    const uint32_t rows = kDownRows * (kWave / dn.lpr);
-    const dim3 grid((dn.rows_padded + rows - 1) / rows, m), block(per_token * kWave);
-#define TQF_DOWN(LPR) hipLaunchKernelGGL(down_kernel<LPR>, grid, block, 0, s, L, plan, hprep, resid, out)
-    if (dn.blocks_padded == 16) TQF_DOWN(16);
-    else if (dn.blocks_padded == 32) TQF_DOWN(32);
-    else if (dn.blocks_padded == 64) TQF_DOWN(64);
+    // The fewest rows a workgroup that still make at most one workgroup per CU
+    // (256): 2048 rows of width 512 at one token are 64 workgroups of whole
+    // octets, whose nine wavefronts then share four SIMDs for 72 block products
+    // a lane.  40-layer stack at one token 681 -> 627 us with two rows a lane
+    // group, 16 layer calls 263 -> 243; whole octets from three tokens on.
+    const uint32_t groups = kWave / dn.lpr;
+    uint32_t rows = 2;
+    while (rows < 8 && dn.rows_padded / (rows * groups) * m > 256) rows *= 2;
+    const dim3 grid((dn.rows_padded + rows * groups - 1) / (rows * groups), m), block(per_token * kWave);
+#define TQF_DOWN(LPR)                                                                                             \
+    {                                                                                                            \
+        if (rows == 2)                                                                                           \
+            hipLaunchKernelGGL((down_kernel<LPR, 2>), grid, block, 0, s, L, plan, hprep, resid, out);            \
+        else if (rows == 4)                                                                                      \
+            hipLaunchKernelGGL((down_kernel<LPR, 4>), grid, block, 0, s, L, plan, hprep, resid, out);            \
+        else                                                                                                     \
+            hipLaunchKernelGGL((down_kernel<LPR, 8>), grid, block, 0, s, L, plan, hprep, resid, out);            \
+    }
+    if (dn.blocks_padded == 16) TQF_DOWN(16)
+    else if (dn.blocks_padded == 32) TQF_DOWN(32)
+    else if (dn.blocks_padded == 64) TQF_DOWN(64)
     else return hipErrorInvalidValue;
 #undef TQF_DOWN
     return hipGetLastError();
