@@ -221,3 +221,13 @@ def test_grouped_tile_edges(backend, small, t):
     ids, w = _routes_with_counts(t, counts, t)
     x = synth.bf16_round(synth.normal((t, small.H), seed=t))
     assert rel_err(backend.grouped_gemm(small.layer, x, ids, w), small.want(x, ids, w)) < FFN_TOL
+
+
+def test_grouped_rows_do_not_depend_on_the_chunk(backend, small):
+    """A row's sums run over the same blocks in the same order whatever tile it
+    falls in: 1024 tokens (tiles of up to 64 rows) and the same tokens in four
+    chunks (up to 32) give the same bits."""
+    ids, w = _routes_with_counts(1024, [1, 15, 16, 17, 33, 48, 49, 64, 65, 200], 7)
+    x = synth.bf16_round(synth.normal((1024, small.H), seed=7))
+    parts = [backend.grouped_gemm(small.layer, x[i:i + 256], ids[i:i + 256], w[i:i + 256]) for i in range(0, 1024, 256)]
+    assert np.array_equal(backend.grouped_gemm(small.layer, x, ids, w), np.concatenate(parts))

@@ -281,24 +281,20 @@ constexpr int kStepBlocks = 8;
 constexpr int kGemmWaves = 4;
 constexpr int kSub = 2;  // weight subtiles per wavefront
 
-struct Desc { u32x4 v; };  // a buffer descriptor in scalar registers; loads past `bytes` return zero
+typedef __amdgpu_buffer_rsrc_t Desc;  // loads past `bytes` return zero
 __device__ __forceinline__ Desc make_desc(const void *p, uint32_t bytes) {
-    const uint64_t a = (uint64_t)p;
-    Desc d;
-    d.v = u32x4{(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)a),
-                (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(a >> 32)) & 0xFFFFu, bytes, 0x00020000u};
-    return d;
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(p), (short)0, (int)bytes, 0x00020000);
 }
-// 16 (4) bytes per lane from descriptor + voff + soff to LDS byte lds + 16 (4) x lane.
-__device__ __forceinline__ void copy16(const Desc &d, uint32_t voff, uint32_t soff, uint32_t lds) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(lds), "v"(voff), "s"(d.v),
-                 "s"(soff)
-                 : "memory", "m0");
+// 16 (4) bytes per lane from descriptor + voff + soff to LDS byte lds + 16 (4) x
+// lane.  Builtins: the wait states between a write of m0 or of a descriptor's
+// register and the load are the compiler's to count, which it cannot inside an
+// assembly string (there, one kernel had three where five are needed).
+typedef __attribute__((address_space(3))) void lds_void;
+__device__ __forceinline__ void copy16(Desc d, uint32_t voff, uint32_t soff, uint32_t lds) {
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(d, (lds_void *)lds, 16, voff, soff, 0, 0);
 }
-__device__ __forceinline__ void copy4(const Desc &d, uint32_t voff, uint32_t soff, uint32_t lds) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dword %1, %2, %3 offen lds" ::"s"(lds), "v"(voff), "s"(d.v),
-                 "s"(soff)
-                 : "memory", "m0");
+__device__ __forceinline__ void copy4(Desc d, uint32_t voff, uint32_t soff, uint32_t lds) {
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(d, (lds_void *)lds, 4, voff, soff, 0, 0);
 }
 // This wavefront's LDS reads and writes are done, then the workgroup's; publish:
 // its copies too.
