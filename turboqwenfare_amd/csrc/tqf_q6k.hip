@@ -415,8 +415,9 @@ __global__ __launch_bounds__(kQ6KWaves * kWave) void q6k_q8k_gemv_kernel(
 constexpr int kQ6SWaves = 4;
 constexpr uint32_t kQ6SGroups = 512;  // two workgroups per CU on a 256-CU part
 
+// (s_nop: an LDS-direct load reads m0 one wait state after its write at the earliest)
 __device__ __forceinline__ void q6k_copy_to_lds_16(const void *gaddr, uint32_t lds) {
-    asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds), "v"(gaddr) : "memory", "m0");
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds), "v"(gaddr) : "memory", "m0");
 }
 
 __host__ __device__ inline bool q6k_streams(const MatrixDims &d) { return d.blocks_padded == 64; }

@@ -164,7 +164,8 @@ __device__ __forceinline__ void lds_barrier() {
 }
 
 // Direct global -> LDS copies: lane l's `size` bytes at gaddr land at LDS
-// byte address lds + l * size (m0 holds the wavefront's LDS base).  Issued as
+// byte address lds + l * size (m0 holds the wavefront's LDS base, written one
+// wait state before the load at the latest: s_nop).  Issued as
 // inline assembly so that the compiler adds no LDS-alias waits for them:
 // every reader of the destination runs after a full s_waitcnt and a barrier
 // (the grid barrier before phase C).  An operation the compiler does not
@@ -175,14 +176,14 @@ __device__ __forceinline__ uint32_t lds_addr(uint32_t byte_off) {
                reinterpret_cast<uint8_t *>(s_dyn)) + byte_off;
 }
 __device__ __forceinline__ void copy_to_lds_16(const void *gaddr, uint32_t lds) {
-    asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds), "v"(gaddr) : "memory", "m0");
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds), "v"(gaddr) : "memory", "m0");
 }
 __device__ __forceinline__ void copy_to_lds_4(const void *gaddr, uint32_t lds) {
-    asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dword %1, off" ::"s"(lds), "v"(gaddr) : "memory", "m0");
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, off" ::"s"(lds), "v"(gaddr) : "memory", "m0");
 }
 // The same at agent scope (sc1), for data other workgroups wrote.
 __device__ __forceinline__ void copy_to_lds_16_coherent(const void *gaddr, uint32_t lds) {
-    asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, off sc1" ::"s"(lds), "v"(gaddr) : "memory", "m0");
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off sc1" ::"s"(lds), "v"(gaddr) : "memory", "m0");
 }
 
 // Copies n 64-bit words written by other workgroups into LDS: every load of
