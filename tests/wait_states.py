@@ -7,8 +7,8 @@ the CDNA3 / CDNA4 instruction set documents ask the program to keep.
           instruction (v_readfirstlane, a compare, ...) wrote: 5
   m0      an LDS-direct load (``lds``, ``global_load_lds_*``) reads m0 that a
           scalar instruction wrote: 1
-  dot     a vector instruction reads or overwrites the result of a v_dot*, but
-          for the same opcode's accumulator: 3
+  dot     a vector instruction reads or overwrites the result of a v_dot*,
+          other than the same opcode as accumulator or result: 3
   sdwa    a vector instruction reads what an SDWA instruction wrote to a part
           of a register: 1
 
@@ -75,11 +75,7 @@ class Instruction:
             src = _regs(rest, "v") if re.search(r"UNUSED_PRESERVE", rest) else _regs(",".join(ops[n_dst:]), "v")
             self.uses += [(r, k) for r in src for k in ("dot", "sdwa")]
             self.uses += [(r, "dot") for r in _regs(dst, "v")]
-        # the accumulator of a v_dot*: the last source, or the destination of the two-operand forms
-        self.acc = set()
-        if name.startswith("v_dot"):
-            self.acc = _regs(dst, "v") if re.match(r"v_dot\d+c", name) else _regs(ops[-1].split(" ")[0], "v")
-            self.sources = _regs(",".join(ops[1:3]), "v")
+        self.factors = _regs(",".join(ops[1:3]), "v")  # of a v_dot*: not its accumulator or result
 
 
 def parse(asm: str):
@@ -120,7 +116,7 @@ def _step(state: dict, ins: Instruction, found):
         got = state.get((reg, rule))
         if got is None or got[0] >= NEED[rule]:
             continue
-        if rule == "dot" and ins.acc == {reg} and got[1] == ins.name and reg not in ins.sources:
+        if rule == "dot" and got[1] == ins.name and reg not in ins.factors:
             continue
         if found is not None:
             found.append((ins.line, rule, reg, got[0], ins.text))

@@ -203,15 +203,17 @@ __device__ __forceinline__ void q8_class_pairs(const uint4 &xa, const uint4 &xb,
         qb[cc] = sext_pair<2>(qd[cc]);
     }
 }
-// lo(a) lo(b) + hi(a) hi(b) (+ c) over signed int16 halves, exact in int32;
-// the first form starts from an inline zero (no accumulator register).
+// lo(a) lo(b) + hi(a) hi(b) (+ c) over signed int16 halves, exact in int32.
+// The first form asks for saturation, which no sum here reaches (below): only
+// the three-operand instruction has it, and that one starts from an inline
+// zero instead of a register set up for it.  Builtins, because the vector
+// instructions that read a dot's result need three wait states after it, which
+// the compiler keeps for its own dots but not for one in an assembly string.
+typedef short short2_t __attribute__((ext_vector_type(2)));
 __device__ __forceinline__ int dot2_i16_0(uint32_t a, uint32_t b) {
-    int r;
-    asm("v_dot2_i32_i16 %0, %1, %2, 0" : "=v"(r) : "v"(a), "v"(b));
-    return r;
+    return __builtin_amdgcn_sdot2(__builtin_bit_cast(short2_t, a), __builtin_bit_cast(short2_t, b), 0, true);
 }
 __device__ __forceinline__ int dot2_i16(uint32_t a, uint32_t b, int c) {
-    typedef short short2_t __attribute__((ext_vector_type(2)));
     return __builtin_amdgcn_sdot2(__builtin_bit_cast(short2_t, a), __builtin_bit_cast(short2_t, b), c, false);
 }
 
@@ -244,6 +246,7 @@ __device__ __forceinline__ void q6k_octet_sums(const uint4 (&nib)[8], const uint
     // every value times its group's scale, once for all tokens, as int16
     // pairs (class bytes 0, 1: group 2j; bytes 2, 3: group 2j + 1;
     // |4 (q - 32) s| <= 2^14), so that a token's class term is two int16 dot2s
+    // (each below 2^22)
     uint32_t wa[64], wb[64];
 #pragma unroll
     for (int p = 0; p < 8; ++p) {
