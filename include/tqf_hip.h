@@ -489,14 +489,17 @@ int32_t tqf_hip_verify_step_device(tqf_hip_ctx *ctx, const tqf_hip_stack *stack,
  *      GpuExecutionState::kernel_kind (backend/metal/expert.rs:56-92).  Each
  *      selector starts from the environment when the context is created
  *      (TQF_HIP_PERSISTENT, TQF_HIP_Q4K_FOLD, TQF_HIP_GRAPHS,
- *      TQF_HIP_RECOVER: "0" selects 0, anything else 1, unset the library's
- *      choice, reported as 1) and is changed per context here, from
- *      when on it holds; a change drops the context's captured graphs, so
- *      no replay keeps an old choice. ------------------------- */
+ *      TQF_HIP_RECOVER: "0" selects 0, anything else 1; unset PERSISTENT
+ *      starts as AUTO, the others as 1) and is changed per context here; a
+ *      change drops the context's captured graphs, so no replay keeps an old
+ *      choice.  What get reports set accepts, so a caller can restore it. -- */
 #define TQF_HIP_VARIANT_PERSISTENT 0 /* 1: the persistent stack kernel where it applies;
-                                        0: per-layer kernels (graph-replayed); unset:
-                                        the faster, which are the per-layer kernels,
-                                        plain launches where the other would apply     */
+                                        0: per-layer kernels (graph-replayed);
+                                        TQF_HIP_VARIANT_AUTO: the library's choice,
+                                        which is the per-layer kernels, as plain
+                                        launches where the other would apply: the same
+                                        results as 0                                   */
+#define TQF_HIP_VARIANT_AUTO 2       /* a value, of PERSISTENT only                    */
 #define TQF_HIP_VARIANT_Q4K_FOLD 1   /* 1: a Q4_K layer's combine folded into its down
                                         launch; 0: the separate combine launch          */
 #define TQF_HIP_VARIANT_GRAPHS 2     /* 1: multi-launch paths replay HIP graphs;

@@ -379,7 +379,13 @@ def test_stack_forward_parity(backend, stack3):
     backend.free(dids)
 
 
-def test_verify_step_graph_replays_match_eager(backend, stack3):
+@pytest.mark.parametrize("persistent", [True, False, _lib.VARIANT_AUTO], ids=["persistent", "per_layer", "auto"])
+def test_verify_step_graph_replays_match_eager(backend, stack3, persistent):
+    with backend.variant(_lib.VARIANT_PERSISTENT, persistent):
+        _verify_step_repeats(backend, stack3)
+
+
+def _verify_step_repeats(backend, stack3):
     layers, norms, st = stack3
     vocab, k = 151936, 3
     rng = np.random.default_rng(5)
@@ -552,6 +558,55 @@ def test_routes_with_tied_router_rows(backend):
         backend.free_stack(st)
 
 
+def test_variant_restores_what_it_found(backend):
+    """A selector that nobody set (the session's context) reads as the
+    library's choice, and a with-block or a caller's own get and set leaves it
+    so; what set refuses changes nothing."""
+    auto = _lib.VARIANT_AUTO
+    assert backend.get_variant(_lib.VARIANT_PERSISTENT) == auto
+    for value in (False, True, auto):
+        with backend.variant(_lib.VARIANT_PERSISTENT, value):
+            assert backend.get_variant(_lib.VARIANT_PERSISTENT) == value
+        assert backend.get_variant(_lib.VARIANT_PERSISTENT) == auto
+    for variant, value in ((_lib.VARIANT_PERSISTENT, 3), (_lib.VARIANT_PERSISTENT, -1), (_lib.VARIANT_GRAPHS, auto),
+                           (_lib.VARIANT_RECOVER, auto), (_lib.VARIANT_Q4K_FOLD, auto)):
+        old = backend.get_variant(variant)
+        assert backend.lib.tqf_hip_set_variant(backend.ctx, variant, value) == ERR_INVALID
+        assert backend.get_variant(variant) == old
+
+
+@pytest.mark.parametrize("in_place", [True, False], ids=["in_place", "out_of_place"])
+@pytest.mark.parametrize("m", [1, 2, 3, 4])
+def test_unset_stack_runs_the_layer_kernels(backend, stack3, m, in_place):
+    """A stack left to the library gives the bits of variant 0 (h, ids,
+    weights, status), launches no persistent kernel, and does both again
+    after a with-block that did."""
+    _, _, st = stack3
+    h0 = synth.normal((4, 2048), seed=440 + m)
+    want = _stack_run(backend, st, h0, m, 3, False)
+    assert want[3] == 0
+    for again in range(2):
+        if again:
+            with backend.variant(_lib.VARIANT_PERSISTENT, True):
+                assert _stack_run(backend, st, h0, m, 3, _lib.VARIANT_AUTO)[3] == 0
+                assert _stack_run(backend, st, h0, m, 3, True)[3] == 0
+        dh0 = None if in_place else backend.to_device(h0[:m])
+        dh = backend.to_device(h0[:m] if in_place else np.full((m, 2048), 7.0, np.float32))
+        dids, dw, dst = backend.alloc(3 * m * 8 * 2), backend.alloc(3 * m * 8 * 4), backend.to_device(np.zeros(1, np.int32))
+        backend.stack_forward_device(st, dh, m, dids, dw, dst, dh0)
+        got = (backend.read(dh, np.float32, (m, 2048)), backend.read(dids, np.uint16, (3, m, 8)),
+               backend.read(dw, np.float32, (3, m, 8)), int(backend.read(dst, np.int32, (1,))[0]))
+        assert got[3] == 0 and all(np.array_equal(a, b) for a, b in zip(got[:3], want[:3]))
+        backend.profile_enable(True)
+        backend.stack_forward_device(st, dh, m)
+        launches = backend.profile_read(_lib.KERNEL_STACK)[0], backend.profile_read(_lib.KERNEL_ROUTE)[0]
+        backend.profile_enable(False)
+        assert launches == (0, 3)
+        for b in (dh0, dh, dids, dw, dst):
+            if b is not None:
+                backend.free(b)
+
+
 def test_persistent_stack_repeats_bit_identically(backend, stack3):
     """Barrier and team counters return to zero at the end of every launch."""
     _, _, st = stack3
@@ -696,8 +751,9 @@ def test_verify_step_recovers_both_parts(backend, stack3, monkeypatch):
     before = backend.recovery_counts()
     monkeypatch.setenv("TQF_HIP_STACK_FAIL_AT_LAYER", "1")
     monkeypatch.setenv("TQF_HIP_ACCEPT_FAIL_POLL", "1")
-    backend.verify_step_device(st, bufs["h0"], dh, 4, bufs["t"], bufs["d"], bufs["dt"], vocab, 0.7, False,
-                               bufs["u"], bufs["ur"], acc, toks, dst)
+    with backend.variant(_lib.VARIANT_PERSISTENT, True):
+        backend.verify_step_device(st, bufs["h0"], dh, 4, bufs["t"], bufs["d"], bufs["dt"], vocab, 0.7, False,
+                                   bufs["u"], bufs["ur"], acc, toks, dst)
     monkeypatch.delenv("TQF_HIP_STACK_FAIL_AT_LAYER")
     monkeypatch.delenv("TQF_HIP_ACCEPT_FAIL_POLL")
     assert backend.recovery_counts() == (before[0] + 1, before[1] + 1)
@@ -709,7 +765,7 @@ def test_verify_step_recovers_both_parts(backend, stack3, monkeypatch):
         backend.free(b)
 
 
-@pytest.mark.parametrize("persistent", [True, False], ids=["persistent", "per_layer"])
+@pytest.mark.parametrize("persistent", [True, False, _lib.VARIANT_AUTO], ids=["persistent", "per_layer", "auto"])
 def test_verify_step_reports_router_error(backend, stack3, persistent):
     """A non-finite router logit inside the verify step reaches its d_status
     (TQF_HIP_ERR_ROUTER); the acceptance, which reads only the logits, still

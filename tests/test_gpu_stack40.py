@@ -44,6 +44,9 @@ from turboqwenfare_amd.workloads import H, SyntheticStack
 pytestmark = pytest.mark.gpu
 
 LAYERS = 40
+# how the stack runs: one persistent launch, replayed graphs of the layer
+# kernels, or as the library chooses (an unset context)
+PATHS = {"persistent": True, "per_layer": False, "auto": _lib.VARIANT_AUTO}
 SPREAD = json.loads((Path(__file__).parent / "golden" / "stack40_spread.json").read_text())
 
 
@@ -74,10 +77,10 @@ def oracle_for(model, m):
     return model.oracle[m]
 
 
-def run_stack(be, model, m, persistent, stack=None, h0=None):
+def run_stack(be, model, m, path, stack=None, h0=None):
     stack = stack or model.stack
     n = len(stack.layers)
-    with be.variant(_lib.VARIANT_PERSISTENT, persistent):
+    with be.variant(_lib.VARIANT_PERSISTENT, PATHS[path]):
         dh = be.to_device(h0_rows(m) if h0 is None else h0)
         dids = be.alloc(n * m * 8 * 2)
         dw = be.alloc(n * m * 8 * 4)
@@ -91,17 +94,17 @@ def run_stack(be, model, m, persistent, stack=None, h0=None):
 
 
 @pytest.mark.parametrize("m", [4, 1])
-@pytest.mark.parametrize("persistent", [True, False], ids=["persistent", "per_layer"])
-def test_stack40_matches_oracle(backend, model40, m, persistent):
+@pytest.mark.parametrize("path", PATHS)
+def test_stack40_matches_oracle(backend, model40, m, path):
     hc, idc, wc = oracle_for(model40, m)
-    h, ids, w, status = run_stack(backend, model40, m, persistent)
+    h, ids, w, status = run_stack(backend, model40, m, path)
     assert status == 0
     for l in range(LAYERS):
         assert np.array_equal(ids[l], idc[l]), f"layer {l} routes differ"
     assert rel_err(w, wc) < 1e-5
     err = rel_err(h, hc)
     unions = [len(mtp.routes_union(idc[l])) for l in range(LAYERS)]
-    print(f"{model40.recipe} m={m} {'persistent' if persistent else 'per-layer'}: h rel err "
+    print(f"{model40.recipe} m={m} {path}: h rel err "
           f"{err:.3e}, |h| rms {np.sqrt(np.mean(hc.astype(np.float64) ** 2)):.2f}, union mean "
           f"{np.mean(unions):.2f} min {min(unions)} max {max(unions)}")
     assert err < h_bound(model40.recipe, m)
@@ -111,8 +114,8 @@ def test_stack40_matches_oracle(backend, model40, m, persistent):
 
 
 @pytest.mark.parametrize("m", [4, 1])
-@pytest.mark.parametrize("persistent", [True, False], ids=["persistent", "per_layer"])
-def test_stack40_layers_teacher_forced(backend, model40, m, persistent):
+@pytest.mark.parametrize("path", PATHS)
+def test_stack40_layers_teacher_forced(backend, model40, m, path):
     """Every layer alone, from the oracle's input to it: routes bit-equal and
     h within the reference's per-layer 1e-3."""
     hc, idc, wc = oracle_for(model40, m)
@@ -121,7 +124,7 @@ def test_stack40_layers_teacher_forced(backend, model40, m, persistent):
     for l in range(LAYERS):
         one = backend.prepare_stack([model40.stack.layers[l]], [model40.stack.norms[l]])
         try:
-            h, ids, w, status = run_stack(backend, model40, m, persistent, one, inputs[l])
+            h, ids, w, status = run_stack(backend, model40, m, path, one, inputs[l])
         finally:
             backend.free_stack(one)
         want = inputs[l + 1] if l + 1 < LAYERS else hc
@@ -131,7 +134,7 @@ def test_stack40_layers_teacher_forced(backend, model40, m, persistent):
         err = rel_err(h, want)
         worst = max(worst, err)
         assert err < 1e-3, f"layer {l}: {err:.3e}"
-    print(f"{model40.recipe} m={m} {'persistent' if persistent else 'per-layer'}: worst "
+    print(f"{model40.recipe} m={m} {path}: worst "
           f"teacher-forced layer {worst:.3e}")
 
 
@@ -146,13 +149,14 @@ def test_stack40_unions_follow_the_recipe(backend, model40):
         assert np.mean(late) < 12
 
 
+@pytest.mark.parametrize("path", PATHS)
 @pytest.mark.parametrize("greedy", [False, True], ids=["stochastic", "greedy"])
-def test_verify_step40_matches_stack_and_acceptance_oracle(backend, model40, greedy):
+def test_verify_step40_matches_stack_and_acceptance_oracle(backend, model40, greedy, path):
     """The full verify step at config 4: h bit-identical to the stack forward,
-    acceptance equal to the oracle's on the config-3 logits, status zero; the
-    graph/persistent step replayed several times with eager work between."""
+    acceptance equal to the oracle's on the config-3 logits, status zero; each
+    path's step repeated several times with eager work between."""
     be, m, k, vocab, T = backend, 4, 3, 151936, 0.7
-    h_ref, _, _, _ = run_stack(be, model40, m, True)
+    h_ref, _, _, _ = run_stack(be, model40, m, path)
     rng = np.random.default_rng(11)
     target = (rng.standard_normal((k + 1, vocab)) * 3.0).astype(np.float32)
     draft = (rng.standard_normal((k, vocab)) * 3.0).astype(np.float32)
@@ -166,26 +170,29 @@ def test_verify_step40_matches_stack_and_acceptance_oracle(backend, model40, gre
                                                  h0=h0_rows(m)).items()}
     dh, acc, toks = be.alloc(m * H * 4), be.alloc(4), be.alloc(4 * (k + 1))
     dst = be.to_device(np.zeros(1, np.int32))
-    for rep in range(3):
-        be.verify_step_device(model40.stack, bufs["h0"], dh, m, bufs["t"],
-                              None if greedy else bufs["d"], bufs["dt"], vocab, T, greedy,
-                              None if greedy else bufs["u"], None if greedy else bufs["ur"],
-                              acc, toks, dst)
-        h = be.read(dh, np.float32, (m, H))
-        a = int(be.read(acc, np.int32, (1,))[0])
-        tk = be.read(toks, np.int32, (k + 1,))
-        assert int(be.read(dst, np.int32, (1,))[0]) == 0
-        assert np.array_equal(h, h_ref), f"step {rep}: h differs from the stack forward"
-        assert (a, [int(v) for v in tk[: a + 1]]) == want
+    with be.variant(_lib.VARIANT_PERSISTENT, PATHS[path]):
+        for rep in range(3):
+            be.verify_step_device(model40.stack, bufs["h0"], dh, m, bufs["t"],
+                                  None if greedy else bufs["d"], bufs["dt"], vocab, T, greedy,
+                                  None if greedy else bufs["u"], None if greedy else bufs["ur"],
+                                  acc, toks, dst)
+            h = be.read(dh, np.float32, (m, H))
+            a = int(be.read(acc, np.int32, (1,))[0])
+            tk = be.read(toks, np.int32, (k + 1,))
+            assert int(be.read(dst, np.int32, (1,))[0]) == 0
+            assert np.array_equal(h, h_ref), f"step {rep}: h differs from the stack forward"
+            assert (a, [int(v) for v in tk[: a + 1]]) == want
     for b in list(bufs.values()) + [dh, acc, toks, dst]:
         be.free(b)
 
 
-def test_verify_step40_repeats_bit_identically(backend, model40):
+@pytest.mark.parametrize("path", ["persistent", "auto"])
+def test_verify_step40_repeats_bit_identically(backend, model40, path):
     """300 verify steps in a row at full depth: every step's h, accepted
-    length and tokens bit-identical to the first, status zero.  The barrier
-    counters of both levels, the logit accumulators and the partial-word tags
-    return to their start state at every launch."""
+    length and tokens bit-identical to the first, status zero.  In the
+    persistent kernel the barrier counters of both levels, the logit
+    accumulators and the partial-word tags return to their start state at
+    every launch."""
     be, m, k, vocab, T = backend, 4, 3, 151936, 0.7
     rng = np.random.default_rng(12)
     target = (rng.standard_normal((k + 1, vocab)) * 3.0).astype(np.float32)
@@ -198,16 +205,17 @@ def test_verify_step40_repeats_bit_identically(backend, model40):
     dh, acc, toks = be.alloc(m * H * 4), be.alloc(4), be.alloc(4 * (k + 1))
     dst = be.to_device(np.zeros(1, np.int32))
     first = None
-    for rep in range(300):
-        be.verify_step_device(model40.stack, bufs["h0"], dh, m, bufs["t"], bufs["d"], bufs["dt"],
-                              vocab, T, False, bufs["u"], bufs["ur"], acc, toks, dst)
-        out = (be.read(dh, np.float32, (m, H)).view(np.uint32), int(be.read(acc, np.int32, (1,))[0]),
-               be.read(toks, np.int32, (k + 1,)).copy(), int(be.read(dst, np.int32, (1,))[0]))
-        assert out[3] == 0, f"step {rep}: status {out[3]}"
-        if first is None:
-            first = out
-        else:
-            assert out[1] == first[1] and np.array_equal(out[2], first[2]), f"step {rep}: tokens differ"
-            assert np.array_equal(out[0], first[0]), f"step {rep}: h differs"
+    with be.variant(_lib.VARIANT_PERSISTENT, PATHS[path]):
+        for rep in range(300):
+            be.verify_step_device(model40.stack, bufs["h0"], dh, m, bufs["t"], bufs["d"], bufs["dt"],
+                                  vocab, T, False, bufs["u"], bufs["ur"], acc, toks, dst)
+            out = (be.read(dh, np.float32, (m, H)).view(np.uint32), int(be.read(acc, np.int32, (1,))[0]),
+                   be.read(toks, np.int32, (k + 1,)).copy(), int(be.read(dst, np.int32, (1,))[0]))
+            assert out[3] == 0, f"step {rep}: status {out[3]}"
+            if first is None:
+                first = out
+            else:
+                assert out[1] == first[1] and np.array_equal(out[2], first[2]), f"step {rep}: tokens differ"
+                assert np.array_equal(out[0], first[0]), f"step {rep}: h differs"
     for b in list(bufs.values()) + [dh, acc, toks, dst]:
         be.free(b)

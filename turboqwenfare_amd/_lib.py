@@ -37,6 +37,7 @@ VARIANT_PERSISTENT = 0
 VARIANT_Q4K_FOLD = 1
 VARIANT_GRAPHS = 2
 VARIANT_RECOVER = 3
+VARIANT_AUTO = 2  # a value, of VARIANT_PERSISTENT only
 FORMAT_Q4_0 = 0
 FORMAT_Q4_K = 1
 FORMAT_Q6_K = 2

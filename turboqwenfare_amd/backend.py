@@ -596,17 +596,20 @@ class HipBackend:
         return (toks[0], vals[0]) if squeeze else (toks, vals)
 
     # ---- kernel variants (GpuKernelKind) ------------------------------------------------
-    def set_variant(self, variant: int, value: bool) -> None:
-        self._check(self.lib.tqf_hip_set_variant(self.ctx, variant, 1 if value else 0))
+    def set_variant(self, variant: int, value) -> None:
+        """True or False, or for VARIANT_PERSISTENT also VARIANT_AUTO."""
+        auto = variant == _lib.VARIANT_PERSISTENT and value == _lib.VARIANT_AUTO
+        self._check(self.lib.tqf_hip_set_variant(self.ctx, variant, _lib.VARIANT_AUTO if auto else 1 if value else 0))
 
-    def get_variant(self, variant: int) -> bool:
+    def get_variant(self, variant: int):
+        """True or False, or VARIANT_AUTO where the choice is the library's."""
         v = C.c_int32()
         self._check(self.lib.tqf_hip_get_variant(self.ctx, variant, C.byref(v)))
-        return bool(v.value)
+        return _lib.VARIANT_AUTO if v.value == _lib.VARIANT_AUTO else bool(v.value)
 
     @contextlib.contextmanager
-    def variant(self, variant: int, value: bool):
-        """Selects a kernel variant for the duration of a with-block."""
+    def variant(self, variant: int, value):
+        """Selects a kernel variant (as set_variant) for the duration of a with-block."""
         old = self.get_variant(variant)
         self.set_variant(variant, value)
         try:

@@ -475,11 +475,11 @@ bool stack_small(const tqf_hip_stack *st, uint32_t m) {
 // either way once captured, 29.8 against 35.3 for two, and nothing to capture
 // when the buffers are new.  The host takes 475 us for 40 layers.
 bool stack_direct(const tqf_hip_ctx *ctx, const tqf_hip_stack *st, uint32_t m) {
-    return ctx->variant[TQF_HIP_VARIANT_PERSISTENT] == kVariantAuto && stack_small(st, m);
+    return ctx->variant[TQF_HIP_VARIANT_PERSISTENT] == TQF_HIP_VARIANT_AUTO && stack_small(st, m);
 }
 
 // The persistent path: asked for, its geometry, a device that can co-schedule
-// one workgroup per CU.  Left to the library (kVariantAuto) a
+// one workgroup per CU.  Left to the library (TQF_HIP_VARIANT_AUTO) a
 // stack runs the per-layer kernels: 692 / 798 / 900 / 994 us for 40 layers at
 // 1 / 2 / 3 / 4 rows and 30 / 35 / 40 / 45 for two, against the persistent
 // kernel's 841 / 946 / 1111 / 1051 and 59 / 64 / 70 / 70.
@@ -693,7 +693,7 @@ extern "C" int32_t tqf_hip_create(int32_t device, tqf_hip_ctx **out) {
                                                               "TQF_HIP_GRAPHS", "TQF_HIP_RECOVER"};
     for (int i = 0; i < TQF_HIP_VARIANTS; ++i) {
         const char *v = std::getenv(kVariantEnv[i]);
-        ctx->variant[i] = v ? (v[0] == '0' ? 0 : 1) : i == TQF_HIP_VARIANT_PERSISTENT ? kVariantAuto : 1;
+        ctx->variant[i] = v ? (v[0] == '0' ? 0 : 1) : i == TQF_HIP_VARIANT_PERSISTENT ? TQF_HIP_VARIANT_AUTO : 1;
     }
     *out = ctx;
     return TQF_HIP_OK;
@@ -701,7 +701,8 @@ extern "C" int32_t tqf_hip_create(int32_t device, tqf_hip_ctx **out) {
 
 extern "C" int32_t tqf_hip_set_variant(tqf_hip_ctx *ctx, int32_t variant, int32_t value) {
     TQF_ENTER(ctx);
-    if (variant < 0 || variant >= TQF_HIP_VARIANTS || (value != 0 && value != 1))
+    if (variant < 0 || variant >= TQF_HIP_VARIANTS ||
+        (value != 0 && value != 1 && !(value == TQF_HIP_VARIANT_AUTO && variant == TQF_HIP_VARIANT_PERSISTENT)))
         return fail(ctx, TQF_HIP_ERR_INVALID, "unknown variant or value");
     if (ctx->variant[variant] == value) return TQF_HIP_OK;
     TQF_HIP(ctx, hipStreamSynchronize(ctx->stream));
@@ -714,7 +715,7 @@ extern "C" int32_t tqf_hip_get_variant(tqf_hip_ctx *ctx, int32_t variant, int32_
     TQF_ENTER(ctx);
     if (variant < 0 || variant >= TQF_HIP_VARIANTS || !value)
         return fail(ctx, TQF_HIP_ERR_INVALID, "unknown variant or null pointer");
-    *value = ctx->variant[variant] ? 1 : 0;
+    *value = ctx->variant[variant];
     return TQF_HIP_OK;
 }
 

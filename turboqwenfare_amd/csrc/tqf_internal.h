@@ -356,9 +356,6 @@ struct tqf_hip_stack {
 
 namespace tqf {
 struct GraphEntry;
-// The persistent stack kernel where it is the faster one, which is nowhere at
-// present; tqf_hip_get_variant reports it as 1.
-constexpr int32_t kVariantAuto = 2;
 }
 
 struct tqf_hip_ctx {
