@@ -305,6 +305,33 @@ def test_moe_router_error_in_any_row(backend, layer, fmt, m):
         backend.free_moe_layer(L.dev)
 
 
+@pytest.mark.parametrize("m", [1, 2, 4, 8])
+def test_router_logits_are_summed_in_64_bits(backend, m):
+    """A router row's partial sums over 64 columns are added in 64 bits, as in
+    the persistent kernel: rows whose partial sums are 2^25, -2^25 and a small
+    multiple of 1 / 8 (all exact in f32), in columns of their own, have that
+    multiple as their logit.  In f32 it is lost wherever it meets one of the
+    others first."""
+    rng = np.random.default_rng(64)
+    want = rng.permutation(256).astype(np.float64) / 8.0 - 16.0
+    router = np.zeros((256, 2048), np.float32)
+    for e in range(256):
+        at = rng.choice(32, 3, replace=False) * 64 + rng.integers(0, 64, 3)
+        router[e, at] = (2.0 ** 25, -(2.0 ** 25), want[e])
+    L = Layer(backend, 9, router=router)
+    try:
+        x = np.ones((m, 2048), np.float32)
+        x[1:] *= 0.5  # other rows: half the logits
+        _, ids, w = backend.moe_forward_batch(L.dev, x)
+        for t in range(m):
+            p = np.exp(want * x[t, 0] - 16.0)
+            order = np.argsort(-p, kind="stable")[:8]
+            assert np.array_equal(ids[t], order), t
+            assert rel_err(w[t], p[order] / p[order].sum()) < 1e-6, t
+    finally:
+        backend.free_moe_layer(L.dev)
+
+
 def test_moe_layer_bf16_input(backend, layer):
     x = synth.normal((4, 2048), seed=7)
     xb = (x.view(np.uint32) >> 16).astype(np.uint16)

@@ -162,7 +162,7 @@ hipError_t launch_gemv(hipStream_t s, const uint8_t *const *d_tables, uint32_t c
 //   3. writes the xprep / Q8_K records of the blocks assigned to it.
 // The routes themselves are made from the logits by the gate/up kernels
 // (tqf_route.h).  Bound by its latencies (loads, two block sums), not by its
-// 2.1 MB: 3.9 / 6.0 / 7.8 us with the norm at 1 / 4 / 8 tokens (with the routing
+// 2.1 MB: 4.4 / 6.1 / 8.3 us with the norm at 1 / 4 / 8 tokens (with the routing
 // behind a poll of every workgroup's logits 7.7 / 10.4 / 14.0).
 // ---------------------------------------------------------------------------
 constexpr int kRouteRows = 2;
@@ -174,6 +174,7 @@ __global__ __launch_bounds__(kRouteThreads) void route_kernel(LayerDev L, const 
                                                               uint32_t bp, uint32_t *__restrict__ xprep,
                                                               float *__restrict__ logits,
                                                               uint32_t *__restrict__ q8, uint32_t bp8) {
+    __shared__ double s_dot[MT * kRouteRows][32];  // per value the partial sums of 32 groups of eight threads
     __shared__ float lds_red[4][MT * kRouteRows];
     __shared__ float lds_norm[4][MT];
     __shared__ float s_blk[MT][32];
@@ -248,25 +249,61 @@ __global__ __launch_bounds__(kRouteThreads) void route_kernel(LayerDev L, const 
         }
     }
 
-    // 2. logits of this workgroup's rows.
-    float dots[MT * kRouteRows];
-#pragma unroll
-    for (int rr = 0; rr < kRouteRows; ++rr) {
+    // 2. logits of this workgroup's rows.  For Q4_0 layers the products and
+    //    sums are in 64 bits: the persistent stack kernel adds its partial
+    //    logits in 64 bits, and what runs in its place holds them in no fewer
+    //    (route weights of one and four normalised rows against 64 bits,
+    //    relative: 0.88e-7 and 0.90e-7; f32 sums 1.45e-7 and 1.42e-7, the
+    //    persistent kernel 1.07e-7 and 1.11e-7; 4.3 / 6.4 / 8.5 -> 4.4 / 6.1 /
+    //    8.3 us at 1 / 4 / 8 tokens).  For Q4_K layers, which the persistent
+    //    kernel does not run, they stay in f32: the 8-bit activations turn a
+    //    changed last bit into another answer.
+    if (q8 == nullptr) {
 #pragma unroll
         for (int t = 0; t < MT; ++t) {
-            float s = 0.0f;
+            double s[kRouteRows] = {};
 #pragma unroll
-            for (int v = 0; v < 8; ++v) s = fmaf(x[t][v], wv[rr][v], s);
-            dots[rr * MT + t] = s;
+            for (int v = 0; v < 8; ++v)
+#pragma unroll
+                for (int rr = 0; rr < kRouteRows; ++rr) s[rr] = fma((double)x[t][v], (double)wv[rr][v], s[rr]);
+#pragma unroll
+            for (int rr = 0; rr < kRouteRows; ++rr) {
+                s[rr] += dpp_d<kDppXor1>(s[rr]);
+                s[rr] += dpp_d<kDppXor2>(s[rr]);
+                s[rr] += dpp_d<kDppHalfMirror>(s[rr]);
+                if ((tid & 7) == 0) s_dot[rr * MT + t][tid >> 3] = s[rr];
+            }
         }
-    }
-    block_sum_256<MT * kRouteRows>(dots, lds_red);
-    if (tid == 0) {
+        __syncthreads();
+        if (tid < 8 * MT * kRouteRows) {  // eight threads a value, four groups of eight threads each
+            const int i = tid >> 3, t = i % MT, g = 4 * (tid & 7);
+            double s = (s_dot[i][g] + s_dot[i][g + 1]) + (s_dot[i][g + 2] + s_dot[i][g + 3]);
+            s += dpp_d<kDppXor1>(s);
+            s += dpp_d<kDppXor2>(s);
+            s += dpp_d<kDppHalfMirror>(s);
+            const uint32_t r = blockIdx.x * kRouteRows + i / MT;
+            if ((tid & 7) == 0 && r <= E && t < (int)m) logits[(size_t)t * (E + 1) + r] = (float)s;
+        }
+    } else {
+        float dots[MT * kRouteRows];
 #pragma unroll
         for (int rr = 0; rr < kRouteRows; ++rr) {
-            const uint32_t r = blockIdx.x * kRouteRows + rr;
-            if (r <= E)
-                for (int t = 0; t < (int)m; ++t) logits[(size_t)t * (E + 1) + r] = dots[rr * MT + t];
+#pragma unroll
+            for (int t = 0; t < MT; ++t) {
+                float s = 0.0f;
+#pragma unroll
+                for (int v = 0; v < 8; ++v) s = fmaf(x[t][v], wv[rr][v], s);
+                dots[rr * MT + t] = s;
+            }
+        }
+        block_sum_256<MT * kRouteRows>(dots, lds_red);
+        if (tid == 0) {
+#pragma unroll
+            for (int rr = 0; rr < kRouteRows; ++rr) {
+                const uint32_t r = blockIdx.x * kRouteRows + rr;
+                if (r <= E)
+                    for (int t = 0; t < (int)m; ++t) logits[(size_t)t * (E + 1) + r] = dots[rr * MT + t];
+            }
         }
     }
     // 3. xprep (when asked for) of block kb is written by workgroup kb, one

@@ -225,7 +225,7 @@ __device__ __forceinline__ void zero_lacc(uint64_t *acc, uint32_t part, uint32_t
 // h with |h| around 10^7, whose normalised logits are ordinary) is a limit of
 // this accumulator only, so the routing aborts the launch, and with recovery
 // on the library re-runs the stack through the per-layer kernels, which sum
-// the logits in f32.
+// the logits in double.
 constexpr uint64_t kCountOne = 1ull << 58, kTermBias = 1ull << 52;
 constexpr uint64_t kFlagNonFinite = 1, kFlagRange = 2;
 __device__ __forceinline__ void add_counted(uint64_t *word, uint64_t *flag, float v) {
