@@ -178,7 +178,8 @@ int32_t tqf_hip_stack_free(tqf_hip_ctx *ctx, tqf_hip_stack *stack);
  * state); the result is written to d_h [m x hidden].  d_h_in may be NULL or
  * equal d_h to update d_h in place.  d_ids/d_w ([n_layers x m x 8], may be
  * NULL) receive every layer's route; *d_status (may be NULL, zeroed by the
- * caller) is set to TQF_HIP_ERR_ROUTER if any layer's routing fails.
+ * caller) is set to TQF_HIP_ERR_ROUTER if any layer's routing fails; such a
+ * layer hands its rows on unchanged and has no routes.
  * Every layer of a stack has one expert format.  Q4_0 layers with m <= 4 on
  * the model geometry (hidden 2048, width <= 2048, <= 256 experts) run the
  * per-layer kernels as plain launches or, with TQF_HIP_VARIANT_PERSISTENT set

@@ -332,6 +332,29 @@ def test_router_logits_are_summed_in_64_bits(backend, m):
         backend.free_moe_layer(L.dev)
 
 
+@pytest.mark.parametrize("persistent", [True, False, _lib.VARIANT_AUTO], ids=["persistent", "per_layer", "auto"])
+@pytest.mark.parametrize("m", [1, 4, 8])
+def test_failed_routing_passes_the_rows_on(backend, stack3, m, persistent):
+    """A stack whose routing fails adds nothing to its rows: out of place, too,
+    d_h holds h_in afterwards and not what was in the buffer, and no later
+    layer takes routes from that."""
+    _, _, st = stack3
+    h0 = synth.normal((m, 2048), seed=520 + m)
+    h0[m - 1, 100] = np.inf
+    dh0, dh = backend.to_device(h0), backend.to_device(synth.normal((m, 2048), seed=530))
+    dids = backend.to_device(np.full((3, m, 8), 999, np.uint16))
+    dst = backend.to_device(np.zeros(1, np.int32))
+    with backend.variant(_lib.VARIANT_PERSISTENT, persistent):
+        backend.stack_forward_device(st, dh, m, dids, None, dst, dh0)
+    assert int(backend.read(dst, np.int32, (1,))[0]) == ERR_ROUTER
+    assert np.array_equal(backend.read(dh, np.float32, (m, 2048)), h0)
+    ids = backend.read(dids, np.uint16, (3, m, 8))
+    # the persistent kernel writes 0 for the routes there are none of
+    assert np.all(ids == (0 if persistent is True and m <= 4 else 999))
+    for b in (dh0, dh, dids, dst):
+        backend.free(b)
+
+
 def test_moe_layer_bf16_input(backend, layer):
     x = synth.normal((4, 2048), seed=7)
     xb = (x.view(np.uint32) >> 16).astype(np.uint16)

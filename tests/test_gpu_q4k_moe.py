@@ -199,6 +199,26 @@ def test_q4k_stack_forward_parity(backend, q4k_stack, m):
         backend.free(b)
 
 
+@pytest.mark.parametrize("fold", [True, False])
+@pytest.mark.parametrize("m", [1, 4, 8])
+def test_q4k_failed_routing_passes_the_rows_on(backend, q4k_stack, m, fold):
+    """As for the Q4_0 stack: out of place d_h holds h_in after a failed
+    routing, whether the combine is folded into the down launch or not."""
+    _, _, st = q4k_stack
+    h0 = synth.normal((m, H), seed=540 + m)
+    h0[m - 1, 100] = np.inf
+    dh0, dh = backend.to_device(h0), backend.to_device(synth.normal((m, H), seed=550))
+    dids = backend.to_device(np.full((2, m, 8), 999, np.uint16))
+    dst = backend.to_device(np.zeros(1, np.int32))
+    with backend.variant(_lib.VARIANT_Q4K_FOLD, fold):
+        backend.stack_forward_device(st, dh, m, dids, None, dst, dh0)
+    assert int(backend.read(dst, np.int32, (1,))[0]) == ERR_ROUTER
+    assert np.array_equal(backend.read(dh, np.float32, (m, H)), h0)
+    assert np.all(backend.read(dids, np.uint16, (2, m, 8)) == 999)
+    for b in (dh0, dh, dids, dst):
+        backend.free(b)
+
+
 def test_stack_formats_do_not_mix(backend, q4k_stack):
     from test_gpu_parity import Layer
 

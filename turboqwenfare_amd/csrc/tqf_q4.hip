@@ -533,8 +533,11 @@ __global__ __launch_bounds__((kTopK + 1) * kWave) void down_kernel(LayerDev L, c
     const uint32_t j = (uint32_t)lane / LPR, b = (uint32_t)lane % LPR;
     const uint32_t t = blockIdx.y, r0 = blockIdx.x * RW, H = L.hidden;
     const DownRec rec = load_down(&plan->down[t][wave]);
-    if (rec.slot < 0) return;  // routing failed: every wavefront leaves
     const uint32_t r = threadIdx.x;
+    if (rec.slot < 0) {  // routing failed: every wavefront leaves, the residual goes on unchanged
+        if (resid && r < RW && r0 + r < H) out[(size_t)t * H + r0 + r] = resid[(size_t)t * H + r0 + r];
+        return;
+    }
     const float res = resid && r < RW && r0 + r < H ? resid[(size_t)t * H + r0 + r] : 0.0f;
     const RowLane W = row_lane(rec.mat, LPR);
     const uint32_t rl = r0 + j * ROWS;

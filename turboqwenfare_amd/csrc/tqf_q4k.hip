@@ -453,7 +453,16 @@ __global__ __launch_bounds__(kQ8KWaves<SRC> * kWave) void q4k_q8k_gemv_kernel(
     } else {
         token = (int)(mat / (kTopK + 1));
         const DownRec rec = load_down(&plan->down[token][mat % (kTopK + 1)]);
-        if (rec.slot < 0) return;  // routing failed: no work for the whole workgroup
+        if (rec.slot < 0) {  // routing failed: no work for the whole workgroup, the residual goes on unchanged
+            if (fold.out && fold.resid && mat % (kTopK + 1) == 0) {
+                const uint32_t n = d.rows / gridDim.x;
+                for (uint32_t r = threadIdx.x; r < n; r += blockDim.x) {
+                    const size_t i = (size_t)token * d.rows + blockIdx.x * n + r;
+                    fold.out[i] = fold.resid[i];
+                }
+            }
+            return;
+        }
         base = rec.mat;
     }
     const bool has_rows = r0 < d.rows_padded;
@@ -724,7 +733,10 @@ __global__ __launch_bounds__(256) void q4k_moe_combine_kernel(const Plan *__rest
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= m * H) return;
     const uint32_t t = i / H, c = i % H;
-    if (plan->down[t][0].slot < 0) return;  // routing failed
+    if (plan->down[t][0].slot < 0) {  // routing failed: the residual goes on unchanged
+        if (resid) y[i] = resid[i];
+        return;
+    }
     const float *row = dn + (size_t)t * (kTopK + 1) * H + c;
     float o = __fmul_rn(row[0], plan->down[t][0].coef);
 #pragma unroll
