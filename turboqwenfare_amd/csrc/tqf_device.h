@@ -526,7 +526,7 @@ __device__ __forceinline__ void xor_stage1(int *v) {
 }
 
 // ---------------------------------------------------------------------------
-// Reduction of N floats per thread over the first 256 threads; result valid in
+// Block-wide reduction of N floats per thread (256 threads); result valid in
 // every thread.
 // ---------------------------------------------------------------------------
 template <int N>
@@ -535,7 +535,7 @@ __device__ __forceinline__ void block_sum_256(float (&v)[N], float (*lds)[N]) {
     for (int i = 0; i < N; ++i) v[i] = group_reduce<64>(v[i], AddOp());
     const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
     __syncthreads();
-    if (lane == 0 && wave < 4)
+    if (lane == 0)
 #pragma unroll
         for (int i = 0; i < N; ++i) lds[wave][i] = v[i];
     __syncthreads();

@@ -2,11 +2,12 @@
 // layer kernels (route, gate/up + SwiGLU, down + weighted combine) for gfx950.
 //
 // The matrix layout and the integer-dot activation format are described in
-// tqf_internal.h.  Every kernel here is HBM-bound: the weight bytes are read
-// exactly once with 128-bit loads (a row's blocks spread over the lanes, 1 KiB
-// per wavefront load), all of a wavefront's loads are issued before any
-// math, and partial sums are combined in a fixed order (DPP / permlane
-// transposes, then LDS), so results are deterministic run to run.
+// tqf_internal.h.  The matvecs read the weight bytes exactly once with 128-bit
+// loads (a row's blocks spread over the lanes, 1 KiB per wavefront load) and
+// combine partial sums in a fixed order (DPP / permlane transposes, then LDS),
+// so results are deterministic run to run.  A pool of matrices is bound by
+// HBM; one matrix, or one layer of a few tokens, by the latencies of its
+// dependent loads (what each kernel says).
 #include <hip/hip_runtime.h>
 
 #include "tqf_device.h"
@@ -411,6 +412,7 @@ hipError_t launch_count_union(hipStream_t s, Plan *plan, uint32_t m) {
 // 1027 at four tokens.  At LPR = 16 and 32 the bound would spill.
 // ---------------------------------------------------------------------------
 constexpr int kGateUpWaves = 4;
+static_assert(kGateUpWaves == kRouteRecordWaves, "its workgroups also run route_record");
 constexpr int kGateUpRows = 8;  // rows per lane group per matrix
 
 template <int LPR, bool ROUTED>

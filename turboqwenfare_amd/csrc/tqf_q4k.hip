@@ -409,6 +409,7 @@ struct Fold {
 // hand-off: 10.8 and 9.6 for the down form; its integer work then sits on 64
 // CUs at one token.)
 constexpr int kSlotWaves = 4;
+static_assert(kSlotWaves == kRouteRecordWaves, "the gate/up form's workgroups also run route_record");
 template <int SRC>
 constexpr int kQ8KWaves = SRC == kSrcTables ? kQ4KWaves : kSlotWaves;
 
@@ -690,6 +691,7 @@ static hipError_t launch_q4k_q8k_slots(hipStream_t s, Plan *plan, uint32_t n_slo
                                        const uint32_t *q8, float *y, const float *gu, const Fold &fold,
                                        const RouteArgs &rt) {
     if (n_slots == 0 || n_slots > (uint32_t)kMaxSlots) return hipErrorInvalidValue;
+    if (d.blocks_padded != d.lpr) return hipErrorInvalidValue;  // the slot forms read one chunk a row (cols <= 2048)
     if (d.lpr == 16) return launch_q4k_q8k_slots_lpr<16>(s, plan, n_slots, d, q8, y, gu, fold, rt);
     if (d.lpr == 32) return launch_q4k_q8k_slots_lpr<32>(s, plan, n_slots, d, q8, y, gu, fold, rt);
     return launch_q4k_q8k_slots_lpr<64>(s, plan, n_slots, d, q8, y, gu, fold, rt);

@@ -82,10 +82,11 @@ __device__ __forceinline__ void route_slot(const LayerDev &L, const float *lt, i
     }
 }
 
-// One workgroup of four wavefronts per token: its down records and route outputs.  The last
-// three wavefronts see whether the logits of all tokens are finite; one that
+// One workgroup of kRouteRecordWaves wavefronts per token: its down records and route outputs.  All but the
+// first wavefront see whether the logits of all tokens are finite; one that
 // is not fails the call, every down record says so, and token 0's workgroup
 // reports it.
+constexpr int kRouteRecordWaves = 4;
 __device__ __forceinline__ void route_record(const LayerDev &L, const float *logits, uint32_t m, int tok, int wave, int lane,
                                              Plan *plan, uint16_t *ids_out, float *w_out, int32_t *status_out) {
     const uint32_t E = L.n_experts;
@@ -100,14 +101,15 @@ __device__ __forceinline__ void route_record(const LayerDev &L, const float *log
         route_probabilities(lv, lane, E, p);
         top8_by_probability(p, lane, E, psel, ids);
     } else {
-        float lv[(kMaxTokens + 2) / 3][4];
+        constexpr int kCheckers = kRouteRecordWaves - 1, kEach = (kMaxTokens + kCheckers - 1) / kCheckers;
+        float lv[kEach][4];
 #pragma unroll
-        for (int i = 0; i < (kMaxTokens + 2) / 3; ++i) {
-            const uint32_t t = (uint32_t)(wave - 1 + 3 * i);
+        for (int i = 0; i < kEach; ++i) {
+            const uint32_t t = (uint32_t)(wave - 1 + kCheckers * i);
             load_logits(logits + (size_t)(t < m ? t : 0) * (E + 1), lane, E, lv[i]);
         }
 #pragma unroll
-        for (int i = 0; i < (kMaxTokens + 2) / 3; ++i)
+        for (int i = 0; i < kEach; ++i)
 #pragma unroll
             for (int c = 0; c < 4; ++c)
                 if ((uint32_t)lane + 64u * c < E && !(fabsf(lv[i][c]) <= 3.402823466e38f)) fin = false;
