@@ -592,25 +592,32 @@ def mtp_loop_bench(be, layers: int, seed: int, recipe: str, steps: int = 40, war
     return out
 
 
-def kernel_source_digest() -> str:
-    """sha256 of the dominant kernel's sources: a committed traffic profile
-    counts for this build only when it was taken on the same sources."""
+# The sources of what the headline step's stack runs, and the committed HBM
+# traffic of one stack: the persistent kernel, or the layer kernels of all layers.
+STACK_SOURCES = {"stack_kernel": ("tqf_stack.hip", "tqf_device.h", "tqf_internal.h"),
+                 "layer_kernels": ("tqf_q4.hip", "tqf_route.h", "tqf_device.h", "tqf_internal.h")}
+STACK_TRAFFIC = {"stack_kernel": "stack_verify_traffic.json", "layer_kernels": "layer_kernels_verify_traffic.json"}
+
+
+def kernel_source_digest(path: str) -> str:
+    """sha256 of the sources of a STACK_SOURCES entry: a committed traffic
+    profile counts for this build only when it was taken on the same sources."""
     import hashlib
 
     hsh = hashlib.sha256()
-    for f in ("tqf_stack.hip", "tqf_device.h", "tqf_internal.h"):
+    for f in STACK_SOURCES[path]:
         hsh.update((ROOT / "turboqwenfare_amd" / "csrc" / f).read_bytes())
     return hsh.hexdigest()[:16]
 
 
-def committed_traffic(recipe: str):
-    """HBM bytes per stack launch from the committed rocprofv3 FETCH/WRITE
-    profile, if it was taken on these kernel sources and this workload."""
-    tfile = ROOT / "profiles" / "stack_verify_traffic.json"
+def committed_traffic(path: str, recipe: str):
+    """HBM bytes per stack from the committed rocprofv3 FETCH/WRITE profile,
+    if it was taken on these kernel sources and this workload."""
+    tfile = ROOT / "profiles" / STACK_TRAFFIC[path]
     if not tfile.exists():
         return None, "no committed traffic profile"
     t = json.loads(tfile.read_text())
-    if t.get("source_digest") != kernel_source_digest():
+    if t.get("source_digest") != kernel_source_digest(path):
         return None, "committed traffic profile was taken on other kernel sources"
     if t.get("recipe") != recipe:
         return None, f"committed traffic profile is for recipe {t.get('recipe')}"
@@ -782,15 +789,14 @@ def main():
 
     prof = head["kernels"]
     if "stack" in prof:
-        dom = prof["stack"]
+        dom, path = prof["stack"], "stack_kernel"
         dom_name = ("stack_kernel (persistent 40-layer MoE stack: router, union-expert gate/up + "
                     "SwiGLU, down + combine)")
-        traffic, traffic_src = committed_traffic(args.recipe)
     else:
-        dom = head["layer_kernels"]
+        dom, path = head["layer_kernels"], "layer_kernels"
         dom_name = ("route_kernel, gate_up_kernel and down_kernel (router, routes + gate/up + SwiGLU, "
                     "down + combine), the launches of all layers")
-        traffic, traffic_src = None, "the committed traffic profile is of the persistent stack kernel"
+    traffic, traffic_src = committed_traffic(path, args.recipe)
     acc_word = "greedy" if args.greedy else "stochastic"
     line = {
         "metric": "MTP k=3 verify steps/sec + Q4 expert GEMV HBM GB/s (% of peak), 1 GPU",
@@ -821,7 +827,7 @@ def main():
                      "traffic_source": traffic_src,
                      "kernel": dom_name,
                      "avg_us": dom["avg_us"], "algorithmic_bytes_per_launch": dom["bytes_per_launch"],
-                     "source_digest": kernel_source_digest()},
+                     "source_digest": kernel_source_digest(path)},
         "expert_union": head["expert_union"],
         "kernels": prof,
         "eager_profiled_ms_per_step": head["eager_profiled_ms_per_step"],

@@ -242,3 +242,28 @@ def test_q4k_stack_routes_change_under_rounding_noise():
     assert first == spread["q4k_m1_first_flip"][2] == 5
     assert dist == pytest.approx(spread["q4k_m1"][2], rel=1e-6)
     assert dist > 1.0
+
+
+@pytest.mark.parametrize("path, kernels", [("stack_kernel", ["stack_kernel"]),
+                                           ("layer_kernels", ["route_kernel", "gate_up_kernel", "down_kernel", "route_slot"])])
+def test_bench_digest_covers_the_reported_kernels(path, kernels, monkeypatch, tmp_path):
+    """The digest beside the headline's traffic is of the sources that define
+    the kernels it names: a change to any of them changes it, one to another
+    path's source does not."""
+    import re
+    import bench
+
+    csrc = Path(bench.ROOT) / "turboqwenfare_amd" / "csrc"
+    where = {k: {f.name for f in csrc.iterdir() if re.search(rf"void(\s+__\w+__\(.*?\))?\s+{k}\(", f.read_text())} for k in kernels}
+    assert all(len(w) == 1 and w <= set(bench.STACK_SOURCES[path]) for w in where.values()), where
+    copy = tmp_path / "turboqwenfare_amd" / "csrc"
+    copy.mkdir(parents=True)
+    for f in csrc.iterdir():
+        (copy / f.name).write_bytes(f.read_bytes())
+    want = bench.kernel_source_digest(path)
+    monkeypatch.setattr(bench, "ROOT", tmp_path)
+    for f in sorted(copy.iterdir()):
+        text = f.read_bytes()
+        f.write_bytes(text + b"\n// changed\n")
+        assert (bench.kernel_source_digest(path) != want) == (f.name in bench.STACK_SOURCES[path]), f.name
+        f.write_bytes(text)
