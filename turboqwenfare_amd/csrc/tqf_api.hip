@@ -471,18 +471,27 @@ bool stack_small(const tqf_hip_stack *st, uint32_t m) {
 }
 
 // Such a stack left to the library runs the per-layer kernels as plain
-// launches, not as a graph per set of buffers: 692 us for 40 layers at one row
-// either way once captured, 29.8 against 35.3 for two, and nothing to capture
-// when the buffers are new.  The host takes 475 us for 40 layers.
+// launches, not as a graph per set of buffers.  The line lies at the persistent
+// kernel's geometry because its callers never had anything to capture: calls on
+// new buffers stay as cheap as any other (625 / 981 us for 40 layers at 1 / 4
+// rows, 42 / 59 for two; with the capture 1019 / 1399 and 104 / 115), repeated
+// ones take what a replay takes (627 / 978 against 632 / 972; two layers 26.5 /
+// 43.9 against 31.9 / 48.7).  It is paid for in host time, 433 us of 40 layers
+// against 86-92 for a replay; the persistent launch with recovery held the host
+// until it was done.  Other stacks always replayed graphs and keep the host's
+// time: for them too the capture costs 390-510 us of the first call on new
+// buffers and a replay saves the host 350-390 us of 40 layers (Q4_K at 1 / 4 / 8
+// rows 775 / 1122 / 1650 us launched, 778 / 1122 / 1637 replayed; Q4_0 at 8 1503
+// either way).
 bool stack_direct(const tqf_hip_ctx *ctx, const tqf_hip_stack *st, uint32_t m) {
     return ctx->variant[TQF_HIP_VARIANT_PERSISTENT] == TQF_HIP_VARIANT_AUTO && stack_small(st, m);
 }
 
 // The persistent path: asked for, its geometry, a device that can co-schedule
 // one workgroup per CU.  Left to the library (TQF_HIP_VARIANT_AUTO) a
-// stack runs the per-layer kernels: 692 / 798 / 900 / 994 us for 40 layers at
-// 1 / 2 / 3 / 4 rows and 30 / 35 / 40 / 45 for two, against the persistent
-// kernel's 841 / 946 / 1111 / 1051 and 59 / 64 / 70 / 70.
+// stack runs the per-layer kernels: 622 / 760 / 895 / 974 us for 40 layers at
+// 1 / 2 / 3 / 4 rows and 26 / 34 / 40 / 44 for two, against the persistent
+// kernel's 845 / 964 / 1110 / 1053 and 59 / 65 / 70 / 69.
 bool stack_persistent_ok(tqf_hip_ctx *ctx, const tqf_hip_stack *st, uint32_t m) {
     if (ctx->variant[TQF_HIP_VARIANT_PERSISTENT] != 1) return false;
     if (!stack_small(st, m)) return false;

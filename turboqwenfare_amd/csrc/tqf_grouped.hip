@@ -272,11 +272,14 @@ __global__ __launch_bounds__(kPlanThreads) void gg_plan_kernel(
 // Measured, gate/up and down kernels in one run each (rocprof, medians): 37
 // Zipf tokens 40.9 + 28.2 -> 32.4 + 20.5 us, 512 116 + 80 -> 89 + 56 us, 4096
 // even tokens 411 + 286 -> 374 + 274 us against 32-row tiles of 8 wavefronts
-// that staged weights through registers.  Tried on the way at 4096 tokens and
-// no faster: 64-row tiles of 8 wavefronts with 4 subtiles each and the next
-// step's weights in flight (334 + 265 us, but 38 us for a lone tile, which a
-// short prompt waits for), double-buffered stages at two workgroups per CU (439
-// + 305), K started at a step of the workgroup's own (no change).
+// that staged weights through registers.  At 4096 tokens the clock falls under
+// sustained load: the same kernels take 304-374 and 229-274 us, so figures of
+// one run each do not rank what lies closer.  Tried on the way there and not
+// kept: double-buffered stages at two workgroups per CU (439 + 305), K started
+// at a step of the workgroup's own (no change).  Open: 64-row tiles of 8
+// wavefronts with 4 subtiles each and the next step's weights in flight took 334
+// + 265 us in a run of their own, not in turn with these (and 38 us for a lone
+// tile, which a short prompt would wait for).
 constexpr int kStepBlocks = 8;
 constexpr int kGemmWaves = 4;
 constexpr int kSub = 2;  // weight subtiles per wavefront

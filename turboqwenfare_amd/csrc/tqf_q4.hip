@@ -398,7 +398,7 @@ hipError_t launch_count_union(hipStream_t s, Plan *plan, uint32_t m) {
 // wavefronts per workgroup (with eight, one token's 9 slots made 72 workgroups
 // for 256 CUs, and at 8 tokens one workgroup was resident per CU: 8.6 and 22.2
 // us, 6.7 and 16.7 with four; 7.7 and 19.8 since the workgroups make their own
-// routes, for which the route kernel takes 3.8 and 6.2 less); G = 64 / LPR lane groups per wavefront, LPR =
+// routes, for which the route kernel takes 3.3 and 5.7 less); G = 64 / LPR lane groups per wavefront, LPR =
 // the gate/up matrices' padded block count (hidden / 32 <= 64).  Lane group
 // j of a wavefront owns 8 rows of both matrices: lane b loads block b of each
 // row (16 nibble loads), the scales of its block for the 8 rows (one 16-byte

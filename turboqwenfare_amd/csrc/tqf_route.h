@@ -5,8 +5,8 @@
 // workgroup the one that it needs.  Its first load is then the logits instead
 // of a plan, and no workgroup waits for another.  While the route kernel's
 // first workgroup polled the others' logits, made the routes and wrote a plan,
-// that kernel took 7.7 / 10.4 / 14.0 us at 1 / 4 / 8 tokens, now 3.9 / 6.0 /
-// 7.8; the routing costs the gate/up kernels 1.0 (Q4_0: 6.7 -> 7.7 us) at one
+// that kernel took 7.7 / 10.4 / 14.0 us at 1 / 4 / 8 tokens, now 4.4 / 6.1 /
+// 8.3; the routing costs the gate/up kernels 1.0 (Q4_0: 6.7 -> 7.7 us) at one
 // token, 1.7 (Q4_K: 12.2 -> 13.9) at four and 3.1 (Q4_0: 16.7 -> 19.8) at
 // eight.  Only one wavefront a workgroup routes, up to its own expert, and
 // what the other kernels read is recorded by workgroups of their own: with
