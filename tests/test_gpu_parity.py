@@ -218,8 +218,8 @@ def test_moe_layer_parity(backend, layer, m):
 def test_moe_layer_kernels_over_widths_and_rows(backend, F):
     """The layer kernels at the block counts of the down matrices (16, 32 and
     64 per lane group), at row counts on both sides of the route kernel's
-    instantiations (4 | 5 rows: one routing wavefront per row from there on)
-    and at the most rows; with the norm through a one-layer stack."""
+    instantiations (4 | 5 rows) and at the most rows; with the norm through a
+    one-layer stack."""
     L = Layer(backend, 40 + F // 256, F=F)
     norm = (1.0 + 0.1 * synth.normal((2048,), seed=970)).astype(np.float32)
     st = backend.prepare_stack([L.dev], [backend.upload_f32(norm)])
